@@ -491,7 +491,7 @@ static void setup_mixed(Box &b) {
   }
   // the z twiddle table exists only for the register-resident transforms
   // (the LDS Stockham kernels build their twiddles in LDS)
-  if (b.zfast) {
+  if (b.ztw) {
     dalloc(b.ztw_f, 2 * (size_t)b.nz);
     k_d2f(b, b.ztw, b.ztw_f, 2 * (size_t)b.nz);
   }
@@ -596,7 +596,11 @@ int otbl_create(const otbl_params *prm, const double *y, otbl_ctx **out) {
   b->zpair = std::getenv("OTBL_Z_NOPAIR") ? 0 : (std::getenv("OTBL_ZP_OCC2") ? 2 : 1);
   b->ytail = std::getenv("OTBL_Y_NOTAIL") == nullptr;
   dalloc(b->rowmax, 3 * (size_t)(b->ny + 1) * b->nx);
-  if (b->zfast) {
+  // lengths without such a plan: several rows per wavefront up to 1024, the
+  // LDS kernels beyond (OTBL_Z_LDS, OTBL_Z_STOCKHAM: always)
+  if (!b->zfast && std::getenv("OTBL_Z_STOCKHAM") == nullptr && std::getenv("OTBL_Z_LDS") == nullptr)
+    b->zteam = zteam_fns(b->nz);
+  if (b->zfast || b->zteam.nz) {
     dalloc(b->ztw, 2 * (size_t)b->nz);
     dalloc(b->zrow, (size_t)b->nz1);
     OTBL_HIP(hipMemset(b->zrow, 0, (size_t)b->nz1 * sizeof(double)));
@@ -1223,11 +1227,12 @@ int otbl_get_paths(otbl_ctx *ctx, char *buf, size_t len) {
   need(buf && len > 0, "otbl_get_paths: null buffer");
   char tmp[256];
   std::snprintf(tmp, sizeof tmp,
-                "y:%s%d%s z:%s%d dct:%s%d x:%s xseg:%d pois:%s%d prun:%d tuned:%d streams:%d tail:%d",
+                "y:%s%d%s z:%s%d dct:%s%d x:%s xseg:%d pois:%s%d prun:%d tuned:%d streams:%d tail:%d "
+                "zteam:%d",
                 b.yL ? "chunk" : "march", b.yL, (b.ytabh_f && b.yhalf) ? "h" : "", b.zfast ? "engine" : "stockham", b.nz,
                 b.dct_zfast ? "engine" : (b.dct_fft ? "stockham" : "gemm"), b.dct_M, b.xwin ? "window" : "march", b.xseg,
                 b.pchunk ? "chunk" : "march", b.pchunk, b.prun > 0 ? b.prun : (b.esz == 4 ? 4 : 2), b.tuned ? 1 : 0,
-                b.s2 ? 2 : 1, b.tail() ? 1 : 0);
+                b.s2 ? 2 : 1, b.tail() ? 1 : 0, b.zteam.lanes);
   std::snprintf(buf, len, "%s", tmp);
   API_END
 }

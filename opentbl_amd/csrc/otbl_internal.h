@@ -71,6 +71,26 @@ struct DevScalars {
   double ener[16];
 };
 
+// The z kernels with several rows per wavefront (otbl_zteam.h) of one row
+// length: lanes per row, rows per workgroup (of one wavefront), kernels.
+struct ZTeamFns {
+  int nz = 0, lanes = 0, rows = 0; // nz 0: none for this length
+  void (*p1d)(const double *, double *, double *, double *, const double *, const double2 *, int, int, double *) = nullptr;
+  void (*p1f)(const float *, float *, float *, float *, const float *, const float2 *, int, int, double *) = nullptr;
+  void (*p2d)(const double *, const double *, double *, double *, double *, const double2 *, int, int) = nullptr;
+  void (*p2f)(const float *, const float *, float *, float *, float *, const float2 *, int, int) = nullptr;
+  void (*fx)(double *, double *, int, const double2 *, int) = nullptr;
+};
+// row lengths of those kernels: even products of 2, 3, 5, 7 from 12 to 1024
+// that the engine of otbl_zfft.h does not run (longer ones stay on the LDS
+// kernels)
+constexpr bool zteam_length(int n) {
+  if (n < 12 || n > 1024 || n % 2 || n == 256 || n == 512 || n == 1024) return false;
+  for (int p : {2, 3, 5, 7})
+    while (n % p == 0) n /= p;
+  return n == 1;
+}
+
 struct Box {
   int nx, ny, nz, nz1, nz2, mz, xout, precision, dt_mode;
   int dev = 0; // the HIP device the box lives on (current at otbl_create)
@@ -169,6 +189,7 @@ struct Box {
   // twiddle table ztw (nz complex), else the LDS Stockham kernels
   FFTPlan zplan{};
   bool zfast = false;
+  ZTeamFns zteam; // else the kernels with several rows per wavefront (nz != 0)
   // FP32 z products with two rows per team (0: one row, OTBL_Z_NOPAIR; 1:
   // plane loop 1's pair kernel held to three waves per SIMD; 2: to two,
   // OTBL_ZP_OCC2)
@@ -291,6 +312,16 @@ void kz_rowmax(Box &b);
 template <typename R> void kz_products2(Box &b);
 void kz_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows);
 size_t k_zfft_shm_bytes(int nz, int nbuf);
+// z transforms with several rows per wavefront (otbl_zteam*.hip), valid when
+// Box::zteam.nz
+ZTeamFns zteam_fns(int nz);
+bool zteam_part1(int n, ZTeamFns &f); // row lengths up to 160
+bool zteam_part2(int n, ZTeamFns &f); // up to 336
+bool zteam_part3(int n, ZTeamFns &f); // up to 600
+bool zteam_part4(int n, ZTeamFns &f); // up to 1024
+template <typename R> void kzt_products1(Box &b);
+template <typename R> void kzt_products2(Box &b);
+void kzt_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows);
 
 // statistics (otbl_stats.hip): one sample of the current state added to
 // Box::st (statsp, stotf.F90:51-291); clearing the accumulators; launch

@@ -804,6 +804,10 @@ void k_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows) {
     kz_fourxz(b, fou, phys, iopt, nrows);
     return;
   }
+  if (b.zteam.nz) {
+    kzt_fourxz(b, fou, phys, iopt, nrows);
+    return;
+  }
   LAUNCH(b, "fourxz", nrows, TPB, zfft_shm(b, 2), fourxz_kernel, fou, phys, iopt, b.zplan, b.nz1, b.nz2);
 }
 
@@ -2283,6 +2287,8 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   // plane loop 1 products
   if (b.zfast) {
     kz_products1<T>(b);
+  } else if (b.zteam.nz) {
+    kzt_products1<T>(b);
   } else {
     LAUNCH(b, "products1", dim3((ny + b.zrb) / b.zrb, nx), TPB, shm, products1_kernel<T>, u, wki1, wki2, wki3, yc,
            plan, ny, nz1, b.nz2, b.rowmax, nx, b.zrb);
@@ -2348,6 +2354,8 @@ template <typename T> static void rhsp_t(Box &b, int m) {
     }
     if (b.zfast)
       kz_products2<T>(b);
+    else if (b.zteam.nz)
+      kzt_products2<T>(b);
     else
       LAUNCH(b, "products2", dim3((ny + b.zrb - 1) / b.zrb, nx - 2), TPB, shm, products2_kernel<T>, resv, resw, ya,
              yb, yc, plan, ny, nz1, b.nz2, b.zrb);

@@ -588,6 +588,50 @@ template <> void kz_dct_pencils<float>(Box &b, float *P, int iopt, int Lp, int l
   dct_launch<float>(b, P, iopt, Lp, ld, b.dct_chirp_f, b.dct_bf_f, b.dct_tw4_f, b.dct_ztw_f);
 }
 
+// ---------------------------------------------------------------------------
+// several rows per wavefront (otbl_zteam.h)
+// ---------------------------------------------------------------------------
+ZTeamFns zteam_fns(int nz) {
+  ZTeamFns f;
+  if (zteam_length(nz))
+    (void)(zteam_part1(nz, f) || zteam_part2(nz, f) || zteam_part3(nz, f) || zteam_part4(nz, f));
+  return f;
+}
+
+static unsigned tgrid(const Box &b, int nrows) { return (unsigned)((nrows + b.zteam.rows - 1) / b.zteam.rows); }
+
+template <typename R> void kzt_products1(Box &b) {
+  zcheck(b);
+  const int nrows = (b.ny + 1) * b.nx;
+  auto launch = [&](auto kf) {
+    LAUNCH(b, "products1", tgrid(b, nrows), 64, 0, kf, (const R *)fld<R>(b.f[OTBL_U]), fld<R>(b.wki1), fld<R>(b.wki2),
+           fld<R>(b.wki3), (const R *)fld<R>(b.yc), ztw<R>(b), b.ny, nrows, b.rowmax);
+  };
+  if constexpr (sizeof(R) == 8) launch(b.zteam.p1d);
+  else launch(b.zteam.p1f);
+  kz_rowmax(b);
+}
+
+template <typename R> void kzt_products2(Box &b) {
+  zcheck(b);
+  const int nrows = b.ny * (b.nx - 2);
+  auto launch = [&](auto kf) {
+    LAUNCH(b, "products2", tgrid(b, nrows), 64, 0, kf, (const R *)fld<R>(b.resv), (const R *)fld<R>(b.resw),
+           fld<R>(b.ya), fld<R>(b.yb), fld<R>(b.yc), ztw<R>(b), b.ny, nrows);
+  };
+  if constexpr (sizeof(R) == 8) launch(b.zteam.p2d);
+  else launch(b.zteam.p2f);
+}
+
+void kzt_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows) {
+  zcheck(b);
+  LAUNCH(b, "fourxz", tgrid(b, nrows), 64, 0, b.zteam.fx, fou, phys, iopt, (const double2 *)b.ztw, nrows);
+}
+
+template void kzt_products1<double>(Box &);
+template void kzt_products1<float>(Box &);
+template void kzt_products2<double>(Box &);
+template void kzt_products2<float>(Box &);
 template void kz_products1<double>(Box &);
 template void kz_products1<float>(Box &);
 template void kz_products2<double>(Box &);

@@ -334,6 +334,48 @@ static double lead_decay(std::vector<double> a, int n) {
   return worst;
 }
 
+// Plan of the chunked x lines for systems a (3, n): the shortest chunks with
+// which a line fits one workgroup, else chunks of lmax planes in spans whose
+// halo damps what lies outside below 1e-17.  depth: chunks after which a
+// carry is below 1e-19.  L 0 where the systems do not decay that fast.
+static XChunk xchunk_plan(std::initializer_list<const std::vector<double> *> systems, int n, int lmax) {
+  XChunk x;
+  for (int L = 4; L <= lmax && !x.L; L += 4)
+    if (XCH * L >= n) x.L = L;
+  const bool one = x.L > 0;
+  if (!one) x.L = lmax;
+  x.nc = (n + x.L - 1) / x.L;
+  double worst = 0.0; // largest product of multipliers over a whole chunk
+  for (const std::vector<double> *sys : systems) {
+    std::vector<double> a = *sys;
+    auto A = [&](int r, int j) -> double & { return a[3 * (size_t)j + r - 1]; };
+    for (int j = 2; j <= n; ++j) {
+      const double d = 1.0 / A(2, j - 1);
+      A(2, j - 1) = d;
+      A(1, j) = -A(1, j) * d;
+      A(2, j) = A(2, j) + A(1, j) * A(3, j - 1);
+    }
+    A(2, n) = 1.0 / A(2, n);
+    for (int q = 0; (q + 1) * x.L <= n; ++q) {
+      double m = 1.0, b = 1.0;
+      for (int j = q * x.L + 1; j <= (q + 1) * x.L; ++j) {
+        m *= j == 1 ? 0.0 : std::fabs(A(1, j));
+        b *= j == n ? 0.0 : std::fabs(A(3, j) * A(2, j));
+      }
+      worst = std::max(worst, std::max(m, b));
+    }
+  }
+  double p = 1.0;
+  for (x.depth = 0; x.depth < XCH && p >= 1e-19; ++x.depth) p *= worst;
+  if (one) return x;
+  p = 1.0;
+  for (x.halo = 0; x.halo < 4 && p >= 1e-17; ++x.halo) p *= worst;
+  if (p >= 1e-17) return XChunk();
+  for (x.ns = 2; (x.nc + x.ns - 1) / x.ns + 2 * x.halo > XCH; ++x.ns) {
+  }
+  return x;
+}
+
 static void free_box(Box *b) {
   if (!b) return;
   for (int q = 0; q < 4; ++q)
@@ -343,11 +385,11 @@ static void free_box(Box *b) {
                     b->wki3, b->ya, b->yb, b->yc, b->rest, b->rest2, b->dct2, b->dct3, b->implu,
                     b->implv, b->um, b->u0, b->v0, b->gwork, b->dct_chirp, b->dct_bf, b->dct_tw4,
                     b->ytab, b->ztw, b->zrow, b->dct_ztw, b->rowmax, b->P0, b->S0, b->p0, b->um64, b->rm64,
-                    b->diag, b->op64, b->rthcf, b->st, b->stcoef, b->stmean};
+                    b->diag, b->op64, b->rthcf, b->st, b->stcoef, b->stmean, b->xtab};
   for (double *p : bufs)
     if (p) (void)hipFree(p);
   if (b->diag_count) (void)hipFree(b->diag_count);
-  float *fbufs[] = {b->coefbuf_f, b->ytab_f, b->ytabh_f, b->ztw_f, b->dct_chirp_f, b->dct_bf_f, b->dct_tw4_f, b->dct_ztw_f};
+  float *fbufs[] = {b->coefbuf_f, b->ytab_f, b->ytabh_f, b->ztw_f, b->dct_chirp_f, b->dct_bf_f, b->dct_tw4_f, b->dct_ztw_f, b->xtab_f};
   for (float *p : fbufs)
     if (p) (void)hipFree(p);
   if (b->ens) (void)hipFree(b->ens);
@@ -488,6 +530,11 @@ static void setup_mixed(Box &b) {
   if (b.yL % 2 == 0 && !(yh && yh[0] == '0') && b.nu < (size_t(1) << 30)) {
     dalloc(b.ytabh_f, YT_COUNT * ytabh_size(b.yL / 2));
     k_ytab_halve_fixed(b);
+  }
+  if (b.xchunk) {
+    const size_t n = 2 * xtab_size(b.xci) + 4 * xtab_size(b.xcd);
+    dalloc(b.xtab_f, n);
+    k_d2f(b, b.xtab, b.xtab_f, n);
   }
   // the z twiddle table exists only for the register-resident transforms
   // (the LDS Stockham kernels build their twiddles in LDS)
@@ -643,6 +690,21 @@ int otbl_create(const otbl_params *prm, const double *y, otbl_ctx **out) {
     // group of XLINE_LEAD planes
     const int smax = std::max(1, std::min(8, b->nx / XLINE_LEAD));
     b->xseg_max = (b->xwin && lead < 1e-17) ? std::max(smax, b->xseg) : 1;
+  }
+  // chunked x lines (OTBL_X_MARCH, OTBL_XSEG, OTBL_X_WINDOW keep the others);
+  // the derivatives only where otbl_xchunk.hip says they gain (FP32 chunks of
+  // 24 planes do not fit the 64 registers of two workgroups per CU)
+  if (std::getenv("OTBL_X_MARCH") == nullptr && std::getenv("OTBL_XSEG") == nullptr &&
+      std::getenv("OTBL_X_WINDOW") == nullptr) {
+    const HostCoef &h = b->hc;
+    b->xci = xchunk_plan({&h.inxu, &h.inxv}, b->nx, 24);
+    const bool march = b->xwin && (b->esz == 8 ? b->pu >= 30000 : b->xseg <= 3 && b->xseg_max > 3);
+    if (!march) b->xcd = xchunk_plan({&h.dcxu, &h.dcxv, &h.vixu, &h.vixv}, b->nx, b->esz == 8 ? 24 : 20);
+    b->xchunk = b->xci.L > 0;
+    if (b->xchunk) {
+      dalloc(b->xtab, 2 * xtab_size(b->xci) + 4 * xtab_size(b->xcd));
+      kxc_tables(*b);
+    }
   }
   // chunked y-line solver unless the columns are longer than its
   // instantiations (or OTBL_Y_MARCH asks for one thread per column)
@@ -1228,11 +1290,11 @@ int otbl_get_paths(otbl_ctx *ctx, char *buf, size_t len) {
   char tmp[256];
   std::snprintf(tmp, sizeof tmp,
                 "y:%s%d%s z:%s%d dct:%s%d x:%s xseg:%d pois:%s%d prun:%d tuned:%d streams:%d tail:%d "
-                "zteam:%d",
+                "zteam:%d xchunk:%d",
                 b.yL ? "chunk" : "march", b.yL, (b.ytabh_f && b.yhalf) ? "h" : "", b.zfast ? "engine" : "stockham", b.nz,
                 b.dct_zfast ? "engine" : (b.dct_fft ? "stockham" : "gemm"), b.dct_M, b.xwin ? "window" : "march", b.xseg,
                 b.pchunk ? "chunk" : "march", b.pchunk, b.prun > 0 ? b.prun : (b.esz == 4 ? 4 : 2), b.tuned ? 1 : 0,
-                b.s2 ? 2 : 1, b.tail() ? 1 : 0, b.zteam.lanes);
+                b.s2 ? 2 : 1, b.tail() ? 1 : 0, b.zteam.lanes, b.xchunk ? b.xci.L : 0);
   std::snprintf(buf, len, "%s", tmp);
   API_END
 }

@@ -91,6 +91,19 @@ constexpr bool zteam_length(int n) {
   return n == 1;
 }
 
+// x lines split over the XCH wavefronts of a workgroup (otbl_xchunk.hip): L
+// planes per chunk (0: off), nc chunks per line, cut into ns spans that
+// overlap by halo chunks; carries reach depth chunks
+constexpr int XCH = 16;
+struct XChunk {
+  int L = 0, nc = 0, ns = 1, halo = 0, depth = 0;
+};
+// values of the table of one system
+constexpr size_t xtab_size(const XChunk &x) { return (size_t)8 * x.nc * x.L + 4 * x.nc; }
+// systems in Box::xtab, in this order: the interpolations with Box::xci, the
+// derivatives with Box::xcd
+enum { XT_INXU = 0, XT_INXV, XT_DCXU, XT_DCXV, XT_VIXU, XT_VIXV };
+
 struct Box {
   int nx, ny, nz, nz1, nz2, mz, xout, precision, dt_mode;
   int dev = 0; // the HIP device the box lives on (current at otbl_create)
@@ -165,6 +178,13 @@ struct Box {
   int xseg = 1;
   // largest segment count the x systems allow (1: segments off)
   int xseg_max = 1;
+  // x lines on the chunked kernels (else the windowed or marching ones): the
+  // plans of the interpolations and of the derivatives (L 0: these are not)
+  // and their tables
+  bool xchunk = false;
+  XChunk xci, xcd;
+  double *xtab = nullptr;
+  float *xtab_f = nullptr;
   // plane run of the element-wise predictor / projection kernels (0: the
   // default for the element size)
   int prun = 0;
@@ -301,6 +321,12 @@ void kx_interpxx(Box &b, const T *gen, T *geni, const T *icon, const T *econ, in
 template <typename T>
 void kx_difvisxx(Box &b, const T *prod, const T *vel, T *out, const T *icon, const T *iconv, const T *econ,
                  const T *econv, int chv, int ic, size_t P, int mode);
+// chunked x lines (otbl_xchunk.hip), valid when Box::xchunk (the derivatives:
+// and xcd.L)
+void kxc_tables(Box &b);
+template <typename T> void kxc_interpxx(Box &b, const T *gen, T *geni, int which_u, int chi, int chi2, size_t P);
+template <typename T>
+void kxc_difvisxx(Box &b, const T *prod, const T *vel, T *out, int which_u, int chv, int ic, size_t P, int mode);
 // register-resident z transforms (otbl_zfft.hip), valid when Box::zfast /
 // Box::dct_zfast
 // Lp lines of the Poisson x transforms on pencils (all (ny-1)*nz1 lines,

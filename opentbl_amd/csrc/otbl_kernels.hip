@@ -185,6 +185,10 @@ void k_interpxx(Box &b, const double *gen, double *geni, int R, int which_u) {
   const double *econ = which_u ? b.dc.cofiux : b.dc.cofivx;
   int chi = which_u ? 2 : 1;
   int chi2 = which_u ? chi + 1 : chi + 3;
+  if (b.xchunk) {
+    kxc_interpxx(b, gen, geni, which_u, chi, chi2, P);
+    return;
+  }
   if (b.xwin) {
     kx_interpxx(b, gen, geni, icon, econ, chi, chi2, P);
     return;
@@ -263,6 +267,10 @@ void k_difvisxx(Box &b, const double *prod, const double *vel, double *out, int 
   size_t P = (size_t)b.nz1 * R;
   const DevCoef &c = b.dc;
   int vel_u = which_u; // viscous coefficient set: u (ic=3) or v/w (ic=1)
+  if (b.xchunk && b.xcd.L) {
+    kxc_difvisxx(b, prod, vel, out, which_u, which_u ? 1 : 2, vel_u ? 3 : 1, P, mode);
+    return;
+  }
   if (b.xwin) {
     kx_difvisxx(b, prod, vel, out, which_u ? c.dcxu : c.dcxv, which_u ? c.vixu : c.vixv,
                 which_u ? c.cofcxu : c.cofcxv, which_u ? c.cofvxu : c.cofvxv, which_u ? 1 : 2, vel_u ? 3 : 1, P,
@@ -273,6 +281,35 @@ void k_difvisxx(Box &b, const double *prod, const double *vel, double *out, int 
          which_u ? c.dcxu : c.dcxv, which_u ? c.vixu : c.vixv, which_u ? c.cofcxu : c.cofcxv,
          which_u ? c.cofvxu : c.cofvxv, c.dcbx, c.cofvbx, which_u ? 1 : 2, vel_u ? 3 : 1, b.nx,
          P, b.hc.rex, b.hc.idx, mode);
+}
+
+// the x operators of the substep in the element type of the fields (FP32: no
+// marching kernels)
+template <typename T> static void x_interp(Box &b, const T *gen, T *geni, int R, int which_u) {
+  if constexpr (sizeof(T) == 8) {
+    k_interpxx(b, gen, geni, R, which_u);
+  } else {
+    const DevCoefT<T> &c = coefs<T>(b);
+    const size_t P = (size_t)b.nz1 * R;
+    const int chi = which_u ? 2 : 1, chi2 = which_u ? 3 : 4;
+    if (b.xchunk) kxc_interpxx<T>(b, gen, geni, which_u, chi, chi2, P);
+    else kx_interpxx<T>(b, gen, geni, which_u ? c.inxu : c.inxv, which_u ? c.cofiux : c.cofivx, chi, chi2, P);
+  }
+}
+template <typename T>
+static void x_difvis(Box &b, const T *prod, const T *vel, T *out, int R, int which_u, int mode) {
+  if constexpr (sizeof(T) == 8) {
+    k_difvisxx(b, prod, vel, out, R, which_u, mode);
+  } else {
+    const DevCoefT<T> &c = coefs<T>(b);
+    const size_t P = (size_t)b.nz1 * R;
+    const int chv = which_u ? 1 : 2, ic = which_u ? 3 : 1;
+    if (b.xchunk && b.xcd.L)
+      kxc_difvisxx<T>(b, prod, vel, out, which_u, chv, ic, P, mode);
+    else
+      kx_difvisxx<T>(b, prod, vel, out, which_u ? c.dcxu : c.dcxv, which_u ? c.vixu : c.vixv,
+                     which_u ? c.cofcxu : c.cofcxv, which_u ? c.cofvxu : c.cofvxv, chv, ic, P, mode);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2267,15 +2304,9 @@ template <typename T> static void rhsp_t(Box &b, int m) {
     });
   }
   // x interpolation (rhsp.F90:105-107)
-  if constexpr (F64) {
-    k_interpxx(b, u, wki1, ru, 1);
-    k_interpxx(b, v, wki2, ny, 0);
-    k_interpxx(b, w, wki3, ru, 0);
-  } else {
-    kx_interpxx<T>(b, u, wki1, c.inxu, c.cofiux, 2, 3, b.pu);
-    kx_interpxx<T>(b, v, wki2, c.inxv, c.cofivx, 1, 4, b.pv);
-    kx_interpxx<T>(b, w, wki3, c.inxv, c.cofivx, 1, 4, b.pu);
-  }
+  x_interp<T>(b, u, wki1, ru, 1);
+  x_interp<T>(b, v, wki2, ny, 0);
+  x_interp<T>(b, w, wki3, ru, 0);
   if (m == 1)
     LAUNCH(b, "energies", 3, 1024, 0, energies_kernel<T>, u, v, w, b.dc.hy, b.ds, nx, ny, nz1, b.nz2);
   // u interpolated to v rows in spectral space (interpyy is linear along y and
@@ -2301,15 +2332,9 @@ template <typename T> static void rhsp_t(Box &b, int m) {
     LAUNCH(b, "rhsu_loop1", nblk((size_t)nz1 * nx), TPB, 0, rhsu_loop1_kernel, wki2, wki3, rhsu, b.dc, ny, nz1,
            nx);
   // x derivatives (rhsp.F90:181-204)
-  if constexpr (F64) {
-    k_difvisxx(b, wki1, u, rhsu, ru, 1, 1);
-    k_difvisxx(b, wki2, v, rhsv, ny, 0, 0);
-    k_difvisxx(b, wki3, w, rhsw, ru, 0, 0);
-  } else {
-    kx_difvisxx<T>(b, wki1, u, rhsu, c.dcxu, c.vixu, c.cofcxu, c.cofvxu, 1, 3, b.pu, 1);
-    kx_difvisxx<T>(b, wki2, v, rhsv, c.dcxv, c.vixv, c.cofcxv, c.cofvxv, 2, 1, b.pv, 0);
-    kx_difvisxx<T>(b, wki3, w, rhsw, c.dcxv, c.vixv, c.cofcxv, c.cofvxv, 2, 1, b.pu, 0);
-  }
+  x_difvis<T>(b, wki1, u, rhsu, ru, 1, 1);
+  x_difvis<T>(b, wki2, v, rhsv, ny, 0, 0);
+  x_difvis<T>(b, wki3, w, rhsw, ru, 0, 0);
   // time step and RK constants
   LAUNCH(b, "dt", 1, 64, 0, dt_kernel, b.ds, b.vmbits, b.dc.dymin, ny, m, b.dt_mode == OTBL_DT_EVERY_STEP ? 1 : 0,
          b.hc.dxmin, b.hc.dtret, b.hc.rex, b.hc.rkc[m], b.hc.rkd[m], b.hc.rkcv[m], b.hc.rkdv[m]);
@@ -2521,31 +2546,33 @@ template <typename F> static double time_launches(Box &b, int reps, F &&launch) 
 }
 
 template <typename T> static void x_lines_once(Box &b) {
-  const DevCoefT<T> &c = coefs<T>(b);
-  T *u = fld<T>(b.f[OTBL_U]), *wki1 = fld<T>(b.wki1), *rhsu = fld<T>(b.rhsu);
-  if constexpr (sizeof(T) == 8) {
-    k_interpxx(b, u, wki1, b.ny + 1, 1);
-    k_difvisxx(b, wki1, u, rhsu, b.ny + 1, 1, 0);
-  } else {
-    kx_interpxx<T>(b, u, wki1, c.inxu, c.cofiux, 2, 3, b.pu);
-    kx_difvisxx<T>(b, wki1, u, rhsu, c.dcxu, c.vixu, c.cofcxu, c.cofvxu, 1, 3, b.pu, 0);
-  }
+  x_interp<T>(b, fld<T>(b.f[OTBL_U]), fld<T>(b.wki1), b.ny + 1, 1);
+  x_difvis<T>(b, fld<T>(b.wki1), fld<T>(b.f[OTBL_U]), fld<T>(b.rhsu), b.ny + 1, 1, 0);
 }
 
 template <typename T> static std::string autotune_t(Box &b, int reps) {
   char buf[256];
   std::string rep;
-  // x lines: segments per line
+  // x lines: segments per line of the windowed kernels, or the chunked ones
   {
     double best = 1e30;
     int pick = b.xseg;
+    bool chunk = b.xci.L > 0;
+    if (chunk) {
+      b.xchunk = true;
+      best = time_launches(b, reps, [&] { x_lines_once<T>(b); });
+      std::snprintf(buf, sizeof buf, "xchunk=%.4fms ", best);
+      rep += buf;
+    }
+    b.xchunk = false;
     for (int n = 1; n <= b.xseg_max; ++n) {
       b.xseg = n;
       const double ms = time_launches(b, reps, [&] { x_lines_once<T>(b); });
       std::snprintf(buf, sizeof buf, "xseg%d=%.4fms ", n, ms);
       rep += buf;
-      if (ms < best) best = ms, pick = n;
+      if (ms < best) best = ms, pick = n, chunk = false;
     }
+    b.xchunk = chunk;
     b.xseg = pick;
   }
   // element-wise predictor and projection: planes per thread, on work fields

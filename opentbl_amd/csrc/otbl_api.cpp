@@ -385,7 +385,7 @@ static void free_box(Box *b) {
                     b->wki3, b->ya, b->yb, b->yc, b->rest, b->rest2, b->dct2, b->dct3, b->implu,
                     b->implv, b->um, b->u0, b->v0, b->gwork, b->dct_chirp, b->dct_bf, b->dct_tw4,
                     b->ytab, b->ztw, b->zrow, b->dct_ztw, b->rowmax, b->P0, b->S0, b->p0, b->um64, b->rm64,
-                    b->diag, b->op64, b->rthcf, b->st, b->stcoef, b->stmean, b->xtab};
+                    b->diag, b->op64, b->rthcf, b->st, b->stcoef, b->stmean, b->xtab, b->sttab};
   for (double *p : bufs)
     if (p) (void)hipFree(p);
   if (b->diag_count) (void)hipFree(b->diag_count);
@@ -643,9 +643,9 @@ int otbl_create(const otbl_params *prm, const double *y, otbl_ctx **out) {
   b->zpair = std::getenv("OTBL_Z_NOPAIR") ? 0 : (std::getenv("OTBL_ZP_OCC2") ? 2 : 1);
   b->ytail = std::getenv("OTBL_Y_NOTAIL") == nullptr;
   dalloc(b->rowmax, 3 * (size_t)(b->ny + 1) * b->nx);
-  // lengths without such a plan: several rows per wavefront up to 1024, the
-  // LDS kernels beyond (OTBL_Z_LDS, OTBL_Z_STOCKHAM: always)
-  if (!b->zfast && std::getenv("OTBL_Z_STOCKHAM") == nullptr && std::getenv("OTBL_Z_LDS") == nullptr)
+  // rows up to 1024 with several per wavefront; other lengths without an
+  // engine plan on the LDS kernels (OTBL_Z_LDS, OTBL_Z_STOCKHAM: always)
+  if (std::getenv("OTBL_Z_STOCKHAM") == nullptr && (b->zfast || std::getenv("OTBL_Z_LDS") == nullptr))
     b->zteam = zteam_fns(b->nz);
   if (b->zfast || b->zteam.nz) {
     dalloc(b->ztw, 2 * (size_t)b->nz);
@@ -1350,7 +1350,7 @@ int otbl_stats_enable(otbl_ctx *ctx, int on) {
   Box &b = box_of(ctx);
   OTBL_HIP(hipStreamSynchronize(b.s));
   drop_graphs(b); // captured samples hold the old buffers
-  for (double **p : {&b.st, &b.stcoef, &b.stmean})
+  for (double **p : {&b.st, &b.stcoef, &b.stmean, &b.sttab})
     if (*p) {
       (void)hipFree(*p);
       *p = nullptr;
@@ -1369,6 +1369,11 @@ int otbl_stats_enable(otbl_ctx *ctx, int on) {
       c.insert(c.end(), v->begin(), v->end());
     dalloc(b.stcoef, c.size());
     h2d(b, b.stcoef, c.data(), c.size() * sizeof(double));
+    const std::vector<double> t = k_stats_tables(b);
+    if (!t.empty()) {
+      dalloc(b.sttab, t.size());
+      h2d(b, b.sttab, t.data(), t.size() * sizeof(double));
+    }
     dalloc(b.ens, (size_t)b.nz * b.ny * b.nx);
     if (b.precision == OTBL_MIXED) dalloc(b.stmean, 5 * (size_t)b.nx * (b.ny + 1));
     k_stats_attrs(b);

@@ -71,6 +71,8 @@ struct DevScalars {
   double ener[16];
 };
 
+struct StatsZ; // arguments of the statistics' z kernels (otbl_stats_row.h)
+
 // The z kernels with several rows per wavefront (otbl_zteam.h) of one row
 // length: lanes per row, rows per workgroup (of one wavefront), kernels.
 struct ZTeamFns {
@@ -80,12 +82,12 @@ struct ZTeamFns {
   void (*p2d)(const double *, const double *, double *, double *, double *, const double2 *, int, int) = nullptr;
   void (*p2f)(const float *, const float *, float *, float *, float *, const float2 *, int, int) = nullptr;
   void (*fx)(double *, double *, int, const double2 *, int) = nullptr;
+  void (*std_)(StatsZ, const double2 *, int, int, int) = nullptr; // statistics
+  void (*stf)(StatsZ, const float2 *, int, int, int) = nullptr;
 };
 // row lengths of those kernels: even products of 2, 3, 5, 7 from 12 to 1024
-// that the engine of otbl_zfft.h does not run (longer ones stay on the LDS
-// kernels)
 constexpr bool zteam_length(int n) {
-  if (n < 12 || n > 1024 || n % 2 || n == 256 || n == 512 || n == 1024) return false;
+  if (n < 12 || n > 1024 || n % 2) return false;
   for (int p : {2, 3, 5, 7})
     while (n % p == 0) n /= p;
   return n == 1;
@@ -209,7 +211,8 @@ struct Box {
   // twiddle table ztw (nz complex), else the LDS Stockham kernels
   FFTPlan zplan{};
   bool zfast = false;
-  ZTeamFns zteam; // else the kernels with several rows per wavefront (nz != 0)
+  // the kernels with several rows per wavefront (nz != 0): rows of 12 to 1024
+  ZTeamFns zteam;
   // FP32 z products with two rows per team (0: one row, OTBL_Z_NOPAIR; 1:
   // plane loop 1's pair kernel held to three waves per SIMD; 2: to two,
   // OTBL_ZP_OCC2)
@@ -244,6 +247,9 @@ struct Box {
   // bl_1.F90:92 (every avcrt steps after step stest), and the request for
   // a sample at the next substep 1
   double *st = nullptr, *stcoef = nullptr;
+  // chunked x and y lines of the statistics (L 0: one thread per line), tables
+  XChunk stx, sty;
+  double *sttab = nullptr;
   // mixed box: FP64 mean-flow lines of the statistics (u_x, du/dx as
   // [ny+1][nx]; B1, B4, B6 as [ny][nx] in slots of [ny+1][nx])
   double *stmean = nullptr;
@@ -327,7 +333,8 @@ void kxc_tables(Box &b);
 template <typename T> void kxc_interpxx(Box &b, const T *gen, T *geni, int which_u, int chi, int chi2, size_t P);
 template <typename T>
 void kxc_difvisxx(Box &b, const T *prod, const T *vel, T *out, int which_u, int chv, int ic, size_t P, int mode);
-// register-resident z transforms (otbl_zfft.hip), valid when Box::zfast /
+// register-resident transforms (otbl_zfft.hip): the z products and fourxz valid
+// when Box::zfast or Box::zteam.nz, the Poisson x transforms when
 // Box::dct_zfast
 // Lp lines of the Poisson x transforms on pencils (all (ny-1)*nz1 lines,
 // or the 2(ny-1) mean-flow lines of the mixed path), line l at P + l ld
@@ -338,16 +345,13 @@ void kz_rowmax(Box &b);
 template <typename R> void kz_products2(Box &b);
 void kz_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows);
 size_t k_zfft_shm_bytes(int nz, int nbuf);
-// z transforms with several rows per wavefront (otbl_zteam*.hip), valid when
-// Box::zteam.nz
+// kernels with several rows per wavefront (otbl_zteam*.hip)
 ZTeamFns zteam_fns(int nz);
 bool zteam_part1(int n, ZTeamFns &f); // row lengths up to 160
 bool zteam_part2(int n, ZTeamFns &f); // up to 336
 bool zteam_part3(int n, ZTeamFns &f); // up to 600
 bool zteam_part4(int n, ZTeamFns &f); // up to 1024
-template <typename R> void kzt_products1(Box &b);
-template <typename R> void kzt_products2(Box &b);
-void kzt_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows);
+template <typename R> void kzt_stats(Box &b, const StatsZ &a);
 
 // statistics (otbl_stats.hip): one sample of the current state added to
 // Box::st (statsp, stotf.F90:51-291); clearing the accumulators; launch
@@ -355,6 +359,8 @@ void kzt_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows);
 void k_statsp(Box &b);
 void k_stats_zero(Box &b);
 void k_stats_attrs(Box &b);
+// plans Box::stx, sty of the chunked lines and their tables (for Box::sttab)
+std::vector<double> k_stats_tables(Box &b);
 size_t k_stats_shm_bytes(int nz);
 
 // launch bookkeeping (otbl_api.cpp)

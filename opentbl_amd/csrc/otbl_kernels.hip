@@ -837,12 +837,8 @@ fourxz_kernel(double *fou, double *phys, int iopt, FFTPlan plan, int nz1, int nz
 static size_t zfft_shm(const Box &b, int nbuf) { return (TW_SLOTS + (size_t)nbuf * b.nz) * sizeof(double2); }
 
 void k_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows) {
-  if (b.zfast) {
+  if (b.zfast || b.zteam.nz) {
     kz_fourxz(b, fou, phys, iopt, nrows);
-    return;
-  }
-  if (b.zteam.nz) {
-    kzt_fourxz(b, fou, phys, iopt, nrows);
     return;
   }
   LAUNCH(b, "fourxz", nrows, TPB, zfft_shm(b, 2), fourxz_kernel, fou, phys, iopt, b.zplan, b.nz1, b.nz2);
@@ -2316,10 +2312,8 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   else
     ky_interpyy<T>(b, u, yc, 0, 1, nx, b.pu, b.pu);
   // plane loop 1 products
-  if (b.zfast) {
+  if (b.zfast || b.zteam.nz) {
     kz_products1<T>(b);
-  } else if (b.zteam.nz) {
-    kzt_products1<T>(b);
   } else {
     LAUNCH(b, "products1", dim3((ny + b.zrb) / b.zrb, nx), TPB, shm, products1_kernel<T>, u, wki1, wki2, wki3, yc,
            plan, ny, nz1, b.nz2, b.rowmax, nx, b.zrb);
@@ -2377,10 +2371,8 @@ template <typename T> static void rhsp_t(Box &b, int m) {
       ky_interpyy<T>(b, resw, ya, 0, 2, nx - 2, b.pu, b.pu);
       ky_interpyy<T>(b, resv, yb, 1, 2, nx - 2, b.pv, b.pu);
     }
-    if (b.zfast)
+    if (b.zfast || b.zteam.nz)
       kz_products2<T>(b);
-    else if (b.zteam.nz)
-      kzt_products2<T>(b);
     else
       LAUNCH(b, "products2", dim3((ny + b.zrb - 1) / b.zrb, nx - 2), TPB, shm, products2_kernel<T>, resv, resw, ya,
              yb, yc, plan, ny, nz1, b.nz2, b.zrb);

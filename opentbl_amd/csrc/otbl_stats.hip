@@ -23,8 +23,14 @@
 #include "otbl_kcommon.h"
 #include "otbl_fft.h"
 #include "otbl_zfft.h"
+#include "otbl_stats_row.h"
+#include "otbl_chunk.h"
 
+#include <algorithm>
+#include <cmath>
+#include <cstdlib>
 #include <type_traits>
+#include <vector>
 
 namespace otbl {
 
@@ -238,31 +244,341 @@ stats_y_mean_kernel(const double *__restrict__ ux0, const double *__restrict__ d
 }
 
 // ---------------------------------------------------------------------------
+// The same x and y lines split over the wavefronts of a workgroup (the method
+// of otbl_xchunk.hip), in FP64 registers whatever the fields hold: a line's
+// planes or rows are read once and its result is written once.  The marching
+// kernels above write the forward sweep to memory and read it back, one
+// dependent step per plane (1024 x 192 x 256 FP64: 4 x 1033 us in x and 2466 us in
+// y for 0.53 and 3.7 GB).
+// ---------------------------------------------------------------------------
+// Forward sweep in place of a chunk whose raw values are in v: rows j0.. of a
+// system of n; b1, b2 the raw rows before the chunk, a1, a2 those after it.
+// Interior rows take the weights wt(q, r), q = 1..5, of rows j-2..j+2; rows 0, 1
+// (the first nlo of them) take lo[], n-2 and n-1 hi[].  Returns y of the last
+// row.
+template <int L, class Wt, class Mu>
+__device__ __forceinline__ double st_forward(double (&v)[L], Wt wt, Mu mu, int j0, int n, double b2, double b1,
+                                             double a1, double a2, const double (&lo)[2], int nlo,
+                                             const double (&hi)[2]) {
+  double y = 0.0;
+#pragma unroll
+  for (int r = 0; r < L; ++r) {
+    if (r % 2 == 0) XFENCE();
+    const int j = j0 + r;
+    const double p1 = r + 1 < L ? v[r + 1 < L ? r + 1 : 0] : a1;
+    const double p2 = r + 2 < L ? v[r + 2 < L ? r + 2 : 0] : (r + 2 == L ? a1 : a2);
+    double x = wt(1, r) * b2 + wt(2, r) * b1 + wt(3, r) * v[r] + wt(4, r) * p1 + wt(5, r) * p2;
+    if (j < nlo) x = j == 0 ? lo[0] : lo[1];
+    if (j >= n - 2) x = j == n - 2 ? hi[0] : hi[1];
+    x = j < n ? x : 0.0;
+    y = x + mu(r) * y;
+    b2 = b1;
+    b1 = v[r];
+    v[r] = y;
+  }
+  XFENCE();
+  return y;
+}
+
+// x lines: KIND 0 d/dx, KIND 1 the midpoint interpolation written one plane up
+template <int L, int KIND, typename T>
+__global__ void __launch_bounds__(XCT)
+stats_xc(const T *__restrict__ in, T *__restrict__ out, const double *__restrict__ tab, const double *__restrict__ c,
+         int nx, size_t P, XChunk x) {
+  __shared__ double xch[2 * XCT];
+  const XPlace w(x, P);
+  const XTabP<double, 1> t(tab, x, L, w.c);
+  const int j0 = w.c * L;
+  auto G = [&](int j) -> double { return (double)(in + (size_t)min(max(j, 0), nx - 1) * P)[w.l]; };
+  double v[L];
+  if (w.act) {
+    T raw[L];
+#pragma unroll
+    for (int r = 0; r < L; ++r) raw[r] = (in + (size_t)min(j0 + r, nx - 1) * P)[w.l];
+    const double b2 = G(j0 - 2), b1 = G(j0 - 1), a1 = G(j0 + L), a2 = G(j0 + L + 1);
+    constexpr int NW = KIND == 0 ? 5 : 4, NLO = KIND == 0 ? 2 : 1;
+    double lo[2] = {0.0, 0.0}, hi[2] = {0.0, 0.0};
+    if (j0 == 0)
+      for (int k = 0; k < NLO; ++k)
+        for (int q = 1; q <= NW; ++q) lo[k] += F8(c, q, k + 1) * G(q - 1);
+    if (j0 + L >= nx - 1)
+      for (int k = 0; k < 2; ++k)
+        for (int q = 1; q <= NW; ++q) hi[k] += F8(c, q, nx - 1 + k) * G(nx - 1 - NW + q);
+#pragma unroll
+    for (int r = 0; r < L; ++r) v[r] = (double)raw[r];
+    // interior rows: row 3's weights on planes j-2..j+2, or j-1..j+2
+    double wi[5];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) wi[q] = KIND == 0 ? F8(c, q + 1, 3) : (q ? F8(c, q, 3) : 0.0);
+    const double y = st_forward<L>(
+        v, [&](int q, int) { return wi[q - 1]; }, [&](int r) { return t.M(r); }, j0, nx, b2, b1, a1, a2, lo, NLO, hi);
+    xback<L>(v, t);
+    xch[w.p * 64 + w.lane] = y;
+    xch[XCT + w.p * 64 + w.lane] = v[0];
+  }
+  __syncthreads();
+  if (!w.own) return;
+  double C, D;
+  xcarry(xch, xch + XCT, t, w, x.depth, C, D);
+#pragma unroll
+  for (int r = 0; r < L; ++r) {
+    if (r % XGRP == 0) XFENCE();
+    const int j = j0 + r;
+    const T o = (T)(v[r] + C * t.G(r) + D * t.S(r));
+    if (KIND == 0) {
+      if (w.ok && j < nx) (out + (size_t)j * P)[w.l] = o;
+    } else {
+      // u_x(i+1) = I(i); u_x(1) = I(1); I(nx) falls off
+      if (w.ok && j < nx - 1) (out + (size_t)(j + 1) * P)[w.l] = o;
+      if (w.ok && j == 0) out[w.l] = o;
+    }
+  }
+}
+
+// One chain of y solves per blockIdx.y: 0 u_x -> B1 -> B6, 1 w -> B2 -> B7, 2
+// dw/dx -> B3, 3 du/dx -> B4, 4 p -> B5, 5 v -> B8.  A workgroup takes 64 columns
+// (kr, plane), wavefront p rows p L .. of them; the derivative of a solved
+// column takes its neighbours' rows through LDS.
+template <int L, typename T>
+__global__ void __launch_bounds__(XCT)
+stats_yc(StatsY a, const double *__restrict__ tiy, const double *__restrict__ tiyp, const double *__restrict__ tdy,
+         int nx, int ny, int nz1, XChunk x) {
+  __shared__ double xch[2 * XCT], edge[5 * XCT];
+  const int chain = blockIdx.y;
+  ChunkAt w;
+  w.lane = threadIdx.x & 63;
+  w.p = w.c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  w.c0 = 0;
+  w.nact = x.nc;
+  const size_t cg = (size_t)blockIdx.x * 64 + w.lane;
+  const bool ok = cg < (size_t)nz1 * nx, act = w.p < x.nc;
+  const size_t col = ok ? cg : 0, i = col / nz1, kr = col - i * nz1;
+  const size_t ou = i * (size_t)(ny + 1) * nz1 + kr, ov = i * (size_t)ny * nz1 + kr;
+  const int j0 = w.p * L;
+  const size_t s = nz1;
+  double v[L];
+  // correction and store of a solved chunk
+  auto finish = [&](const XTabP<double, 6> &t, double y, T *out) {
+    __syncthreads(); // earlier readers of xch are done
+    if (act) {
+      xch[w.p * 64 + w.lane] = y;
+      xch[XCT + w.p * 64 + w.lane] = v[0];
+    }
+    __syncthreads();
+    if (!act) return;
+    double C, D;
+    xcarry(xch, xch + XCT, t, w, XCH, C, D);
+#pragma unroll
+    for (int r = 0; r < L; ++r) {
+      if (r % XGRP == 0) XFENCE();
+      v[r] = v[r] + C * t.G(r) + D * t.S(r);
+      if (ok && j0 + r < ny) out[(size_t)(j0 + r) * s] = (T)v[r];
+    }
+  };
+  const bool deriv_only = chain == 5;
+  if (!deriv_only) {
+    // midpoint interpolation of nin rows to the ny v rows (1-based rows in the
+    // comments of col_interpy)
+    const int nin = chain == 4 ? ny : ny + 1;
+    const T *g = (const T *)(chain == 0   ? a.ux
+                             : chain == 1 ? a.w
+                             : chain == 2 ? a.dwdx
+                             : chain == 3 ? a.dudx
+                                          : a.p) +
+                 (chain == 4 ? ov : ou);
+    const double *c = chain == 4 ? a.fd_iyp : a.fd_iy;
+    const XTabP<double, 6> t(chain == 4 ? tiyp : tiy, x, L, act ? w.p : 0);
+    auto G = [&](int j) -> double { return (double)g[(size_t)min(max(j, 0), nin - 1) * s]; };
+    double y = 0.0;
+    if (act) {
+      T raw[L];
+#pragma unroll
+      for (int r = 0; r < L; ++r) raw[r] = g[(size_t)min(j0 + r, nin - 1) * s];
+      const double b1 = G(j0 - 1), a1 = G(j0 + L), a2 = G(j0 + L + 1);
+      double lo[2] = {0.0, 0.0}, hi[2] = {0.0, 0.0};
+      if (j0 == 0) {
+        if (chain == 4)
+          for (int q = 1; q <= 4; ++q) lo[0] += F8(c, q, 1) * G(q);
+        for (int q = 1; q <= 5; ++q) lo[1] += F8(c, q, 2) * G(q);
+      }
+      if (j0 + L >= ny - 1)
+        for (int k = 0; k < 2; ++k)
+          for (int q = 1; q <= (chain == 4 ? 3 : 4); ++q) hi[k] += F8(c, q, ny - 1 + k) * G(ny - 4 + q);
+#pragma unroll
+      for (int r = 0; r < L; ++r) v[r] = (double)raw[r];
+      y = st_forward<L>(
+          v, [&](int q, int r) { return t.E(q, r); }, [&](int r) { return t.M(r); }, j0, ny, 0.0, b1, a1, a2, lo, 2,
+          hi);
+      xback<L>(v, t);
+    }
+    finish(t, y, (T *)a.B[chain] + ov);
+    if (chain >= 2) return;
+  }
+  // d/dy of the column in v (chains 0, 1), rounded as it was stored, or of the
+  // field v (chain 5)
+  const XTabP<double, 6> t(tdy, x, L, act ? w.p : 0);
+  double b3 = 0.0, b2 = 0.0, b1 = 0.0, a1 = 0.0, a2 = 0.0;
+  if (deriv_only) {
+    const T *g = (const T *)a.v + ov;
+    auto G = [&](int j) -> double { return (double)g[(size_t)min(max(j, 0), ny - 1) * s]; };
+    T raw[L];
+#pragma unroll
+    for (int r = 0; r < L; ++r) raw[r] = g[(size_t)min(j0 + r, ny - 1) * s];
+    b3 = G(j0 - 3), b2 = G(j0 - 2), b1 = G(j0 - 1), a1 = G(j0 + L), a2 = G(j0 + L + 1);
+#pragma unroll
+    for (int r = 0; r < L; ++r) v[r] = (double)raw[r];
+  } else {
+#pragma unroll
+    for (int r = 0; r < L; ++r) v[r] = (double)(T)v[r];
+    const int at = w.p * 64 + w.lane;
+    if (act) {
+      edge[at] = v[0];
+      edge[XCT + at] = v[1];
+      edge[2 * XCT + at] = v[L - 3];
+      edge[3 * XCT + at] = v[L - 2];
+      edge[4 * XCT + at] = v[L - 1];
+    }
+    __syncthreads();
+    if (act && w.p > 0) b3 = edge[2 * XCT + at - 64], b2 = edge[3 * XCT + at - 64], b1 = edge[4 * XCT + at - 64];
+    if (act && w.p + 1 < x.nc) a1 = edge[at + 64], a2 = edge[XCT + at + 64];
+  }
+  double y = 0.0;
+  if (act) {
+    const double *c = a.fd_dvdy;
+    double lo[2] = {0.0, 0.0}, hi[2] = {0.0, 0.0};
+    if (j0 == 0)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        lo[0] += F8(c, q + 1, 1) * v[q];
+        lo[1] += F8(c, q + 1, 2) * v[q];
+      }
+    if (j0 + L >= ny - 1) {
+      // the last four rows: raw row j of this chunk or just before it (a row
+      // after it, when the chunk ends at row ny-2, is a1)
+      double e[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int j = ny - 4 + q - j0; // row in the chunk
+        double r0 = j == -3 ? b3 : (j == -2 ? b2 : (j == -1 ? b1 : (j == L ? a1 : 0.0)));
+#pragma unroll
+        for (int r = 0; r < L; ++r) r0 = j == r ? v[r] : r0;
+        e[q] = r0;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        hi[0] += F8(c, q + 1, ny - 1) * e[q];
+        hi[1] += F8(c, q + 1, ny) * e[q];
+      }
+    }
+    y = st_forward<L>(
+        v, [&](int q, int r) { return t.E(q, r); }, [&](int r) { return t.M(r); }, j0, ny, b2, b1, a1, a2, lo, 2, hi);
+    xback<L>(v, t);
+  }
+  finish(t, y, (T *)a.B[deriv_only ? 7 : 5 + chain] + ov);
+}
+
+// Table of a stats scheme c (8, n), system rows from f (1-based) on, in chunks
+// of L: FS 1 the multiplier alone, FS 6 weights (rows 3..n-2 on rows j-2..j+2
+// from column col) and the multiplier.
+static void stats_table(std::vector<double> &out, const std::vector<double> &c, int n, int f, int L, int nc, int FS,
+                        int first) {
+  const size_t NL = (size_t)nc * L, at = out.size();
+  out.resize(at + (FS + 4) * NL + 4 * (size_t)nc, 0.0);
+  double *F = out.data() + at, *K = F + FS * NL, *R = K + 2 * NL, *E = R + 2 * NL;
+  auto C = [&](int r, int j) { return c[8 * (size_t)j + r - 1]; };
+  for (int q = 0; q < nc; ++q) {
+    double pr = 1.0;
+    for (int r = 0; r < L; ++r) {
+      const int j = q * L + r, i = j + 1;
+      double m = 0.0, a2 = 0.0, b = 0.0;
+      if (i < f) a2 = 1.0; // a row kept as given
+      else if (i <= n) {
+        m = i == f ? 0.0 : -C(6, i);
+        a2 = C(7, i);
+        b = i == n ? 0.0 : -C(8, i) * C(7, i);
+      }
+      F[FS * (size_t)j + FS - 1] = m;
+      if (FS == 6 && i >= 3 && i <= n - 2)
+        for (int k = 1; k <= 5 && k + first <= 5; ++k) F[6 * (size_t)j + k + first - 1] = C(k, i);
+      K[2 * j] = a2;
+      K[2 * j + 1] = b;
+      pr *= m;
+      R[2 * j] = pr;
+    }
+    E[4 * q] = pr;
+    double g = 0.0, sa = 1.0;
+    for (int r = L - 1; r >= 0; --r) {
+      const int j = q * L + r;
+      g = K[2 * j] * R[2 * j] + K[2 * j + 1] * g;
+      sa *= K[2 * j + 1];
+      R[2 * j] = g;
+      R[2 * j + 1] = sa;
+    }
+    E[4 * q + 1] = g;
+    E[4 * q + 2] = sa;
+  }
+}
+
+// values of a stats table with FS forward values per row
+static size_t stats_table_size(const XChunk &x, int FS) {
+  return (size_t)(FS + 4) * x.nc * x.L + 4 * (size_t)x.nc;
+}
+
+std::vector<double> k_stats_tables(Box &b) {
+  const HostCoef &h = b.hc;
+  std::vector<double> t;
+  b.stx = XChunk();
+  b.sty = XChunk();
+  // products of the multipliers over whole chunks of L planes
+  auto damp = [&](const std::vector<double> &c, int n, int L) {
+    double worst = 0.0;
+    for (int q = 0; (q + 1) * L <= n; ++q) {
+      double m = 1.0, k = 1.0;
+      for (int i = q * L + 1; i <= (q + 1) * L; ++i) {
+        m *= i == 1 ? 0.0 : std::fabs(c[8 * (size_t)i + 5]);
+        k *= i == n ? 0.0 : std::fabs(c[8 * (size_t)i + 7] * c[8 * (size_t)i + 6]);
+      }
+      worst = std::max(worst, std::max(m, k));
+    }
+    return worst;
+  };
+  XChunk x;
+  for (int L = 4; L <= 24 && !x.L; L += 4)
+    if (XCH * L >= b.nx) x.L = L;
+  const bool one = x.L > 0;
+  if (!one) x.L = 24;
+  x.nc = (b.nx + x.L - 1) / x.L;
+  const double worst = std::max(damp(h.fd_dx, b.nx, x.L), damp(h.fd_ix, b.nx, x.L));
+  double p = 1.0;
+  for (x.depth = 0; x.depth < XCH && p >= 1e-19; ++x.depth) p *= worst;
+  bool fit = true;
+  if (!one) {
+    p = 1.0;
+    for (x.halo = 0; x.halo < 5 && p >= 1e-17; ++x.halo) p *= worst;
+    fit = p < 1e-17;
+    if (fit)
+      for (x.ns = 2; (x.nc + x.ns - 1) / x.ns + 2 * x.halo > XCH; ++x.ns) {
+      }
+  }
+  if (fit && std::getenv("OTBL_STATS_MARCH") == nullptr) {
+    b.stx = x;
+    stats_table(t, h.fd_ix, b.nx, 1, x.L, x.nc, 1, 0);
+    stats_table(t, h.fd_dx, b.nx, 1, x.L, x.nc, 1, 0);
+  }
+  if (b.yL && std::getenv("OTBL_STATS_MARCH") == nullptr) {
+    b.sty.L = b.yL;
+    b.sty.nc = (b.ny + b.yL - 1) / b.yL;
+    stats_table(t, h.fd_iy, b.ny, 2, b.yL, b.sty.nc, 6, 1);
+    stats_table(t, h.fd_iyp, b.ny, 2, b.yL, b.sty.nc, 6, 1);
+    stats_table(t, h.fd_dvdy, b.ny, 1, b.yL, b.sty.nc, 6, 0);
+  }
+  return t;
+}
+
+// ---------------------------------------------------------------------------
 // Row sums of one (j, i) row
 // ---------------------------------------------------------------------------
-// accumulator ids (the order of the reference's statistics files:
-// escru.F90:318-341 then 490-516)
-enum {
-  S_US, S_VS, S_WS, S_UV, S_UA, S_VA, S_WA, S_PP, S_PM, S_VORTX, S_VORTY, S_VORTZ, S_VORTXA, S_VORTYA,
-  S_VORTZA, S_UW, S_VW, S_DISPU, S_DISPV, S_DISPW, S_DISPUV, S_PUP, S_PVP, S_PDUDX, S_PDVDY, S_PDUDY,
-  S_PDVDX, S_PDWDZ, S_V3, S_U2V, S_V2U, S_W2V, S_DUDX0, S_DUDY0, S_DVDX0, S_DVDY0, S_DWDX0, S_DWDY0, S_U3,
-  S_W2U, S_COUNT
-};
-static_assert(S_COUNT == OTBL_NSTAT, "statistic count");
-
-// the sums over modes and over z reduced across the workgroup
-constexpr int NSUM = 21 + 6;
 constexpr int ZSLOTS = 4096 / TPB; // physical points per thread (nz <= 4096)
-
-struct StatsZ {
-  const void *B[8], *v, *dvdx;
-  // mixed box: the real part of mode 0 of B1, B4, B6 from the FP64 mean
-  // flow, [ny][nx] (null: from the fields)
-  const double *m1, *m4, *m6;
-  const double *kaz;
-  double *acc; // [S_COUNT][nx][ny+1]
-  float *ens;  // [nx][ny][nz]
-};
 
 template <typename T>
 __global__ void __launch_bounds__(TPB) stats_z_kernel(StatsZ a, FFTPlan plan, int nx, int ny, int nz1, int nz2) {
@@ -287,38 +603,12 @@ __global__ void __launch_bounds__(TPB) stats_z_kernel(StatsZ a, FFTPlan plan, in
   double sum[NSUM];
 #pragma unroll
   for (int q = 0; q < NSUM; ++q) sum[q] = 0.0;
-  auto re = [](double2 x, double2 y) { return x.x * y.x + x.y * y.y; }; // Re(x conj(y))
   for (int k = t; k <= nz2; k += TPB) {
     const double cte = k == 0 ? 1.0 : 2.0, kz = a.kaz[k];
     const double2 b1 = ld(Bq[0], k), b2 = ld(Bq[1], k), b3 = ld(Bq[2], k), b4 = ld(Bq[3], k);
     const double2 b5 = ld(Bq[4], k), b6 = ld(Bq[5], k), b7 = ld(Bq[6], k), b8 = ld(Bq[7], k);
     const double2 v = ld(V, k), dv = ld(DV, k);
-    // z derivatives: x kaz = (-kz x.y, kz x.x)
-    const double2 uz = make_double2(-kz * b1.y, kz * b1.x), vz = make_double2(-kz * v.y, kz * v.x);
-    const double2 wz = make_double2(-kz * b2.y, kz * b2.x);
-    const double2 ox = make_double2(b7.x - vz.x, b7.y - vz.y), oy = make_double2(uz.x - b3.x, uz.y - b3.y);
-    const double2 oz = make_double2(dv.x - b6.x, dv.y - b6.y);
-    sum[0] += cte * re(b1, b1);  // us
-    sum[1] += cte * re(v, v);    // vs
-    sum[2] += cte * re(b2, b2);  // ws
-    sum[3] += cte * re(b1, v);   // uv
-    sum[4] += cte * re(b5, b5);  // pp
-    sum[5] += cte * re(ox, ox);  // vortx
-    sum[6] += cte * re(oy, oy);  // vorty
-    sum[7] += cte * re(oz, oz);  // vortz
-    sum[8] += cte * re(b1, b2);  // uw
-    sum[9] += cte * re(v, b2);   // vw
-    sum[10] += cte * (re(b4, b4) + re(uz, uz) + re(b6, b6)); // dispu
-    sum[11] += cte * (re(dv, dv) + re(vz, vz) + re(b8, b8)); // dispv
-    sum[12] += cte * (re(wz, wz) + re(b3, b3) + re(b7, b7)); // dispw
-    sum[13] += cte * (re(uz, vz) + re(b4, dv) + re(b6, b8)); // dispuv
-    sum[14] += cte * re(b5, b1); // pup
-    sum[15] += cte * re(b5, v);  // pvp
-    sum[16] += cte * re(b5, b4); // pdudx
-    sum[17] += cte * re(b5, b8); // pdvdy
-    sum[18] += cte * re(b5, b6); // pdudy
-    sum[19] += cte * re(b5, dv); // pdvdx
-    sum[20] += cte * re(b5, wz); // pdwdz
+    stats_mode(sum, cte, kz, b1, b2, b3, b4, b5, b6, b7, b8, v, dv);
   }
   // ---- physical space (stotf.F90:148-154, 256-283) ----
   // spectrum of signal q at mode k <= nz2: 0 omega_x, 1 omega_y, 2 omega_z,
@@ -394,55 +684,18 @@ __global__ void __launch_bounds__(TPB) stats_z_kernel(StatsZ a, FFTPlan plan, in
   __syncthreads();
   if (t != 0) return;
 #pragma unroll
-  for (int q = 0; q < NSUM; ++q)
-    for (int w = 1; w < TPB / 64; ++w) red[0][q] += red[w][q];
-  const double *r = red[0];
+  for (int q = 0; q < NSUM; ++q) {
+    sum[q] = red[0][q];
+    for (int w = 1; w < TPB / 64; ++w) sum[q] += red[w][q];
+  }
   const size_t NR = (size_t)(ny + 1), at0 = (size_t)(i - 1) * NR + (j - 1), S = (size_t)nx * NR;
   double *acc = a.acc + at0;
-  acc[S_US * S] += r[0];
-  acc[S_VS * S] += r[1];
-  acc[S_WS * S] += r[2];
-  acc[S_UV * S] += r[3];
-  acc[S_PP * S] += r[4];
-  acc[S_VORTX * S] += r[5];
-  acc[S_VORTY * S] += r[6];
-  acc[S_VORTZ * S] += r[7];
-  acc[S_UW * S] += r[8];
-  acc[S_VW * S] += r[9];
-  acc[S_DISPU * S] += r[10];
-  acc[S_DISPV * S] += r[11];
-  acc[S_DISPW * S] += r[12];
-  acc[S_DISPUV * S] += r[13];
-  acc[S_PUP * S] += r[14];
-  acc[S_PVP * S] += r[15];
-  acc[S_PDUDX * S] += r[16];
-  acc[S_PDVDY * S] += r[17];
-  acc[S_PDUDY * S] += r[18];
-  acc[S_PDVDX * S] += r[19];
-  acc[S_PDWDZ * S] += r[20];
-  acc[S_U3 * S] += r[21];
-  acc[S_W2U * S] += r[22];
-  acc[S_V3 * S] += r[23];
-  acc[S_W2V * S] += r[24];
-  acc[S_V2U * S] += r[25];
-  acc[S_U2V * S] += r[26];
+  stats_add_sums(acc, S, sum);
   // k = 0 means (stotf.F90:128-144): real parts
   const double b1 = ld(Bq[0], 0).x, b2 = (double)Bq[1][0], b3 = (double)Bq[2][0], b4 = ld(Bq[3], 0).x;
   const double b5 = (double)Bq[4][0], b6 = ld(Bq[5], 0).x, b7 = (double)Bq[6][0], b8 = (double)Bq[7][0];
   const double v0 = (double)V[0], dv0 = (double)DV[0];
-  acc[S_UA * S] += b1;
-  acc[S_WA * S] += b2;
-  acc[S_VA * S] += v0;
-  acc[S_PM * S] += b5;
-  acc[S_DUDX0 * S] += b4;
-  acc[S_DVDX0 * S] += dv0;
-  acc[S_DWDX0 * S] += b3;
-  acc[S_DUDY0 * S] += b6;
-  acc[S_DVDY0 * S] += b8;
-  acc[S_DWDY0 * S] += b7;
-  acc[S_VORTYA * S] -= b3;
-  acc[S_VORTXA * S] += b7;
-  acc[S_VORTZA * S] += dv0 - b6;
+  stats_add_means(acc, S, b1, b2, b3, b4, b5, b6, b7, b8, v0, dv0);
 }
 
 // ---------------------------------------------------------------------------
@@ -452,10 +705,6 @@ __global__ void __launch_bounds__(TPB) stats_z_kernel(StatsZ a, FFTPlan plan, in
 // precision in registers (their inputs formed from the spectral rows as
 // they are loaded), the physical products and every sum in FP64.
 // ---------------------------------------------------------------------------
-template <typename C> struct CPair {
-  C x, y;
-};
-
 // Complex input of the c2r transform of two real signals whose spectra
 // spec(k) gives for 0 <= k <= nz2: the Hermitian-extended spectrum of
 // x + i y in the register slots of the engine's first pass (Im of mode 0
@@ -557,7 +806,6 @@ stats_zr(StatsZ a, const typename CT<T>::c *__restrict__ tw, int nx, int ny, int
     }
   }
   // ---- sums over the modes (stotf.F90:156-218), modes t + G it ----
-  auto re = [](double2 x, double2 y) { return x.x * y.x + x.y * y.y; }; // Re(x conj(y))
   auto wd = [](C x) { return make_double2((double)x.x, (double)x.y); };
   // one mode per lane at a time: the 10 loads and 21 FP64 sums of a mode
   // fill the registers the transforms no longer need
@@ -573,31 +821,7 @@ stats_zr(StatsZ a, const typename CT<T>::c *__restrict__ tw, int nx, int ny, int
     }
     const double2 b2 = wd(Bq[1][k]), b3 = wd(Bq[2][k]), b5 = wd(Bq[4][k]), b7 = wd(Bq[6][k]), b8 = wd(Bq[7][k]);
     const double2 v = wd(V[k]), dv = wd(DV[k]);
-    const double2 uz = make_double2(-kz * b1.y, kz * b1.x), vz = make_double2(-kz * v.y, kz * v.x);
-    const double2 wz = make_double2(-kz * b2.y, kz * b2.x);
-    const double2 ox = make_double2(b7.x - vz.x, b7.y - vz.y), oy = make_double2(uz.x - b3.x, uz.y - b3.y);
-    const double2 oz = make_double2(dv.x - b6.x, dv.y - b6.y);
-    sum[0] += cte * re(b1, b1);
-    sum[1] += cte * re(v, v);
-    sum[2] += cte * re(b2, b2);
-    sum[3] += cte * re(b1, v);
-    sum[4] += cte * re(b5, b5);
-    sum[5] += cte * re(ox, ox);
-    sum[6] += cte * re(oy, oy);
-    sum[7] += cte * re(oz, oz);
-    sum[8] += cte * re(b1, b2);
-    sum[9] += cte * re(v, b2);
-    sum[10] += cte * (re(b4, b4) + re(uz, uz) + re(b6, b6));
-    sum[11] += cte * (re(dv, dv) + re(vz, vz) + re(b8, b8));
-    sum[12] += cte * (re(wz, wz) + re(b3, b3) + re(b7, b7));
-    sum[13] += cte * (re(uz, vz) + re(b4, dv) + re(b6, b8));
-    sum[14] += cte * re(b5, b1);
-    sum[15] += cte * re(b5, v);
-    sum[16] += cte * re(b5, b4);
-    sum[17] += cte * re(b5, b8);
-    sum[18] += cte * re(b5, b6);
-    sum[19] += cte * re(b5, dv);
-    sum[20] += cte * re(b5, wz);
+    stats_mode(sum, cte, kz, b1, b2, b3, b4, b5, b6, b7, b8, v, dv);
   }
   // ---- reduce across the team ----
 #pragma unroll
@@ -615,29 +839,13 @@ stats_zr(StatsZ a, const typename CT<T>::c *__restrict__ tw, int nx, int ny, int
   if (t != 0) return;
   const size_t NR = (size_t)(ny + 1), at0 = (size_t)(i - 1) * NR + (j - 1), S = (size_t)nx * NR;
   double *acc = a.acc + at0;
-  constexpr int ID[NSUM] = {S_US,   S_VS,    S_WS,    S_UV,    S_PP,    S_VORTX, S_VORTY, S_VORTZ, S_UW,
-                            S_VW,   S_DISPU, S_DISPV, S_DISPW, S_DISPUV, S_PUP,  S_PVP,   S_PDUDX, S_PDVDY,
-                            S_PDUDY, S_PDVDX, S_PDWDZ, S_U3,   S_W2U,   S_V3,    S_W2V,   S_V2U,   S_U2V};
-#pragma unroll
-  for (int q = 0; q < NSUM; ++q) acc[ID[q] * S] += sum[q];
+  stats_add_sums(acc, S, sum);
   // k = 0 means (stotf.F90:128-144): real parts
   const double b1 = a.m1 ? a.m1[om] : (double)Bq[0][0].x, b4 = a.m1 ? a.m4[om] : (double)Bq[3][0].x;
   const double b6 = a.m1 ? a.m6[om] : (double)Bq[5][0].x;
   const double b2 = Bq[1][0].x, b3 = Bq[2][0].x, b5 = Bq[4][0].x, b7 = Bq[6][0].x, b8 = Bq[7][0].x;
   const double v0 = V[0].x, dv0 = DV[0].x;
-  acc[S_UA * S] += b1;
-  acc[S_WA * S] += b2;
-  acc[S_VA * S] += v0;
-  acc[S_PM * S] += b5;
-  acc[S_DUDX0 * S] += b4;
-  acc[S_DVDX0 * S] += dv0;
-  acc[S_DWDX0 * S] += b3;
-  acc[S_DUDY0 * S] += b6;
-  acc[S_DVDY0 * S] += b8;
-  acc[S_DWDY0 * S] += b7;
-  acc[S_VORTYA * S] -= b3;
-  acc[S_VORTXA * S] += b7;
-  acc[S_VORTZA * S] += dv0 - b6;
+  stats_add_means(acc, S, b1, b2, b3, b4, b5, b6, b7, b8, v0, dv0);
 }
 
 __global__ void stats_zero_kernel(double *a, size_t n) {
@@ -645,6 +853,17 @@ __global__ void stats_zero_kernel(double *a, size_t n) {
 }
 
 size_t k_stats_shm_bytes(int nz) { return (192 + 2 * (size_t)nz) * sizeof(double2); }
+
+#define SDISPATCH(LL, ...)                                                     \
+  switch (LL) {                                                                \
+  case 4: { constexpr int L = 4; __VA_ARGS__; } break;                         \
+  case 8: { constexpr int L = 8; __VA_ARGS__; } break;                         \
+  case 12: { constexpr int L = 12; __VA_ARGS__; } break;                       \
+  case 16: { constexpr int L = 16; __VA_ARGS__; } break;                       \
+  case 20: { constexpr int L = 20; __VA_ARGS__; } break;                       \
+  case 24: { constexpr int L = 24; __VA_ARGS__; } break;                       \
+  default: throw std::invalid_argument("stats: chunk length not instantiated"); \
+  }
 
 template <typename T> static void statsp_t(Box &b) {
   const int nx = b.nx, ny = b.ny, nz1 = b.nz1;
@@ -655,10 +874,24 @@ template <typename T> static void statsp_t(Box &b) {
              fld<T>(b.yb),   fld<T>(b.yc),   fld<T>(b.resv), fld<T>(b.wki2)};
   const double *fd_dvdy = b.stcoef, *fd_iy = fd_dvdy + 8 * (size_t)(ny + 1), *fd_iyp = fd_iy + 8 * (size_t)(ny + 1);
   const double *fd_dx = fd_iyp + 8 * (size_t)(ny + 1), *fd_ix = fd_dx + 8 * (size_t)(nx + 1);
-  LAUNCH(b, "stats_x", nblk(b.pu), TPB, 0, (stats_x_kernel<T, 1>), u, ux, fd_ix, nx, b.pu, 1, b.pu);
-  LAUNCH(b, "stats_x", nblk(b.pu), TPB, 0, (stats_x_kernel<T, 0>), ux, dudx, fd_dx, nx, b.pu, 1, b.pu);
-  LAUNCH(b, "stats_x", nblk(b.pv), TPB, 0, (stats_x_kernel<T, 0>), v, dvdx, fd_dx, nx, b.pv, 1, b.pv);
-  LAUNCH(b, "stats_x", nblk(b.pu), TPB, 0, (stats_x_kernel<T, 0>), w, dwdx, fd_dx, nx, b.pu, 1, b.pu);
+  if (b.stx.L) {
+    const double *ti = b.sttab, *td = ti + stats_table_size(b.stx, 1);
+    auto line = [&](auto interp, const T *in, T *out, size_t P) {
+      constexpr int KIND = decltype(interp)::value;
+      const unsigned grid = nblk(P, 64) * (unsigned)b.stx.ns;
+      SDISPATCH(b.stx.L, auto kf = &stats_xc<L, KIND, T>;
+                LAUNCH(b, "stats_x", grid, XCT, 0, kf, in, out, KIND ? ti : td, KIND ? fd_ix : fd_dx, nx, P, b.stx));
+    };
+    line(std::integral_constant<int, 1>(), u, ux, b.pu);
+    line(std::integral_constant<int, 0>(), ux, dudx, b.pu);
+    line(std::integral_constant<int, 0>(), v, dvdx, b.pv);
+    line(std::integral_constant<int, 0>(), w, dwdx, b.pu);
+  } else {
+    LAUNCH(b, "stats_x", nblk(b.pu), TPB, 0, (stats_x_kernel<T, 1>), u, ux, fd_ix, nx, b.pu, 1, b.pu);
+    LAUNCH(b, "stats_x", nblk(b.pu), TPB, 0, (stats_x_kernel<T, 0>), ux, dudx, fd_dx, nx, b.pu, 1, b.pu);
+    LAUNCH(b, "stats_x", nblk(b.pv), TPB, 0, (stats_x_kernel<T, 0>), v, dvdx, fd_dx, nx, b.pv, 1, b.pv);
+    LAUNCH(b, "stats_x", nblk(b.pu), TPB, 0, (stats_x_kernel<T, 0>), w, dwdx, fd_dx, nx, b.pu, 1, b.pu);
+  }
   // mixed box: the mean-flow u (mode 0, real part) is held in FP64 (its
   // FP32 rounding, amplified by d/dx, would swamp du/dx of the mean flow);
   // its lines run in FP64 beside the FP32 fields
@@ -677,7 +910,15 @@ template <typename T> static void statsp_t(Box &b) {
   }
   StatsY ay{ux, w, dwdx, dudx, p, v, {}, fd_iy, fd_iyp, fd_dvdy};
   for (int q = 0; q < 8; ++q) ay.B[q] = B[q];
-  LAUNCH(b, "stats_y", nblk((size_t)nz1 * nx), TPB, 0, stats_y_kernel<T>, ay, nx, ny, nz1);
+  if (b.sty.L) {
+    const double *tiy = b.sttab + (b.stx.L ? 2 * stats_table_size(b.stx, 1) : 0);
+    const double *tiyp = tiy + stats_table_size(b.sty, 6), *tdy = tiyp + stats_table_size(b.sty, 6);
+    SDISPATCH(b.sty.L, auto kf = &stats_yc<L, T>;
+              LAUNCH(b, "stats_y", dim3(nblk((size_t)nz1 * nx, 64), 6), XCT, 0, kf, ay, tiy, tiyp, tdy, nx, ny, nz1,
+                     b.sty));
+  } else {
+    LAUNCH(b, "stats_y", nblk((size_t)nz1 * nx), TPB, 0, stats_y_kernel<T>, ay, nx, ny, nz1);
+  }
   if (m1)
     LAUNCH(b, "stats_y", nblk(nx), TPB, 0, stats_y_mean_kernel, (const double *)ux0, (const double *)dudx0, m1, m4,
            m6, fd_iy, fd_dvdy, nx, ny);
@@ -691,6 +932,10 @@ template <typename T> static void statsp_t(Box &b) {
   az.kaz = b.dc.kaz;
   az.acc = b.st;
   az.ens = b.ens;
+  if (b.zteam.nz) {
+    kzt_stats<T>(b, az);
+    return;
+  }
   if (b.zfast) {
     const int nrows = ny * nx;
     const typename CT<T>::c *tw = std::is_same<T, double>::value ? (const typename CT<T>::c *)b.ztw
@@ -701,9 +946,6 @@ template <typename T> static void statsp_t(Box &b) {
            (stats_zr<NN, T>), az, tw, nx, ny, nz1, nrows);                                                      \
     break;
     switch (b.nz) {
-      SZR(256)
-      SZR(512)
-      SZR(1024)
       SZR(2048)
       SZR(4096)
 #undef SZR

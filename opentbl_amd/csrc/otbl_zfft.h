@@ -25,10 +25,6 @@ namespace otbl {
 
 // radix plans (the inverse runs the radices in reverse order)
 template <int N> struct ZPlan;
-template <> struct ZPlan<256> {
-  static constexpr int W = 1, NP = 4;
-  static constexpr int rad(int p) { return 4; }
-};
 template <> struct ZPlan<512> {
   static constexpr int W = 1, NP = 3;
   static constexpr int rad(int p) { return 8; }

@@ -4,6 +4,7 @@
 // movement, one LDS exchange buffer per team.
 #include "otbl_kcommon.h"
 #include "otbl_zfft.h"
+#include "otbl_stats_row.h"
 
 #include <type_traits>
 
@@ -492,13 +493,22 @@ dct_rows_z(const R *src, R *dst, int Lp, int N, int ld, const typename CT<R>::c 
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+#define ZCASE(NN, ...) case NN: { constexpr int N = NN; __VA_ARGS__; } break;
+// rows of one wavefront or more: the lengths beyond those with several rows
+// per wavefront, and for the FP32 pair kernel 512 and 1024 too (there it is
+// the faster one: 396 against 430 us on a 512 x 192 x 512 box)
 #define ZDISPATCH(n, ...)                                                      \
   switch (n) {                                                                 \
-  case 256: { constexpr int N = 256; __VA_ARGS__; } break;                     \
-  case 512: { constexpr int N = 512; __VA_ARGS__; } break;                     \
-  case 1024: { constexpr int N = 1024; __VA_ARGS__; } break;                   \
-  case 2048: { constexpr int N = 2048; __VA_ARGS__; } break;                   \
-  case 4096: { constexpr int N = 4096; __VA_ARGS__; } break;                   \
+  ZCASE(2048, __VA_ARGS__)                                                     \
+  ZCASE(4096, __VA_ARGS__)                                                     \
+  default: throw std::invalid_argument("z transform length not instantiated"); \
+  }
+#define ZDISPATCH_PAIR(n, ...)                                                 \
+  switch (n) {                                                                 \
+  ZCASE(512, __VA_ARGS__)                                                      \
+  ZCASE(1024, __VA_ARGS__)                                                     \
+  ZCASE(2048, __VA_ARGS__)                                                     \
+  ZCASE(4096, __VA_ARGS__)                                                     \
   default: throw std::invalid_argument("z transform length not instantiated"); \
   }
 
@@ -516,24 +526,58 @@ template <typename R> static const typename CT<R>::c *ztw(const Box &b);
 template <> const double2 *ztw<double>(const Box &b) { return (const double2 *)b.ztw; }
 template <> const float2 *ztw<float>(const Box &b) { return (const float2 *)b.ztw_f; }
 
+// ---------------------------------------------------------------------------
+// several rows per wavefront (otbl_zteam.h)
+// ---------------------------------------------------------------------------
+ZTeamFns zteam_fns(int nz) {
+  ZTeamFns f;
+  if (zteam_length(nz))
+    (void)(zteam_part1(nz, f) || zteam_part2(nz, f) || zteam_part3(nz, f) || zteam_part4(nz, f));
+  return f;
+}
+
+static unsigned tgrid(const Box &b, int nrows) { return (unsigned)((nrows + b.zteam.rows - 1) / b.zteam.rows); }
+
+template <typename R> static void team_products1(Box &b) {
+  const int nrows = (b.ny + 1) * b.nx;
+  auto launch = [&](auto kf) {
+    LAUNCH(b, "products1", tgrid(b, nrows), 64, 0, kf, (const R *)fld<R>(b.f[OTBL_U]), fld<R>(b.wki1), fld<R>(b.wki2),
+           fld<R>(b.wki3), (const R *)fld<R>(b.yc), ztw<R>(b), b.ny, nrows, b.rowmax);
+  };
+  if constexpr (sizeof(R) == 8) launch(b.zteam.p1d);
+  else launch(b.zteam.p1f);
+}
+
+template <typename R> static void team_products2(Box &b) {
+  const int nrows = b.ny * (b.nx - 2);
+  auto launch = [&](auto kf) {
+    LAUNCH(b, "products2", tgrid(b, nrows), 64, 0, kf, (const R *)fld<R>(b.resv), (const R *)fld<R>(b.resw),
+           fld<R>(b.ya), fld<R>(b.yb), fld<R>(b.yc), ztw<R>(b), b.ny, nrows);
+  };
+  if constexpr (sizeof(R) == 8) launch(b.zteam.p2d);
+  else launch(b.zteam.p2f);
+}
+
 template <typename R> void kz_products1(Box &b) {
   zcheck(b);
   const int nrows = (b.ny + 1) * b.nx;
   const R *zrow = fld<R>(b.zrow);
-  if (std::is_same<R, float>::value && b.zpair) {
+  if (std::is_same<R, float>::value && b.zpair && b.zfast && b.nz > 256) {
     // FP32: two rows per team (the registers two rows need are there in FP32)
     const float *zr = (const float *)b.zrow;
     if (b.zpair == 1) {
-      ZDISPATCH(b.nz, auto kf = &products1_zp<N, 3>;
+      ZDISPATCH_PAIR(b.nz, auto kf = &products1_zp<N, 3>;
                 LAUNCH(b, "products1", zgrid<N>((nrows + 1) / 2), ZTeam<N>::TPB_, 0, kf, fld<float>(b.f[OTBL_U]),
                        fld<float>(b.wki1), fld<float>(b.wki2), fld<float>(b.wki3), fld<float>(b.yc),
                        (const float2 *)b.ztw_f, zr, b.ny, b.nz1, b.nz2, nrows, b.rowmax));
     } else {
-      ZDISPATCH(b.nz, auto kf = &products1_zp<N, 1>;
+      ZDISPATCH_PAIR(b.nz, auto kf = &products1_zp<N, 1>;
                 LAUNCH(b, "products1", zgrid<N>((nrows + 1) / 2), ZTeam<N>::TPB_, 0, kf, fld<float>(b.f[OTBL_U]),
                        fld<float>(b.wki1), fld<float>(b.wki2), fld<float>(b.wki3), fld<float>(b.yc),
                        (const float2 *)b.ztw_f, zr, b.ny, b.nz1, b.nz2, nrows, b.rowmax));
     }
+  } else if (b.zteam.nz) {
+    team_products1<R>(b);
   } else {
     ZDISPATCH(b.nz, auto kf = &products1_z<N, R>;
               LAUNCH(b, "products1", zgrid<N>(nrows), ZTeam<N>::TPB_, 0, kf, fld<R>(b.f[OTBL_U]), fld<R>(b.wki1),
@@ -549,6 +593,10 @@ void kz_rowmax(Box &b) {
 
 template <typename R> void kz_products2(Box &b) {
   zcheck(b);
+  if (b.zteam.nz) {
+    team_products2<R>(b);
+    return;
+  }
   const int nrows = b.ny * (b.nx - 2);
   ZDISPATCH(b.nz, auto kf = &products2_z<N, R>;
             LAUNCH(b, "products2", zgrid<N>(nrows), ZTeam<N>::TPB_, 0, kf, fld<R>(b.resv), fld<R>(b.resw),
@@ -588,50 +636,16 @@ template <> void kz_dct_pencils<float>(Box &b, float *P, int iopt, int Lp, int l
   dct_launch<float>(b, P, iopt, Lp, ld, b.dct_chirp_f, b.dct_bf_f, b.dct_tw4_f, b.dct_ztw_f);
 }
 
-// ---------------------------------------------------------------------------
-// several rows per wavefront (otbl_zteam.h)
-// ---------------------------------------------------------------------------
-ZTeamFns zteam_fns(int nz) {
-  ZTeamFns f;
-  if (zteam_length(nz))
-    (void)(zteam_part1(nz, f) || zteam_part2(nz, f) || zteam_part3(nz, f) || zteam_part4(nz, f));
-  return f;
-}
-
-static unsigned tgrid(const Box &b, int nrows) { return (unsigned)((nrows + b.zteam.rows - 1) / b.zteam.rows); }
-
-template <typename R> void kzt_products1(Box &b) {
+template <typename R> void kzt_stats(Box &b, const StatsZ &a) {
   zcheck(b);
-  const int nrows = (b.ny + 1) * b.nx;
-  auto launch = [&](auto kf) {
-    LAUNCH(b, "products1", tgrid(b, nrows), 64, 0, kf, (const R *)fld<R>(b.f[OTBL_U]), fld<R>(b.wki1), fld<R>(b.wki2),
-           fld<R>(b.wki3), (const R *)fld<R>(b.yc), ztw<R>(b), b.ny, nrows, b.rowmax);
-  };
-  if constexpr (sizeof(R) == 8) launch(b.zteam.p1d);
-  else launch(b.zteam.p1f);
-  kz_rowmax(b);
+  const int nrows = b.ny * b.nx;
+  auto launch = [&](auto kf) { LAUNCH(b, "stats_z", tgrid(b, nrows), 64, 0, kf, a, ztw<R>(b), b.nx, b.ny, nrows); };
+  if constexpr (sizeof(R) == 8) launch(b.zteam.std_);
+  else launch(b.zteam.stf);
 }
 
-template <typename R> void kzt_products2(Box &b) {
-  zcheck(b);
-  const int nrows = b.ny * (b.nx - 2);
-  auto launch = [&](auto kf) {
-    LAUNCH(b, "products2", tgrid(b, nrows), 64, 0, kf, (const R *)fld<R>(b.resv), (const R *)fld<R>(b.resw),
-           fld<R>(b.ya), fld<R>(b.yb), fld<R>(b.yc), ztw<R>(b), b.ny, nrows);
-  };
-  if constexpr (sizeof(R) == 8) launch(b.zteam.p2d);
-  else launch(b.zteam.p2f);
-}
-
-void kzt_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows) {
-  zcheck(b);
-  LAUNCH(b, "fourxz", tgrid(b, nrows), 64, 0, b.zteam.fx, fou, phys, iopt, (const double2 *)b.ztw, nrows);
-}
-
-template void kzt_products1<double>(Box &);
-template void kzt_products1<float>(Box &);
-template void kzt_products2<double>(Box &);
-template void kzt_products2<float>(Box &);
+template void kzt_stats<double>(Box &, const StatsZ &);
+template void kzt_stats<float>(Box &, const StatsZ &);
 template void kz_products1<double>(Box &);
 template void kz_products1<float>(Box &);
 template void kz_products2<double>(Box &);
@@ -639,6 +653,10 @@ template void kz_products2<float>(Box &);
 
 void kz_fourxz(Box &b, double *fou, double *phys, int iopt, int nrows) {
   zcheck(b);
+  if (b.zteam.nz) {
+    LAUNCH(b, "fourxz", tgrid(b, nrows), 64, 0, b.zteam.fx, fou, phys, iopt, (const double2 *)b.ztw, nrows);
+    return;
+  }
   ZDISPATCH(b.nz, auto kf = &fourxz_z<N>;
             LAUNCH(b, "fourxz", zgrid<N>(nrows), ZTeam<N>::TPB_, 0, kf, fou, phys, iopt, (const double2 *)b.ztw,
                    b.zrow, b.nz1, b.nz2, nrows));

@@ -386,14 +386,14 @@ template <typename C, typename R> __device__ __forceinline__ void tst(R *base, u
   *(C *)((char *)base + at * (unsigned)sizeof(C)) = v;
 }
 
-// The first pass's inputs from the spectral rows of two real signals (modes
-// 0..nz2 = N/3 - 1; PAIR false: Y is absent): the Hermitian-extended spectrum
-// of x + i y.  Slots that lie in the zero band nz2 < k < N - nz2 for every lane
-// load nothing, slots wholly on one side of it need no select.
-template <int N, bool PAIR, typename R>
-__device__ __forceinline__ void tload_spectral(typename CT<R>::c *v, int t, const R *X, unsigned ox, const R *Y,
-                                               unsigned oy) {
-  using C = typename CT<R>::c;
+// The first pass's inputs from the spectra of two real signals x, y (modes
+// 0..nz2 = N/3 - 1): the Hermitian-extended spectrum of x + i y, where get(k, x, y)
+// gives both signals' mode k (PAIR false: y is absent).  Slots that lie in the
+// zero band nz2 < k < N - nz2 for every lane load nothing, slots wholly on one
+// side of it need no select.
+template <int N, bool PAIR, typename C, class Get>
+__device__ __forceinline__ void tload_modes(C *v, int t, Get get) {
+  using R = decltype(v[0].x);
   constexpr int G = ZRow<N>::G, RD = ZRow<N>::rad(0), NB = N / RD, MB = (NB + G - 1) / G, nz2 = N / 3 - 1;
 #pragma unroll
   for (int m = 0; m < MB; ++m)
@@ -412,9 +412,8 @@ __device__ __forceinline__ void tload_spectral(typename CT<R>::c *v, int t, cons
         const bool use = own && (low || high);
         unsigned kk = low ? k : N - k;
         if (!(full && (hi <= nz2 || lo >= N - nz2))) kk = use ? kk : 0u;
-        const C x = tld<C>(X, ox + kk);
-        C y = mkc<C>(0.0, 0.0);
-        if (PAIR) y = tld<C>(Y, oy + kk);
+        C x, y = mkc<C>(0.0, 0.0);
+        get(kk, x, y);
         const R s = low ? R(-1) : R(1);
         z = PAIR ? mkc<C>(x.x + s * y.y, -s * x.y + y.x) : mkc<C>(x.x, -s * x.y);
         if (lo == 0) z = k == 0 ? mkc<C>(x.x, y.x) : z; // Im of mode 0 does not enter
@@ -422,6 +421,17 @@ __device__ __forceinline__ void tload_spectral(typename CT<R>::c *v, int t, cons
       }
       v[m * RD + r] = z;
     }
+}
+
+// the same from the signals' spectral rows
+template <int N, bool PAIR, typename R>
+__device__ __forceinline__ void tload_spectral(typename CT<R>::c *v, int t, const R *X, unsigned ox, const R *Y,
+                                               unsigned oy) {
+  using C = typename CT<R>::c;
+  tload_modes<N, PAIR, C>(v, t, [&](unsigned k, C &x, C &y) {
+    x = tld<C>(X, ox + k);
+    if (PAIR) y = tld<C>(Y, oy + k);
+  });
 }
 
 // After the last inverse pass (outputs j + q N / R in order): the spectra of

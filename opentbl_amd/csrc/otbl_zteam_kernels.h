@@ -4,6 +4,7 @@
 // single wavefronts pack a CU's LDS and registers tightest.
 #pragma once
 #include "otbl_kcommon.h"
+#include "otbl_stats_row.h"
 #include "otbl_zteam.h"
 
 namespace otbl {
@@ -187,6 +188,120 @@ fourxz_t(double *fou, double *phys, int iopt, const double2 *__restrict__ tw, in
   }
 }
 
+// sum over a team, in its lane 0
+template <int G> __device__ __forceinline__ double team_sum(double v, int t) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    if (o < G) {
+      const double w = __shfl_down(v, o, 64);
+      v = t + o < G ? v + w : v;
+    }
+  return v;
+}
+
+// Row sums of the statistics (stotf.F90:148-283) for one (j, i) row, as
+// stats_zr: three packed c2r transforms in the fields' precision, the physical
+// products and every sum in FP64.
+template <int N, typename R>
+__global__ void __launch_bounds__(64)
+stats_t(StatsZ a, const typename CT<R>::c *__restrict__ tw, int nx, int ny, int nrows) {
+  using C = typename CT<R>::c;
+  using Z = ZRow<N>;
+  using F = ZRowPhys<N>;
+  constexpr int nz1 = 2 * (N / 3), nz2 = N / 3 - 1;
+  __shared__ C lds_all[Z::T * Z::lds()];
+  TeamRow<N> w;
+  if (!w.init(nrows)) return;
+  const int t = w.t, row = w.row;
+  C *lds = lds_all + w.team * Z::lds();
+  const int i = row / ny, j = row - i * ny; // 0-based plane and row
+  const size_t ov = (size_t)w.row0 * nz1;
+  const unsigned o = (unsigned)w.team * (nz1 / 2);
+  const R *Bq[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) Bq[q] = (const R *)a.B[q] + ov;
+  const R *V = (const R *)a.v + ov, *DV = (const R *)a.dvdx + ov;
+  const size_t om = (size_t)j * nx + i; // (i, j) of the [ny][nx] mean-flow rows
+  // mode 0 of B1 (u_x at the v rows) with the FP64 mean flow of a mixed box
+  const R m1 = a.m1 ? (R)a.m1[om] : R(0);
+  auto b1at = [&](unsigned k) {
+    C b = tld<C>(Bq[0], o + k);
+    if (a.m1 && k == 0) b.x = m1;
+    return b;
+  };
+  double sum[NSUM];
+#pragma unroll
+  for (int q = 0; q < NSUM; ++q) sum[q] = 0.0;
+  R s2[F::E], U[F::E];
+  C v[Z::E];
+  // omega_x + i omega_y
+  tload_modes<N, true, C>(v, t, [&](unsigned k, C &x, C &y) {
+    const R kz = (R)a.kaz[k];
+    const C b7 = tld<C>(Bq[6], o + k), vv = tld<C>(V, o + k), b1 = b1at(k), b3 = tld<C>(Bq[2], o + k);
+    x = mkc<C>(b7.x + kz * vv.y, b7.y - kz * vv.x);
+    y = mkc<C>(-kz * b1.y - b3.x, kz * b1.x - b3.y);
+  });
+  trun<N, +1, false>(v, t, tw, lds);
+#pragma unroll
+  for (int e = 0; e < F::E; ++e) s2[e] = v[e].x * v[e].x + v[e].y * v[e].y;
+  // omega_z + i u
+  tload_modes<N, true, C>(v, t, [&](unsigned k, C &x, C &y) {
+    const C dv = tld<C>(DV, o + k), b6 = tld<C>(Bq[5], o + k);
+    x = mkc<C>(dv.x - b6.x, dv.y - b6.y);
+    y = b1at(k);
+  });
+  trun<N, +1, false>(v, t, tw, lds);
+  float *ens = a.ens + (size_t)row * N;
+#pragma unroll
+  for (int m = 0; m < F::MB; ++m) {
+    const bool own = town<F::NB, Z::G>(t, m);
+#pragma unroll
+    for (int q = 0; q < F::R; ++q) {
+      const int e = m * F::R + q;
+      if (own) ens[t + Z::G * m + q * F::NB] = (float)sqrt((double)s2[e] + (double)v[e].x * (double)v[e].x);
+      U[e] = v[e].y;
+    }
+  }
+  // v + i w (a lane without a butterfly holds zeros: nothing in the sums)
+  tload_modes<N, true, C>(v, t, [&](unsigned k, C &x, C &y) {
+    x = tld<C>(V, o + k);
+    y = tld<C>(Bq[1], o + k);
+  });
+  trun<N, +1, false>(v, t, tw, lds);
+#pragma unroll
+  for (int e = 0; e < F::E; ++e) {
+    const double u = U[e], vv = v[e].x, ww = v[e].y;
+    sum[21] += u * u * u;    // u3
+    sum[22] += u * ww * ww;  // w2u
+    sum[23] += vv * vv * vv; // v3
+    sum[24] += vv * ww * ww; // w2v
+    sum[25] += u * vv * vv;  // v2u
+    sum[26] += vv * u * u;   // u2v
+  }
+  auto wd = [](C x) { return make_double2((double)x.x, (double)x.y); };
+#pragma unroll 1
+  for (int k = t; k <= nz2; k += Z::G) {
+    double2 b1 = wd(tld<C>(Bq[0], o + k)), b4 = wd(tld<C>(Bq[3], o + k)), b6 = wd(tld<C>(Bq[5], o + k));
+    if (a.m1 && k == 0) {
+      b1.x = a.m1[om];
+      b4.x = a.m4[om];
+      b6.x = a.m6[om];
+    }
+    stats_mode(sum, k == 0 ? 1.0 : 2.0, a.kaz[k], b1, wd(tld<C>(Bq[1], o + k)), wd(tld<C>(Bq[2], o + k)), b4,
+               wd(tld<C>(Bq[4], o + k)), b6, wd(tld<C>(Bq[6], o + k)), wd(tld<C>(Bq[7], o + k)),
+               wd(tld<C>(V, o + k)), wd(tld<C>(DV, o + k)));
+  }
+#pragma unroll
+  for (int q = 0; q < NSUM; ++q) sum[q] = team_sum<Z::G>(sum[q], t);
+  if (t != 0) return;
+  const size_t S = (size_t)nx * (ny + 1);
+  double *acc = a.acc + (size_t)i * (ny + 1) + j;
+  stats_add_sums(acc, S, sum);
+  auto re0 = [&](const R *p) { return (double)tld<C>(p, o).x; };
+  stats_add_means(acc, S, a.m1 ? a.m1[om] : re0(Bq[0]), re0(Bq[1]), re0(Bq[2]), a.m1 ? a.m4[om] : re0(Bq[3]),
+                  re0(Bq[4]), a.m1 ? a.m6[om] : re0(Bq[5]), re0(Bq[6]), re0(Bq[7]), re0(V), re0(DV));
+}
+
 template <int N> static void team_fns(ZTeamFns &f) {
   f.nz = N;
   f.lanes = ZRow<N>::G;
@@ -196,6 +311,8 @@ template <int N> static void team_fns(ZTeamFns &f) {
   f.p2d = &products2_t<N, double>;
   f.p2f = &products2_t<N, float>;
   f.fx = &fourxz_t<N>;
+  f.std_ = &stats_t<N, double>;
+  f.stf = &stats_t<N, float>;
 }
 
 // the kernels of length n if it is one of LO, LO + 2, .. HI

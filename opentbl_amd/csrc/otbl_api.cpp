@@ -525,9 +525,10 @@ static void setup_mixed(Box &b) {
   dalloc(b.ytab_f, YT_COUNT * ytab_size(b.yL));
   k_d2f(b, b.ytab, b.ytab_f, YT_COUNT * ytab_size(b.yL));
   // the half-wave rk_final addresses a field by 32-bit byte offsets: fields
-  // of 2^30 FP32 values or more take the full-wave kernel
+  // of 2^30 FP32 values or more take the full-wave kernel, as do rows so short
+  // that a workgroup meets more mean-flow columns than its LDS rows
   const char *yh = std::getenv("OTBL_Y_HALF");
-  if (b.yL % 2 == 0 && !(yh && yh[0] == '0') && b.nu < (size_t(1) << 30)) {
+  if (b.yL % 2 == 0 && !(yh && yh[0] == '0') && b.nu < (size_t(1) << 30) && b.nz1 >= YH_NZ1) {
     dalloc(b.ytabh_f, YT_COUNT * ytabh_size(b.yL / 2));
     k_ytab_halve_fixed(b);
   }

@@ -71,6 +71,9 @@ struct DevScalars {
   double ener[16];
 };
 
+// shortest row (nz1) of the half-wave y chunks
+static constexpr int YH_NZ1 = 8;
+
 struct StatsZ; // arguments of the statistics' z kernels (otbl_stats_row.h)
 
 // The z kernels with several rows per wavefront (otbl_zteam.h) of one row
@@ -190,7 +193,7 @@ struct Box {
   // plane run of the element-wise predictor / projection kernels (0: the
   // default for the element size)
   int prun = 0;
-  // the FP32 rk_final on half-wave chunks when its tables exist
+  // the FP32 rk_final on half-wave chunks when its tables exist (nz1 >= YH_NZ1)
   bool yhalf = true;
   // rhs_loop2, boun and rk_final fused per component (ky_rk_tail) where the
   // y solves run on full-wave chunks (Box::tail()); OTBL_Y_NOTAIL at create

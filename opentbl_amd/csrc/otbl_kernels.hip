@@ -14,6 +14,7 @@
 // Stockham, radices 8/4/2/3/5/7), two real signals per complex transform.
 #include "otbl_kcommon.h"
 #include "otbl_fft.h"
+#include "otbl_predict.h"
 #include "otbl_ycol.h"
 
 #include <algorithm>
@@ -1173,143 +1174,63 @@ __global__ void rhsu_loop1_kernel(const double *__restrict__ uv, const double *_
 }
 
 // Save the velocities (rhsp.F90:281-285) and apply the pressure-gradient
-// predictor (rhsp.F90:291-339) in one pass over u-type elements.  The
-// velocities u, v, w are left in place as the saved copy; the predicted
-// velocities (or the copies, outside the predictor's rows and planes) are
-// written to un, vn, wn, and the caller swaps the roles of the two sets.
-// With FP32 fields: p0, the FP64 mean-flow pressure [nx][ny], whose
-// gradients replace those of p's mode-0 real part; um, the FP64 mean-flow u
-// [ny+1][nx] (mode-0 real part), updated in FP64 and saved to rm (else
-// all null).
-template <typename T>
-__device__ __forceinline__ void save_predict_col(const T *__restrict__ u, const T *__restrict__ v,
-                                                 const T *__restrict__ w, const T *__restrict__ p,
-                                                 T *__restrict__ un, T *__restrict__ vn, T *__restrict__ wn,
-                                                 const T *idyy, const T *kaz, const DevScalars *ds, double idxx_d,
-                                                 int nx, int ny, int nz1, const double *__restrict__ p0,
-                                                 const double *idyy_d, double *um, double *rm, int pm, int kr,
-                                                 int j) {
+// predictor (rhsp.F90:291-339) in one pass over u-type elements, for y lines
+// too long for the chunked solver (whose final update forms the predicted
+// velocity itself, otbl_predict.h).  The velocities u, v, w are left in place
+// as the saved copy; the predicted velocities (or the copies, outside the
+// predictor's rows and planes) are written to un, vn, wn, and the caller swaps
+// the roles of the two sets.
+__global__ void save_predict_kernel(const double *__restrict__ u, const double *__restrict__ v,
+                                    const double *__restrict__ w, const double *__restrict__ p,
+                                    double *__restrict__ un, double *__restrict__ vn, double *__restrict__ wn,
+                                    const double *idyy, const double *kaz, const DevScalars *ds, double idxx, int nx,
+                                    int ny, int nz1, int pm) {
+  int kr, j;
+  if (!pcol(nz1, ny + 1, kr, j)) return;
   const int i0 = (int)blockIdx.y * pm + 1, i1 = min(nx, i0 + pm - 1);
   const size_t pu = (size_t)nz1 * (ny + 1), pv = (size_t)nz1 * ny;
-  const T var1 = (T)ds->var1, idxx = (T)idxx_d;
-  const bool mean = p0 && kr == 0, vrow = j <= ny;
+  const double var1 = ds->var1;
+  const bool vrow = j <= ny;
   size_t e = (size_t)(i0 - 1) * pu + (size_t)(j - 1) * nz1 + kr;
   size_t ev = (size_t)(i0 - 1) * pv + (size_t)(j - 1) * nz1 + kr;
-  T pc = vrow ? p[ev] : T(0); // p(i, j), carried from plane to plane
+  double pc = vrow ? p[ev] : 0.0; // p(i, j), carried from plane to plane
   for (int i = i0; i <= i1; ++i, e += pu, ev += pv) {
-    const T pn = (vrow && i < nx) ? p[ev + pv] : T(0); // p(i+1, j)
-    const T uu = u[e], ww = w[e];
-    const double *pm = mean ? p0 + (size_t)(i - 1) * ny + (j - 1) : nullptr; // mean pressure at (i, j)
-    const bool upred = i >= 2 && i <= nx - 1 && j >= 2 && j <= ny;
-    T uo = uu;
-    if (um && kr == 0) {
-      const size_t q = (size_t)(j - 1) * nx + (i - 1);
-      double U = um[q];
-      rm[q] = U;
-      if (upred) {
-        U -= ds->var1 * idxx_d * (pm[ny] - pm[0]);
-        um[q] = U;
-        uo = (T)U;
-      }
-    } else if (upred) {
-      if (mean)
-        uo = (T)((double)uu - ds->var1 * idxx_d * (pm[ny] - pm[0]));
-      else
-        uo = uu - var1 * idxx * (pn - pc);
-    }
-    un[e] = uo;
-    T wo = ww;
+    const double pn = (vrow && i < nx) ? p[ev + pv] : 0.0; // p(i+1, j)
+    const double uu = u[e], ww = w[e];
+    un[e] = i >= 2 && i <= nx - 1 && j >= 2 && j <= ny ? uu - var1 * idxx * (pn - pc) : uu;
+    double wo = ww;
     if (i >= 2 && j >= 2 && j <= ny) {
       // w -= var1 * (i kz p): Re gets -(-kz Im p), Im gets -(kz Re p)
-      T kz = kaz[kr / 2];
-      T pp = p[ev ^ 1];
-      T t = (kr & 1) ? (kz * pp) : (-kz * pp);
+      const double kz = kaz[kr / 2], pp = p[ev ^ 1];
+      const double t = (kr & 1) ? (kz * pp) : (-kz * pp);
       wo = ww - var1 * t;
     }
     wn[e] = wo;
     if (vrow) {
-      const T vv = v[ev];
-      T vo = vv;
-      if (i >= 2 && j >= 2 && j <= ny - 1) {
-        if (mean)
-          vo = (T)((double)vv - ds->var1 * idyy_d[j] * (pm[1] - pm[0]));
-        else
-          vo = vv - var1 * idyy[j] * (p[ev + nz1] - pc);
-      }
-      vn[ev] = vo;
+      const double vv = v[ev];
+      vn[ev] = i >= 2 && j >= 2 && j <= ny - 1 ? vv - var1 * idyy[j] * (p[ev + nz1] - pc) : vv;
     }
     pc = pn;
   }
 }
 
-template <typename T>
-__global__ void save_predict_kernel(const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-                                    const T *__restrict__ p, T *__restrict__ un, T *__restrict__ vn,
-                                    T *__restrict__ wn, const T *idyy, const T *kaz, const DevScalars *ds,
-                                    double idxx_d, int nx, int ny, int nz1, const double *__restrict__ p0,
-                                    const double *idyy_d, double *um, double *rm, int pm) {
-  int kr, j;
-  if (!pcol(nz1, ny + 1, kr, j)) return;
-  save_predict_col(u, v, w, p, un, vn, wn, idyy, kaz, ds, idxx_d, nx, ny, nz1, p0, idyy_d, um, rm, pm, kr, j);
-}
-
-// The FP32 save and predictor with one thread per mode (Re, Im as float2,
-// as project_pair_kernel); mode 0 (its Re part carries the FP64 mean flow)
-// runs save_predict_col per part.
-__global__ void save_predict_pair_kernel(const float *__restrict__ u, const float *__restrict__ v,
-                                         const float *__restrict__ w, const float *__restrict__ p,
-                                         float *__restrict__ un, float *__restrict__ vn, float *__restrict__ wn,
-                                         const float *idyy, const float *kaz, const DevScalars *ds, double idxx_d,
-                                         int nx, int ny, int nz1, const double *__restrict__ p0,
-                                         const double *idyy_d, double *um, double *rm, int pm) {
-  int kp, j;
-  if (!pcol(nz1 / 2, ny + 1, kp, j)) return;
-  if (kp == 0) {
-    for (int kr = 0; kr < 2; ++kr)
-      save_predict_col(u, v, w, p, un, vn, wn, idyy, kaz, ds, idxx_d, nx, ny, nz1, p0, idyy_d, um, rm, pm, kr, j);
-    return;
-  }
-  const int i0 = (int)blockIdx.y * pm + 1, i1 = min(nx, i0 + pm - 1);
-  const size_t pu2 = (size_t)nz1 * (ny + 1) / 2, pv2 = (size_t)nz1 * ny / 2, s2 = (size_t)nz1 / 2;
-  const float var1 = (float)ds->var1, idxx = (float)idxx_d;
-  const bool vrow = j <= ny;
-  const float kz = kaz[kp];
-  const float2 *u2 = reinterpret_cast<const float2 *>(u), *v2 = reinterpret_cast<const float2 *>(v);
-  const float2 *w2 = reinterpret_cast<const float2 *>(w), *p2 = reinterpret_cast<const float2 *>(p);
-  float2 *un2 = reinterpret_cast<float2 *>(un), *vn2 = reinterpret_cast<float2 *>(vn);
-  float2 *wn2 = reinterpret_cast<float2 *>(wn);
-  size_t e = (size_t)(i0 - 1) * pu2 + (size_t)(j - 1) * s2 + kp;
-  size_t ev = (size_t)(i0 - 1) * pv2 + (size_t)(j - 1) * s2 + kp;
-  float2 pc = vrow ? p2[ev] : make_float2(0.0f, 0.0f); // p(i, j), carried from plane to plane
-  for (int i = i0; i <= i1; ++i, e += pu2, ev += pv2) {
-    const float2 pn = (vrow && i < nx) ? p2[ev + pv2] : make_float2(0.0f, 0.0f); // p(i+1, j)
-    const float2 uu = u2[e], ww = w2[e];
-    float2 uo = uu;
-    if (i >= 2 && i <= nx - 1 && j >= 2 && j <= ny) {
-      uo.x = uu.x - var1 * idxx * (pn.x - pc.x);
-      uo.y = uu.y - var1 * idxx * (pn.y - pc.y);
-    }
-    un2[e] = uo;
-    float2 wo = ww;
-    if (i >= 2 && j >= 2 && j <= ny) {
-      // w -= var1 * (i kz p): Re gets -(-kz Im p), Im gets -(kz Re p)
-      const float tx = -kz * pc.y, ty = kz * pc.x;
-      wo.x = ww.x - var1 * tx;
-      wo.y = ww.y - var1 * ty;
-    }
-    wn2[e] = wo;
-    if (vrow) {
-      const float2 vv = v2[ev];
-      float2 vo = vv;
-      if (i >= 2 && j >= 2 && j <= ny - 1) {
-        const float2 pj = p2[ev + s2]; // p(i, j+1)
-        vo.x = vv.x - var1 * idyy[j] * (pj.x - pc.x);
-        vo.y = vv.y - var1 * idyy[j] * (pj.y - pc.y);
-      }
-      vn2[ev] = vo;
-    }
-    pc = pn;
-  }
+// The same for the mean flow of the mixed substep, by its FP64 pressure p0
+// [nx][ny]: the FP64 u um [ny+1][nx] is saved to rm and predicted in place; the
+// real part of v's mode 0 goes from the saved field v to the new one, vn.
+__global__ void mean_predict_kernel(double *um, double *__restrict__ rm, const double *__restrict__ p0,
+                                    const float *__restrict__ v, float *__restrict__ vn, const double *idyy,
+                                    const DevScalars *ds, double idxx, int nx, int ny, int nz1) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nx * (ny + 1)) return;
+  const int i = e % nx + 1, j = e / nx + 1;
+  const double U = um[e];
+  rm[e] = U;
+  const double *pm = p0 + (size_t)(i - 1) * ny + (j - 1);
+  if (i >= 2 && i <= nx - 1 && j >= 2 && j <= ny) um[e] = U - ds->var1 * idxx * (pm[ny] - pm[0]);
+  if (j > ny) return;
+  const size_t ev = ((size_t)(i - 1) * ny + (j - 1)) * nz1;
+  const float vv = v[ev];
+  vn[ev] = i >= 2 && j >= 2 && j <= ny - 1 ? (float)((double)vv - ds->var1 * idyy[j] * (pm[1] - pm[0])) : vv;
 }
 
 // dt from the CFL limits (rhsp.F90:214-262, coeft.f90:432-454) and the RK3
@@ -1660,9 +1581,12 @@ __global__ void rhs_loop2_kernel(double *rhsu, double *rhsv, double *rhsw, const
 // (rhsp.F90:421-445) for every plane.  Columns (kr, i).
 // um: with FP32 fields, the FP64 mean-flow u [ny+1][nx], whose boundary
 // rows are extrapolated in FP64 from its own interior (else null).
-template <typename T>
+// PRED: the rows come from the saved velocities resu, resw and the pressure
+// gradient (planes past the inflow's), as the final update forms them.
+template <typename T, bool PRED>
 __global__ void boun_kernel(T *u, T *v, T *w, T *rhsu, T *rhsv, T *rhsw, DevCoefT<T> c, int ny, int nz1, int nx,
-                            double *um, DevCoef cd) {
+                            double *um, DevCoef cd, const T *__restrict__ resu, const T *__restrict__ resw,
+                            const DevScalars *__restrict__ ds, Predictor<T> P) {
   size_t cidx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (cidx >= (size_t)nz1 * nx) return;
   int kr = (int)(cidx % nz1);
@@ -1671,7 +1595,7 @@ __global__ void boun_kernel(T *u, T *v, T *w, T *rhsu, T *rhsv, T *rhsw, DevCoef
   T *vi = v + ip * pv + kr;
   vi[0] = T(0);
   vi[(size_t)(ny - 1) * s] = (kr == 0) ? c.vmagic[ip + 1] : T(0);
-  const T i21 = T(-1) / M4(c.inby, 2, 1), c11 = T(-1) / M2(c.ccon, 1, 1);
+  const T i21 = T(-1) / M4(c.inby, 2, 1);
   T *f[2] = {u + ip * pu + kr, w + ip * pu + kr};
   for (int q = 0; q < 2; ++q) {
     T *a = f[q];
@@ -1685,9 +1609,15 @@ __global__ void boun_kernel(T *u, T *v, T *w, T *rhsu, T *rhsv, T *rhsw, DevCoef
       a[(size_t)ny * s] = (T)UR(ny);
       continue;
     }
-    a[0] = i21 * (M4(c.inby, 2, 2) * a[s] + M4(c.inby, 2, 3) * a[2 * s] + M4(c.inby, 2, 4) * a[3 * s]);
-    a[(size_t)ny * s] = c11 * (M2(c.ccon, 1, 2) * a[(size_t)(ny - 1) * s] + M2(c.ccon, 1, 3) * a[(size_t)(ny - 2) * s] +
-                               M2(c.ccon, 1, 4) * a[(size_t)(ny - 3) * s]);
+    const T *sv = (q == 0 ? resu : resw) + ip * pu + kr;
+    const PredCol<2, T> pw(P, c, ds, kr, ip);
+    const PredCol<3, T> px(P, c, ds, kr, ip);
+    auto at = [&](int j) -> T {
+      if (PRED && ip > 0) return q == 0 ? px.pred(sv[(size_t)j * s], j) : pw.pred(sv[(size_t)j * s], j);
+      return a[(size_t)j * s];
+    };
+    a[0] = boun_first(c, at);
+    a[(size_t)ny * s] = boun_last(c, ny, at);
   }
   // rhs: plane 1 zero, v rows 1 and ny zero, u/w row 1 extrapolated, row ny+1 zero
   T *rvi = rhsv + ip * pv + kr;
@@ -2134,23 +2064,9 @@ __global__ void project_pair_kernel(float *u, float *v, float *w, float *p, cons
   }
 }
 
-// The save and pressure-gradient predictor launch (rhsp.F90:281-339): u, v,
-// w, p read, the predicted velocities written to un, vn, wn; in the mixed
-// substep the FP64 mean-flow u um is saved to rm and predicted in place.
-template <typename T>
-static void save_predict_launch(Box &b, const T *u, const T *v, const T *w, const T *p, T *un, T *vn, T *wn,
-                                double *um, double *rm, int pm) {
-  const DevCoefT<T> &c = coefs<T>(b);
-  constexpr bool F64 = sizeof(T) == 8;
-  if constexpr (!F64) {
-    const dim3 pg(nblk(b.pu / 2), (unsigned)((b.nx + pm - 1) / pm)); // one thread per mode (Re, Im)
-    LAUNCH(b, "save_predict", pg, TPB, 0, save_predict_pair_kernel, u, v, w, p, un, vn, wn, c.idyy, c.kaz, b.ds,
-           b.hc.idxx, b.nx, b.ny, b.nz1, (const double *)b.p0, b.dc.idyy, um, rm, pm);
-  } else {
-    LAUNCH(b, "save_predict", pgrid(b, pm), TPB, 0, save_predict_kernel<T>, u, v, w, p, un, vn, wn, c.idyy, c.kaz,
-           b.ds, b.hc.idxx, b.nx, b.ny, b.nz1, (const double *)nullptr, b.dc.idyy, (double *)nullptr,
-           (double *)nullptr, pm);
-  }
+static void save_predict_launch(Box &b, double *un, double *vn, double *wn, int pm) {
+  LAUNCH(b, "save_predict", pgrid(b, pm), TPB, 0, save_predict_kernel, b.f[OTBL_U], b.f[OTBL_V], b.f[OTBL_W],
+         b.f[OTBL_P], un, vn, wn, b.dc.idyy, b.dc.kaz, b.ds, b.hc.idxx, b.nx, b.ny, b.nz1, pm);
 }
 
 // The projection launch of pois (pois.f90:144-181): phi (planes layout,
@@ -2257,7 +2173,7 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   constexpr bool F64 = std::is_same<T, double>::value;
   const int nx = b.nx, ny = b.ny, nz1 = b.nz1;
   const int ru = ny + 1;
-  T *u = fld<T>(b.f[OTBL_U]), *v = fld<T>(b.f[OTBL_V]), *w = fld<T>(b.f[OTBL_W]), *p = fld<T>(b.f[OTBL_P]);
+  T *u = fld<T>(b.f[OTBL_U]), *v = fld<T>(b.f[OTBL_V]), *w = fld<T>(b.f[OTBL_W]);
   T *resu = fld<T>(b.resu), *resv = fld<T>(b.resv), *resw = fld<T>(b.resw);
   T *rhsu = fld<T>(b.rhsu), *rhsv = fld<T>(b.rhsv), *rhsw = fld<T>(b.rhsw);
   // the previous substep's rhs (read before the role swap below)
@@ -2332,11 +2248,17 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   // time step and RK constants
   LAUNCH(b, "dt", 1, 64, 0, dt_kernel, b.ds, b.vmbits, b.dc.dymin, ny, m, b.dt_mode == OTBL_DT_EVERY_STEP ? 1 : 0,
          b.hc.dxmin, b.hc.dtret, b.hc.rex, b.hc.rkc[m], b.hc.rkd[m], b.hc.rkcv[m], b.hc.rkdv[m]);
-  // save velocities, pressure-gradient predictor
+  // save velocities, pressure-gradient predictor: the chunked final update
+  // forms the predicted velocities from the saved ones itself, only the mean
+  // flow of the mixed substep is predicted here
   double *um = F64 ? nullptr : b.um64; // the FP64 mean-flow u of the mixed substep
-  save_predict_launch<T>(b, u, v, w, p, resu, resv, resw, um, b.rm64, prun<T>(b));
-  // the predicted velocities now live in the former save buffers, and this
-  // substep's rhs buffers become the rhs_prev fields
+  if (um)
+    LAUNCH(b, "save_predict", nblk((size_t)nx * (ny + 1)), TPB, 0, mean_predict_kernel, um, b.rm64,
+           (const double *)b.p0, (const float *)v, (float *)resv, b.dc.idyy, b.ds, b.hc.idxx, nx, ny, nz1);
+  if constexpr (F64)
+    if (!b.yL) save_predict_launch(b, resu, resv, resw, prun<T>(b));
+  // the save buffers take the new velocities, and this substep's rhs buffers
+  // become the rhs_prev fields
   k_swap_saved(b);
   std::swap(u, resu);
   std::swap(v, resv);
@@ -2401,19 +2323,20 @@ template <typename T> static void rhsp_t(Box &b, int m) {
     return;
   }
   // boundary conditions (rhsp.F90:421-445)
-  LAUNCH(b, "boun", nblk((size_t)nz1 * nx), TPB, 0, boun_kernel<T>, u, v, w, rhsu, rhsv, rhsw, c, ny, nz1, nx, um,
-         b.dc);
+  auto kb = b.yL ? &boun_kernel<T, true> : &boun_kernel<T, false>;
+  LAUNCH(b, "boun", nblk((size_t)nz1 * nx), TPB, 0, kb, u, v, w, rhsu, rhsv, rhsw, c, ny, nz1, nx, um, b.dc, resu,
+         resw, b.ds, predictor<T>(b));
   // implicit factors for this dt, then the final update per component
   launch_impl_factor(b, 0.0, 0);
   if (b.yL) {
-    ky_rk_final<T>(b, v, resv, rhsv, rp[1], ny);
+    ky_rk_final<T>(b, 1, v, resv, rhsv, rp[1]);
     if constexpr (!F64) // the FP64 mean-flow u (kz = 0 real part)
       ky_mean_rk_final<T>(b, um, b.rm64, rhsu, rp[0]);
-    ky_rk_final<T>(b, u, resu, rhsu, rp[0], ny + 1);
+    ky_rk_final<T>(b, 3, u, resu, rhsu, rp[0]);
     if (um)
       LAUNCH(b, "rk_mean", nblk((size_t)nx * (ny + 1)), TPB, 0, mean_to_field_kernel<T>, u, (const double *)um, nx,
              ny + 1, nz1);
-    ky_rk_final<T>(b, w, resw, rhsw, rp[2], ny + 1);
+    ky_rk_final<T>(b, 2, w, resw, rhsw, rp[2]);
   } else if constexpr (F64) {
     size_t ncol = (size_t)nz1 * nx;
     LAUNCH(b, "rk_final", nblk(ncol), TPB, 0, rk_final_kernel, v, resv, rhsv, rp[1], wki2, b.dc, b.implv, b.ds, ny,
@@ -2572,15 +2495,15 @@ template <typename T> static std::string autotune_t(Box &b, int reps) {
   {
     double *scr = nullptr;
     const size_t nm = (size_t)b.nx * (b.ny + 1);
-    OTBL_HIP(hipMalloc((void **)&scr, 3 * nm * sizeof(double)));
-    double *um = b.um64 ? scr : nullptr, *rm = b.um64 ? scr + nm : nullptr, *p0 = b.p0 ? scr + 2 * nm : nullptr;
-    T *u = fld<T>(b.f[OTBL_U]), *v = fld<T>(b.f[OTBL_V]), *w = fld<T>(b.f[OTBL_W]), *p = fld<T>(b.f[OTBL_P]);
+    OTBL_HIP(hipMalloc((void **)&scr, 2 * nm * sizeof(double)));
+    double *um = b.um64 ? scr : nullptr, *p0 = b.p0 ? scr + nm : nullptr;
     double best = 1e30;
     int pick = prun<T>(b);
     try {
       for (int pm : {1, 2, 4, 8}) {
         const double ms = time_launches(b, reps, [&] {
-          save_predict_launch<T>(b, u, v, w, p, fld<T>(b.resu), fld<T>(b.resv), fld<T>(b.resw), um, rm, pm);
+          if constexpr (sizeof(T) == 8)
+            if (!b.yL) save_predict_launch(b, b.resu, b.resv, b.resw, pm);
           project_launch(b, b.resu, b.resv, b.resw, b.rhsv, b.rest, b.phs, 0.0, false, p0, um, pm);
         });
         std::snprintf(buf, sizeof buf, "prun%d=%.4fms ", pm, ms);
@@ -2603,8 +2526,8 @@ template <typename T> static std::string autotune_t(Box &b, int reps) {
       for (bool half : {true, false}) {
         b.yhalf = half;
         const double ms = time_launches(b, reps, [&] {
-          ky_rk_final<T>(b, fld<T>(b.wki2), fld<T>(b.resv), fld<T>(b.rhsv), fld<T>(b.f[OTBL_RHSVPA]), b.ny);
-          ky_rk_final<T>(b, fld<T>(b.wki1), fld<T>(b.resu), fld<T>(b.rhsu), fld<T>(b.f[OTBL_RHSUPA]), b.ny + 1);
+          ky_rk_final<T>(b, 1, fld<T>(b.wki2), fld<T>(b.resv), fld<T>(b.rhsv), fld<T>(b.f[OTBL_RHSVPA]));
+          ky_rk_final<T>(b, 3, fld<T>(b.wki1), fld<T>(b.resu), fld<T>(b.rhsu), fld<T>(b.f[OTBL_RHSUPA]));
         });
         std::snprintf(buf, sizeof buf, "yhalf%d=%.4fms ", half ? 1 : 0, ms);
         rep += buf;

@@ -210,7 +210,7 @@ template <typename T> void ky_rhsu_loop1(Box &b, const T *uv, const T *uw, T *rh
 template <typename T>
 void ky_rhs_loop2(Box &b, T *rhsu, T *rhsv, T *rhsw, const T *resu, const T *resv, const T *resw, const T *vw,
                   const T *vv, const T *ww);
-template <typename T> void ky_rk_final(Box &b, T *u, const T *res, const T *rhs, const T *rhsp, int jee);
+template <typename T> void ky_rk_final(Box &b, int k, T *u, const T *res, const T *rhs, const T *rhsp);
 // plane loop 2's y terms, boun's rows and rk_final of one component in one
 // pass (k2 = 1 v, 2 w, 3 u); pa, pb: the loop's products (v: vw, vv; w: ww,
 // vw; u: none)

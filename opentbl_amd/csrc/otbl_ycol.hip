@@ -21,6 +21,7 @@
 // they are scalar loads into scalar registers (FP32 rk_final, which measured
 // faster that way, stages its two tables in LDS).
 #include "otbl_kcommon.h"
+#include "otbl_predict.h"
 #include "otbl_ycol.h"
 
 namespace otbl {
@@ -98,7 +99,7 @@ __device__ __forceinline__ int yclamp(int j, int n) { return j < 0 ? 0 : (j >= n
 
 // An opaque copy of a wave-uniform value: row offsets built from it in one
 // phase of a kernel are not shared with (and kept live from) another phase.
-__device__ __forceinline__ size_t yopaque(size_t x) {
+template <typename I> __device__ __forceinline__ I yopaque(I x) {
   asm volatile("" : "+s"(x));
   return x;
 }
@@ -128,21 +129,23 @@ template <typename T>
 __device__ __forceinline__ T bnd4(const T *cf, int ld, int row, const T *col, size_t s, int j1, int dir) {
   T r = 0;
 #pragma unroll
-  for (int k = 1; k <= 4; ++k) r += cf[ld * (k - 1) + row - 1] * col[(size_t)(j1 + dir * (k - 1) - 1) * s];
+  for (int k = 1; k <= 4; ++k) r = fma(cf[ld * (k - 1) + row - 1], col[(size_t)(j1 + dir * (k - 1) - 1) * s], r);
   return r;
 }
 
 // Right-hand side of one chunk fused with the forward local sweep.  fetch(k)
 // returns input row j0-1+k (k = 0..L+1, 0-based rows, j0 = p*L); interior
 // rows take the table's 3-point stencil, the system's first row takes `bot`
-// and its last row (n-1) `top`; add1 and addm are added to rows 1 and n-2
-// (the boundary columns of implzy).  Rows past n have a zero stencil.
+// and its last row (n-1) `top`; with ADD, c1 bot and cm top are added to rows 1
+// and n-2 (the boundary columns of implzy).  Rows past n have a zero stencil.
 // Returns y at the chunk's last row (its forward carry-out).
 // G: rows per fenced group (a group's input loads are issued together);
 // the FP32 interpolation and rhsu kernels gain from whole-chunk groups, the
 // kernels with more live state lose.
-template <int L, int G = YGRP, int NCH = YNCH, typename T, class Fetch>
-__device__ __forceinline__ T yfwd(T (&v)[L], Fetch fetch, const T *tab, int p, int n, T bot, T top, T add1, T addm) {
+// The sums are written as explicit multiply-adds: kernels that share the sweep
+// are compared bit for bit, and the compiler's own choice varies with them.
+template <int L, int G = YGRP, int NCH = YNCH, bool ADD = false, typename T, class Fetch>
+__device__ __forceinline__ T yfwd(T (&v)[L], Fetch fetch, const T *tab, int p, int n, T bot, T top, T c1 = 0, T cm = 0) {
   constexpr int NL = NCH * L;
   const T *M = tab + p * L, *E1 = tab + 5 * NL + p * L, *E2 = tab + 6 * NL + p * L, *E3 = tab + 7 * NL + p * L;
   const int j0 = p * L;
@@ -152,12 +155,14 @@ __device__ __forceinline__ T yfwd(T (&v)[L], Fetch fetch, const T *tab, int p, i
     if (r % G == 0) YFENCE();
     const int j = j0 + r;
     const T gp = fetch(r + 2);
-    T x = E1[r] * gm + E2[r] * g0 + E3[r] * gp;
+    T x = fma(E3[r], gp, fma(E1[r], gm, E2[r] * g0));
     x = j == 0 ? bot : x;
     x = j == n - 1 ? top : x;
-    x = j == 1 ? x + add1 : x;
-    x = j == n - 2 ? x + addm : x;
-    y = x + M[r] * y;
+    if constexpr (ADD) {
+      x = j == 1 ? fma(c1, bot, x) : x;
+      x = j == n - 2 ? fma(cm, top, x) : x;
+    }
+    y = fma(M[r], y, x);
     v[r] = y;
     gm = g0;
     g0 = gp;
@@ -179,7 +184,7 @@ __device__ __forceinline__ void ybwd(T (&v)[L], T yend, const T *tab, int p, int
 #pragma unroll
   for (int r = L - 2; r >= 0; --r) {
     if (r % YGRP == 0) YFENCE();
-    v[r] = A2[r] * v[r] + B[r] * v[r + 1];
+    v[r] = fma(A2[r], v[r], B[r] * v[r + 1]);
   }
   YFENCE();
   __syncthreads(); // earlier readers of xch are done
@@ -200,7 +205,7 @@ __device__ __forceinline__ void ybwd(T (&v)[L], T yend, const T *tab, int p, int
 #pragma unroll
   for (int r = 0; r < L; ++r) {
     if (r % YGRP == 0) YFENCE();
-    v[r] = v[r] + C * G[r] + D * S[r];
+    v[r] = fma(D, S[r], fma(C, G[r], v[r]));
   }
   YFENCE();
 }
@@ -211,7 +216,7 @@ __device__ __forceinline__ void ysolve_col(T (&v)[L], const T *col, size_t s, in
                                            int n, T bot, T top, T *xch) {
   const int j0 = p * L;
   const T yend = yfwd<L, G, NCH>(
-      v, [&](int k) { return col[(size_t)yclamp(j0 - 1 + k, nin) * s]; }, tab, p, n, bot, top, T(0), T(0));
+      v, [&](int k) { return col[(size_t)yclamp(j0 - 1 + k, nin) * s]; }, tab, p, n, bot, top);
   ybwd<L, NCH, CW>(v, yend, tab, p, lane, xch);
 }
 
@@ -336,9 +341,8 @@ implzy_y(T *u, const T *__restrict__ res, const T *__restrict__ tab, const doubl
   __syncthreads();
   T w[L];
   const T *rc = res + off;
-  const T yend = yfwd<L>(
-      w, [&](int k) { return rc[(size_t)yclamp(j0 - 1 + k, jee) * s]; }, tl, q.p, jee, u1, uj, -a1b * u1,
-      -a3b * uj);
+  const T yend = yfwd<L, YGRP, YNCH, true>(
+      w, [&](int k) { return rc[(size_t)yclamp(j0 - 1 + k, jee) * s]; }, tl, q.p, jee, u1, uj, -a1b, -a3b);
   ybwd<L>(w, yend, tl, q.p, q.lane, xch);
 #pragma unroll
   for (int r = 0; r < L; ++r) {
@@ -480,15 +484,52 @@ rhs_loop2_y(T *rhsu, T *rhsv, T *rhsw, const T *__restrict__ resu,
   }
 }
 
+// The predicted row j of a component from its saved value x; the boundary rows
+// are boun's (b0 row 1, bn row jee)
+template <int K, typename T, typename I>
+__device__ __forceinline__ T pred_row(const PredCol<K, T, I> &pc, T x, int j, int jee, T b0, T bn) {
+  x = pc.pred(x, j);
+  x = j == 0 ? b0 : x;
+  return j == jee - 1 ? bn : x;
+}
+
+// The same for the L rows of a chunk of an FP32 column (col: the saved
+// velocity, un: the new one), every load issued before any use
+template <int L, int K, typename T>
+__device__ __forceinline__ void pred_rows(T (&w)[L], const Predictor<T> &P, const DevCoefT<T> &c, const DevScalars *ds,
+                                          const T *col, const T *un, int kr, size_t ip, size_t s, int jee, int j0,
+                                          T b0, T bn) {
+  const PredCol<K, T> pc(P, c, ds, kr, ip);
+  T a[L + 1], e[K == 3 ? L : 1];
+  if (K == 1 && pc.mean) col = un; // the mean lane of v
+#pragma unroll
+  for (int r = 0; r < L; ++r) w[r] = col[(size_t)yclamp(j0 + r, jee) * s];
+#pragma unroll
+  for (int r = 0; r < L + (K == 1); ++r) a[r] = pc.at(j0 + r);
+  if constexpr (K == 3)
+#pragma unroll
+    for (int r = 0; r < L; ++r) e[r] = pc.after(j0 + r);
+#pragma unroll
+  for (int r = 0; r < L; ++r) {
+    const int j = j0 + r;
+    w[r] = pc.apply(w[r], j, a[r], K == 3 ? e[K == 3 ? r : 0] : a[r + (K == 1)], pc.dyi(j));
+    w[r] = j == 0 ? b0 : w[r];
+    w[r] = j == jee - 1 ? bn : w[r];
+  }
+}
+
 // Explicit RK3 combination with vistyy (rhsp.F90:448-475) and the implicit
-// y-viscous solve (rhsp.F90:479-484) for one component, planes 2..nx
-// (plane nx: no viscous term).  The reference then copies rhs into rhs_prev
-// (rhsp.F90:475); here the buffers swap roles instead (k_swap_saved).
-template <int L, typename T>
+// y-viscous solve (rhsp.F90:479-484) for one component (K: 1 v, 2 w, 3 u),
+// planes 2..nx (plane nx: no viscous term), from the velocity that the
+// pressure gradient predicts out of the saved one, res; u holds boun's rows.
+// The reference then copies rhs into rhs_prev (rhsp.F90:475); here the buffers
+// swap roles instead (k_swap_saved).
+template <int L, typename T, int K>
 __global__ void __launch_bounds__(YTPB)
 rk_final_y(T *u, const T *__restrict__ res, const T *__restrict__ rhs, const T *__restrict__ rhsp,
            const T *__restrict__ tabv, const T *__restrict__ tabi, DevCoefT<T> c,
-           const double *__restrict__ f, const DevScalars *__restrict__ ds, int jee, int ny, int nz1, int nx) {
+           const double *__restrict__ f, const DevScalars *__restrict__ ds, Predictor<T> P, int jee, int ny, int nz1,
+           int nx) {
   __shared__ T xch[2 * YNCH * 64];
   __shared__ T hal[2 * YNCH * 64];
   // FP64: the tables are read in place (wave-uniform indices: scalar loads,
@@ -519,35 +560,36 @@ rk_final_y(T *u, const T *__restrict__ res, const T *__restrict__ rhs, const T *
     // live through the vistyy solve
     T w[L];
     {
-      T rh[L], rp[L], uu[L];
+      pred_rows<L, K>(w, P, c, ds, res + off, u + off, q.kr, q.ip, yopaque(s), jee, j0, u1, uj);
+      T rh[L], rp[L];
       const size_t s1 = yopaque(s);
 #pragma unroll
       for (int r = 0; r < L; ++r) {
         const size_t o = off + (size_t)yclamp(j0 + r, jee) * s1;
         rh[r] = rhs[o];
         rp[r] = rhsp[o];
-        uu[r] = u[o];
       }
 #pragma unroll
-      for (int r = 0; r < L; ++r) w[r] = uu[r] - (var3 * rh[r] + var4 * rp[r]);
+      for (int r = 0; r < L; ++r) w[r] = w[r] - fma(var3, rh[r], var4 * rp[r]);
     }
     YFENCE();
     __syncthreads();
     ysolve_col<L>(t, res + off, s, jee, tlv, q.p, q.lane, jee, bd.bot, bd.top, xch);
 #pragma unroll
     for (int r = 0; r < L; ++r)
-      if (act && j0 + r < jee) t[r] = w[r] - var2 * t[r];
+      if (act && j0 + r < jee) t[r] = fma(-var2, t[r], w[r]);
   } else {
     __syncthreads();
     ysolve_col<L>(t, res + off, s, jee, tlv, q.p, q.lane, jee, bd.bot, bd.top, xch);
     const size_t s1 = yopaque(s);
+    const PredCol<K, T> pc(P, c, ds, q.kr, q.ip);
 #pragma unroll
     for (int r = 0; r < L; ++r) {
       if (r % YGRP == 0) YFENCE();
       const int j = j0 + r;
       const size_t o = off + (size_t)yclamp(j, jee) * s1;
-      const T rh = rhs[o], rp = rhsp[o], uu = u[o];
-      if (act && j < jee) t[r] = uu - (var3 * rh + var2 * t[r] + var4 * rp);
+      const T rh = rhs[o], rp = rhsp[o], uu = pred_row(pc, res[o], j, jee, u1, uj);
+      if (act && j < jee) t[r] = rk_sum(uu, var3, rh, var2, t[r], var4, rp);
     }
   }
   YFENCE();
@@ -558,9 +600,8 @@ rk_final_y(T *u, const T *__restrict__ res, const T *__restrict__ rhs, const T *
   const T tm = q.p > 0 ? hal[(YNCH + q.p - 1) * 64 + q.lane] : T(0);
   const T tp = q.p < YNCH - 1 ? hal[(q.p + 1) * 64 + q.lane] : T(0);
   // implzy on t, in place (row r is overwritten after rows r+1 is read)
-  const T yend = yfwd<L>(
-      t, [&](int k) { return k == 0 ? tm : (k == L + 1 ? tp : t[k - 1]); }, tli, q.p, jee, u1, uj, -a1b * u1,
-      -a3b * uj);
+  const T yend = yfwd<L, YGRP, YNCH, true>(
+      t, [&](int k) { return k == 0 ? tm : (k == L + 1 ? tp : t[k - 1]); }, tli, q.p, jee, u1, uj, -a1b, -a3b);
   ybwd<L>(t, yend, tli, q.p, q.lane, xch);
   const size_t s2 = yopaque(s);
 #pragma unroll
@@ -582,9 +623,11 @@ rk_final_y(T *u, const T *__restrict__ res, const T *__restrict__ rhs, const T *
 // checks that every field stays below 2^30 values).  The one-solve FP32
 // kernels (interpyy, rhsu_loop1) measured slower in this layout, and
 // rhs_loop2's live state does not fit 64 VGPRs: they keep the full-wave
-// chunks.
+// chunks.  HBM-bound: 5 passes over the field, 1.42 to 1.66 ms per component
+// at 1536 x 315 x 1024 (3.9 to 4.6 TB/s).
 // ---------------------------------------------------------------------------
 static constexpr int YHC = 32;
+static constexpr int YHMEAN = YHC / YH_NZ1; // mean-flow columns of a workgroup at most
 
 struct YColH {
   int p, lane;
@@ -611,16 +654,22 @@ __device__ __forceinline__ float &yref(float *base, unsigned e) {
   return *reinterpret_cast<float *>(reinterpret_cast<char *>(base) + (size_t)(e * 4u));
 }
 
+// a wave-uniform value that was computed in the vector unit, into a scalar register
+__device__ __forceinline__ float yuniform(float x) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+}
+
 template <int L> __device__ __forceinline__ void ytabh_stage(float *dst, const float *__restrict__ src) {
   for (int k = threadIdx.x; k < (int)ytabh_size(L); k += YTPB) dst[k] = src[k];
 }
 
 // rk_final (rhsp.F90:448-484), as rk_final_y
-template <int L>
+template <int L, int K>
 __global__ void __launch_bounds__(YTPB, 8)
 rk_final_yh(float *u, const float *__restrict__ res, const float *__restrict__ rhs, const float *__restrict__ rhsp,
             const float *__restrict__ tabv, const float *__restrict__ tabi, DevCoefT<float> c,
-            const double *__restrict__ f, const DevScalars *__restrict__ ds, int jee, int ny, int nz1, int nx) {
+            const double *__restrict__ f, const DevScalars *__restrict__ ds, Predictor<float> P, int jee, int ny,
+            int nz1, int nx) {
   using T = float;
   __shared__ T xch[2 * YHCH * YHC];
   __shared__ T hal[2 * YHCH * YHC];
@@ -631,26 +680,68 @@ rk_final_yh(float *u, const float *__restrict__ res, const float *__restrict__ r
   const unsigned s = nz1, off = q.ip * s * (unsigned)jee + q.kr;
   const bool act = q.ok && q.ip > 0;
   const int p = q.p, lane = q.lane, j0 = p * L;
+  // v's mean lanes (the real part of mode 0) take the rows predicted in the new
+  // field, through LDS: loading them in the sweep below costs 10 to 30 spilled
+  // registers.  A lane reads back what it wrote.
+  __shared__ T vmean[K == 1 ? YHMEAN * YHCH * L : 1];
+  const int mrow = K == 1 ? (lane / nz1 * YHCH + p) * L : 0;
+  if (K == 1 && act && q.kr == 0) {
+    const unsigned s1 = yopaque(s);
+#pragma unroll
+    for (int r = 0; r < L; ++r) vmean[mrow + r] = yat(u, off + (unsigned)yclamp(j0 + r, jee) * s1);
+  }
+  // a chunk meets the first rows of its column or the last ones, never both
+  // (32 chunks, jee >= L + 2): one register for either end's closure, and for
+  // either end's boundary row
   const YBnd<T> bd = vistyy_bnd(jee, j0, L, ny, c.cofvby, res + off, (size_t)s);
-  const T u1 = yat(u, off), uj = yat(u, off + (unsigned)(jee - 1) * s);
-  const T a1b = (T)f[3 * (jee + 1)], a3b = (T)f[3 * (jee + 1) + 1];
+  const T vb = p == 0 ? bd.bot : bd.top;
+  const T ub = yat(u, p == 0 ? off : off + (unsigned)(jee - 1) * s);
+  const T a1b = yuniform((T)f[3 * (jee + 1)]), a3b = yuniform((T)f[3 * (jee + 1) + 1]);
   const T var2 = (q.ip == (unsigned)(nx - 1)) ? T(0) : (T)ds->var2;
-  const T var3 = (T)ds->var3, var4 = (T)ds->var4;
+  const T var3 = yuniform((T)ds->var3), var4 = yuniform((T)ds->var4);
   T t[L], w[L];
   {
-    // the explicit part w = u - (var3 rhs + var4 rhs_prev), its 3L rows
-    // issued at once
-    T rh[L], rp[L], uu[L];
+    // the predicted velocity, then the explicit part w = u - (var3 rhs + var4
+    // rhs_prev): the loads of each issued at once
+    PredCol<K, T, unsigned> pc(P, c, ds, (int)q.kr, q.ip);
+    pc.var1 = yuniform(pc.var1);
+    if constexpr (K == 3) pc.f = yuniform(pc.f);
+#pragma unroll
+    for (int r = 0; r < L; ++r) w[r] = yat(res, off + (unsigned)yclamp(j0 + r, jee) * s);
+    T a[L + 1], e[K == 3 ? L : 1];
+#pragma unroll
+    for (int r = 0; r < L + (K == 1); ++r) a[r] = pc.at(j0 + r);
+    if constexpr (K == 3)
+#pragma unroll
+      for (int r = 0; r < L; ++r) e[r] = pc.after(j0 + r);
 #pragma unroll
     for (int r = 0; r < L; ++r) {
-      const unsigned o = off + (unsigned)yclamp(j0 + r, jee) * s;
+      const int j = j0 + r;
+      const T x = pc.apply(w[r], j, a[r], K == 3 ? e[K == 3 ? r : 0] : a[r + (K == 1)], pc.dyi(j));
+      w[r] = j == 0 || j == jee - 1 ? ub : x;
+    }
+    if (K == 1 || L > 10) YFENCE(); // these spill with both phases' loads in flight
+    if constexpr (K == 1) {
+#pragma unroll
+      for (int r = 0; r < L; ++r) {
+        if (r % YGRP == 0) YFENCE();
+        T m = vmean[mrow + r];
+        asm volatile("" : "+v"(m)); // read by every lane: a branch here spills, too
+        w[r] = pc.mean ? m : w[r];
+      }
+      YFENCE();
+    }
+    T rh[L], rp[L];
+    const unsigned s1 = yopaque(s);
+#pragma unroll
+    for (int r = 0; r < L; ++r) {
+      const unsigned o = off + (unsigned)yclamp(j0 + r, jee) * s1;
       rh[r] = yat(rhs, o);
       rp[r] = yat(rhsp, o);
-      uu[r] = yat(u, o);
     }
 #pragma unroll
     for (int r = 0; r < L; ++r) {
-      w[r] = uu[r] - (var3 * rh[r] + var4 * rp[r]);
+      w[r] = w[r] - fma(var3, rh[r], var4 * rp[r]);
       asm volatile("" : "+v"(w[r])); // formed here, not sunk to its use after the solve
     }
   }
@@ -658,13 +749,12 @@ rk_final_yh(float *u, const float *__restrict__ res, const float *__restrict__ r
   __syncthreads(); // tables staged
   {
     const T yend = yfwd<L, YGRP, YHCH>(
-        t, [&](int k) { return yat(res, off + (unsigned)yclamp(j0 - 1 + k, jee) * s); }, tlv, p, jee, bd.bot,
-        bd.top, T(0), T(0));
+        t, [&](int k) { return yat(res, off + (unsigned)yclamp(j0 - 1 + k, jee) * s); }, tlv, p, jee, vb, vb);
     ybwd<L, YHCH, YHC>(t, yend, tlv, p, lane, xch);
   }
 #pragma unroll
   for (int r = 0; r < L; ++r)
-    if (act && j0 + r < jee) t[r] = w[r] - var2 * t[r];
+    if (act && j0 + r < jee) t[r] = fma(-var2, t[r], w[r]);
   YFENCE();
   // neighbour rows of the combined right-hand side
   hal[p * YHC + lane] = t[0];
@@ -673,9 +763,8 @@ rk_final_yh(float *u, const float *__restrict__ res, const float *__restrict__ r
   const T tm = p > 0 ? hal[(YHCH + p - 1) * YHC + lane] : T(0);
   const T tp = p < YHCH - 1 ? hal[(p + 1) * YHC + lane] : T(0);
   // implzy on t, in place
-  const T yend = yfwd<L, YGRP, YHCH>(
-      t, [&](int k) { return k == 0 ? tm : (k == L + 1 ? tp : t[k - 1]); }, tli, p, jee, u1, uj, -a1b * u1,
-      -a3b * uj);
+  const T yend = yfwd<L, YGRP, YHCH, true>(
+      t, [&](int k) { return k == 0 ? tm : (k == L + 1 ? tp : t[k - 1]); }, tli, p, jee, ub, ub, -a1b, -a3b);
   ybwd<L, YHCH, YHC>(t, yend, tli, p, lane, xch);
 #pragma unroll
   for (int r = 0; r < L; ++r) {
@@ -706,14 +795,6 @@ rk_final_yh(float *u, const float *__restrict__ res, const float *__restrict__ r
 // boun_kernel and rk_final_y, in the same order: the same results bit for bit.
 // ---------------------------------------------------------------------------
 
-// u / w field rows 1 and ny+1 of boun from the column's interior rows
-template <typename T, class At>
-__device__ __forceinline__ void tail_field_bnd(const DevCoefT<T> &c, int ny, At at, T &b0, T &bn) {
-  const T i21 = T(-1) / M4(c.inby, 2, 1), c11 = T(-1) / M2(c.ccon, 1, 1);
-  b0 = i21 * (M4(c.inby, 2, 2) * at(1) + M4(c.inby, 2, 3) * at(2) + M4(c.inby, 2, 4) * at(3));
-  bn = c11 * (M2(c.ccon, 1, 2) * at(ny - 1) + M2(c.ccon, 1, 3) * at(ny - 2) + M2(c.ccon, 1, 4) * at(ny - 3));
-}
-
 // The fused tail runs on the full-wave chunks (FP64, and FP32 fields of 2^30
 // values or more).  Each rhs row is written as soon as it is formed, with
 // rows 2..4 also to LDS for row 1, and the RK update reads it back from cache.
@@ -726,7 +807,8 @@ __global__ void __launch_bounds__(YTPB)
 rk_tail_y(T *u, T *rhs, const T *__restrict__ res, const T *__restrict__ rhsp, const T *__restrict__ pa,
           const T *__restrict__ pb, const T *__restrict__ tabv, const T *__restrict__ tabi,
           const T *__restrict__ tabd, DevCoefT<T> c, const double *__restrict__ f,
-          const DevScalars *__restrict__ ds, const double *__restrict__ um, int jee, int ny, int nz1, int nx) {
+          const DevScalars *__restrict__ ds, const double *__restrict__ um, Predictor<T> P, int jee, int ny, int nz1,
+          int nx) {
   constexpr bool SOLVE = K2 != 3;
   __shared__ T xch[2 * YNCH * 64];
   __shared__ T hal[2 * YNCH * 64];
@@ -812,20 +894,28 @@ rk_tail_y(T *u, T *rhs, const T *__restrict__ res, const T *__restrict__ rhsp, c
     }
   }
   YFENCE();
-  T u1, uj;
-  if constexpr (K2 == 1) {
-    u1 = T(0);
-    uj = q.kr == 0 ? c.vmagic[q.ip + 1] : T(0);
-  } else if (K2 == 3 && um && q.kr == 0) {
-    u1 = (T)um[q.ip];
-    uj = (T)um[(size_t)ny * nx + q.ip];
-  } else {
-    tail_field_bnd(c, ny, [&](int j) { return u[off + (size_t)j * s]; }, u1, uj);
+  // boun's boundary rows, by the waves that hold them: from the predicted rows
+  // (plane 1: the inflow's)
+  T u1 = T(0), uj = T(0);
+  {
+    const PredCol<K2, T> pc(P, c, ds, q.kr, q.ip);
+    auto at = [&](int j) {
+      const size_t o = off + (size_t)j * s;
+      return q.ip == 0 ? u[o] : pc.pred(res[o], j);
+    };
+    const bool mean = K2 == 3 && um && q.kr == 0;
+    if (j0 == 0) {
+      if (K2 != 1) u1 = mean ? (T)um[q.ip] : boun_first(c, at);
+      if (q.ok) u[off] = u1;
+    }
+    if (jee - 1 >= j0 && jee - 2 < j0 + L) { // the implicit system takes it on row jee - 1, too
+      if (K2 == 1)
+        uj = q.kr == 0 ? c.vmagic[q.ip + 1] : T(0);
+      else
+        uj = mean ? (T)um[(size_t)ny * nx + q.ip] : boun_last(c, ny, at);
+      if (q.ok && jee - 1 < j0 + L) u[off + (size_t)(jee - 1) * s] = uj;
+    }
   }
-  // boun's boundary rows into the field now, by the lanes that hold them:
-  // the RK update below reads them back
-  if (q.ok && j0 == 0) u[off] = u1;
-  if (q.ok && jee - 1 >= j0 && jee - 1 < j0 + L) u[off + (size_t)(jee - 1) * s] = uj;
   YFENCE();
   const T a1b = (T)f[3 * (jee + 1)], a3b = (T)f[3 * (jee + 1) + 1];
   const T var2 = (q.ip == (size_t)(nx - 1)) ? T(0) : (T)ds->var2;
@@ -835,34 +925,35 @@ rk_tail_y(T *u, T *rhs, const T *__restrict__ res, const T *__restrict__ rhsp, c
   if constexpr (sizeof(T) == 4) {
     T w[L];
     {
-      T rh[L], rp[L], uu[L];
+      pred_rows<L, K2>(w, P, c, ds, res + off, u + off, q.kr, q.ip, yopaque(s), jee, j0, u1, uj);
+      T rh[L], rp[L];
       const size_t s1 = yopaque(s);
 #pragma unroll
       for (int r = 0; r < L; ++r) {
         const size_t o = off + (size_t)yclamp(j0 + r, jee) * s1;
         rh[r] = rhs[o];
         rp[r] = rhsp[o];
-        uu[r] = u[o];
       }
 #pragma unroll
-      for (int r = 0; r < L; ++r) w[r] = uu[r] - (var3 * rh[r] + var4 * rp[r]);
+      for (int r = 0; r < L; ++r) w[r] = w[r] - fma(var3, rh[r], var4 * rp[r]);
     }
     YFENCE();
     ysolve_col<L>(t, res + off, s, jee, tlv, q.p, q.lane, jee, bd.bot, bd.top, xch);
 #pragma unroll
     for (int r = 0; r < L; ++r)
-      if (act && j0 + r < jee) t[r] = w[r] - var2 * t[r];
+      if (act && j0 + r < jee) t[r] = fma(-var2, t[r], w[r]);
   } else {
     YFENCE();
     ysolve_col<L>(t, res + off, s, jee, tlv, q.p, q.lane, jee, bd.bot, bd.top, xch);
     const size_t s1 = yopaque(s);
+    const PredCol<K2, T> pc(P, c, ds, q.kr, q.ip);
 #pragma unroll
     for (int r = 0; r < L; ++r) {
       if (r % YGRP == 0) YFENCE();
       const int j = j0 + r;
       const size_t o = off + (size_t)yclamp(j, jee) * s1;
-      const T rr = rhs[o], rp = rhsp[o], uu = u[o];
-      if (act && j < jee) t[r] = uu - (var3 * rr + var2 * t[r] + var4 * rp);
+      const T rr = rhs[o], rp = rhsp[o], uu = pred_row(pc, res[o], j, jee, u1, uj);
+      if (act && j < jee) t[r] = rk_sum(uu, var3, rr, var2, t[r], var4, rp);
     }
   }
   YFENCE();
@@ -871,9 +962,8 @@ rk_tail_y(T *u, T *rhs, const T *__restrict__ res, const T *__restrict__ rhsp, c
   __syncthreads();
   const T tm = q.p > 0 ? hal[(YNCH + q.p - 1) * 64 + q.lane] : T(0);
   const T tp = q.p < YNCH - 1 ? hal[(q.p + 1) * 64 + q.lane] : T(0);
-  const T yend = yfwd<L>(
-      t, [&](int k) { return k == 0 ? tm : (k == L + 1 ? tp : t[k - 1]); }, tli, q.p, jee, u1, uj, -a1b * u1,
-      -a3b * uj);
+  const T yend = yfwd<L, YGRP, YNCH, true>(
+      t, [&](int k) { return k == 0 ? tm : (k == L + 1 ? tp : t[k - 1]); }, tli, q.p, jee, u1, uj, -a1b, -a3b);
   ybwd<L>(t, yend, tli, q.p, q.lane, xch);
   const size_t s2 = yopaque(s);
 #pragma unroll
@@ -938,9 +1028,8 @@ mean_rk_final_y(double *um, const double *__restrict__ rm, const T *__restrict__
   __syncthreads();
   const double tm = q.p > 0 ? hal[(YNCH + q.p - 1) * 64 + q.lane] : 0.0;
   const double tp = q.p < YNCH - 1 ? hal[(q.p + 1) * 64 + q.lane] : 0.0;
-  const double yend = yfwd<L>(
-      t, [&](int k) { return k == 0 ? tm : (k == L + 1 ? tp : t[k - 1]); }, tli, q.p, jee, u1, uj, -a1b * u1,
-      -a3b * uj);
+  const double yend = yfwd<L, YGRP, YNCH, true>(
+      t, [&](int k) { return k == 0 ? tm : (k == L + 1 ? tp : t[k - 1]); }, tli, q.p, jee, u1, uj, -a1b, -a3b);
   ybwd<L>(t, yend, tli, q.p, q.lane, xch);
 #pragma unroll
   for (int r = 0; r < L; ++r) {
@@ -1024,23 +1113,25 @@ void ky_rhs_loop2(Box &b, T *rhsu, T *rhsv, T *rhsw, const T *resu, const T *res
                    ytab<T>(b, YT_DCYU), ytab<T>(b, YT_DCYV), coefs<T>(b), b.ny, b.nz1, b.nx - 2));
 }
 
-template <typename T> void ky_rk_final(Box &b, T *u, const T *res, const T *rhs, const T *rhsp, int jee) {
+// component k (1 v, 2 w, 3 u)
+template <typename T> void ky_rk_final(Box &b, int k, T *u, const T *res, const T *rhs, const T *rhsp) {
   const unsigned g = ygrid((size_t)b.nz1 * b.nx);
-  const bool uu = jee == b.ny + 1;
+  const int jee = k == 1 ? b.ny : b.ny + 1;
+  const int kv = k == 1 ? YT_VIYV : YT_VIYU, ki = k == 1 ? YT_IMPV : YT_IMPU;
+  const double *f = k == 1 ? b.implv : b.implu;
+  const Predictor<T> P = predictor<T>(b);
   if constexpr (sizeof(T) == 4) {
     if (b.ytabh_f && b.yhalf) {
       yh_check((size_t)b.nz1 * b.nx * (b.ny + 1));
-      YDISPATCH(b.yL, auto kf = &rk_final_yh<L / 2>;
-                LAUNCH(b, "rk_final", ygridh((size_t)b.nz1 * b.nx), YTPB, 0, kf, u, res, rhs, rhsp,
-                       ytabh(b, uu ? YT_VIYU : YT_VIYV), ytabh(b, uu ? YT_IMPU : YT_IMPV), coefs<T>(b),
-                       uu ? b.implu : b.implv, b.ds, jee, b.ny, b.nz1, b.nx));
+      YDISPATCH(b.yL, auto kf = k == 1 ? &rk_final_yh<L / 2, 1> : (k == 2 ? &rk_final_yh<L / 2, 2> : &rk_final_yh<L / 2, 3>);
+                LAUNCH(b, "rk_final", ygridh((size_t)b.nz1 * b.nx), YTPB, 0, kf, u, res, rhs, rhsp, ytabh(b, kv),
+                       ytabh(b, ki), coefs<T>(b), f, b.ds, P, jee, b.ny, b.nz1, b.nx));
       return;
     }
   }
-  YDISPATCH(b.yL, auto kf = &rk_final_y<L, T>;
-            LAUNCH(b, "rk_final", g, YTPB, 0, kf, u, res, rhs, rhsp, ytab<T>(b, uu ? YT_VIYU : YT_VIYV),
-                   ytab<T>(b, uu ? YT_IMPU : YT_IMPV), coefs<T>(b), uu ? b.implu : b.implv, b.ds, jee, b.ny, b.nz1,
-                   b.nx));
+  YDISPATCH(b.yL, auto kf = k == 1 ? &rk_final_y<L, T, 1> : (k == 2 ? &rk_final_y<L, T, 2> : &rk_final_y<L, T, 3>);
+            LAUNCH(b, "rk_final", g, YTPB, 0, kf, u, res, rhs, rhsp, ytab<T>(b, kv), ytab<T>(b, ki), coefs<T>(b), f,
+                   b.ds, P, jee, b.ny, b.nz1, b.nx));
 }
 
 // the fused tail of one component (k2 = 1 v, 2 w, 3 u) on the full-wave
@@ -1056,7 +1147,8 @@ void ky_rk_tail(Box &b, int k2, T *u, T *rhs, const T *res, const T *rhsp, const
   const unsigned g = ygrid((size_t)b.nz1 * b.nx);
   YDISPATCH(b.yL, auto kf = k2 == 1 ? &rk_tail_y<L, T, 1> : (k2 == 2 ? &rk_tail_y<L, T, 2> : &rk_tail_y<L, T, 3>);
             LAUNCH(b, "rk_tail", g, YTPB, 0, kf, u, rhs, res, rhsp, pa, pb, ytab<T>(b, kv), ytab<T>(b, ki),
-                   ytab<T>(b, kd), coefs<T>(b), uu ? b.implu : b.implv, b.ds, um, jee, b.ny, b.nz1, b.nx));
+                   ytab<T>(b, kd), coefs<T>(b), uu ? b.implu : b.implv, b.ds, um, predictor<T>(b), jee,
+                   b.ny, b.nz1, b.nx));
 }
 template void ky_rk_tail<double>(Box &, int, double *, double *, const double *, const double *, const double *,
                                  const double *);
@@ -1083,7 +1175,7 @@ template void ky_mean_rk_final<float>(Box &, double *, const double *, const flo
   template void ky_rhsu_loop1<T>(Box &, const T *, const T *, T *);                                            \
   template void ky_rhs_loop2<T>(Box &, T *, T *, T *, const T *, const T *, const T *, const T *, const T *,     \
                                 const T *);                                                                    \
-  template void ky_rk_final<T>(Box &, T *, const T *, const T *, const T *, int);
+  template void ky_rk_final<T>(Box &, int, T *, const T *, const T *, const T *);
 YINST(double)
 YINST(float)
 

@@ -15,7 +15,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libopentbl_amd.so")
-SOURCES = ["otbl_api.cpp", "otbl_coef.cpp", "otbl_kernels.hip", "otbl_ycol.hip", "otbl_zfft.hip", "otbl_xline.hip",
+SOURCES = ["otbl_api.cpp", "otbl_coef.cpp", "otbl_hostio.cpp", "otbl_kernels.hip", "otbl_ycol.hip", "otbl_zfft.hip", "otbl_xline.hip",
            "otbl_xchunk.hip", "otbl_poisson.hip", "otbl_stats.hip", "otbl_zteam_1.hip", "otbl_zteam_2.hip", "otbl_zteam_3.hip",
            "otbl_zteam_4.hip"]
 ARCH = os.environ.get("OTBL_ARCH", "gfx950")

@@ -7,6 +7,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <stdexcept>
+#include <memory>
 #include <mutex>
 #include <string>
 
@@ -404,6 +405,7 @@ static void free_box(Box *b) {
   if (b->s2) (void)hipStreamDestroy(b->s2);
   for (hipEvent_t e : {b->ev_fork, b->ev_p1, b->ev_join})
     if (e) (void)hipEventDestroy(e);
+  free_stage(*b);
   if (b->s) (void)hipStreamDestroy(b->s);
   delete b;
 }
@@ -527,6 +529,7 @@ static void setup_mixed(Box &b) {
   // the half-wave rk_final addresses a field by 32-bit byte offsets: fields
   // of 2^30 FP32 values or more take the full-wave kernel, as do rows so short
   // that a workgroup meets more mean-flow columns than its LDS rows
+  if (const char *e = std::getenv("OTBL_READ_MIN")) b.read_min = std::strtoull(e, nullptr, 10);
   const char *yh = std::getenv("OTBL_Y_HALF");
   if (b.yL % 2 == 0 && !(yh && yh[0] == '0') && b.nu < (size_t(1) << 30) && b.nz1 >= YH_NZ1) {
     dalloc(b.ytabh_f, YT_COUNT * ytabh_size(b.yL / 2));
@@ -801,17 +804,28 @@ int otbl_get_field(otbl_ctx *ctx, int id, double *host) {
   if (b.esz == 8) {
     d2h(b, host, b.f[id], n * sizeof(double));
   } else {
-    const size_t chunk = b.nu / 2;
-    for (size_t o = 0; o < n; o += chunk) {
-      const size_t m = std::min(chunk, n - o);
-      k_f2d(b, fld<float>(b.f[id]) + o, b.ya, m);
-      OTBL_HIP(hipStreamSynchronize(b.s));
-      d2h(b, host + o, b.ya, m * sizeof(double));
-    }
+    // mode 0's real part of p and u comes from their FP64 mean flow
+    HostMean mean;
+    std::unique_ptr<double[]> m;
     if (id == OTBL_P || id == OTBL_U) {
-      std::vector<double> m(n / b.nz1);
-      d2h(b, m.data(), id == OTBL_P ? b.p0 : b.um64, m.size() * sizeof(double));
-      for (size_t r = 0; r < m.size(); ++r) host[r * b.nz1] = m[mean_slot(b, id, r)];
+      mean.row = b.nz1;
+      mean.nx = b.nx;
+      mean.rows = id == OTBL_P ? b.ny : b.ny + 1;
+      mean.tr = id == OTBL_U;
+      m.reset(new double[mean.nx * mean.rows]);
+      d2h(b, m.get(), id == OTBL_P ? b.p0 : b.um64, mean.nx * mean.rows * sizeof(double));
+      mean.v = m.get();
+    }
+    if (!field_to_host(b, fld<float>(b.f[id]), host, n, mean)) {
+      const size_t chunk = b.nu / 2; // widened on the GPU, in a work field
+      for (size_t o = 0; o < n; o += chunk) {
+        const size_t c = std::min(chunk, n - o);
+        k_f2d(b, fld<float>(b.f[id]) + o, b.ya, c);
+        OTBL_HIP(hipStreamSynchronize(b.s));
+        d2h(b, host + o, b.ya, c * sizeof(double));
+      }
+      if (mean.v)
+        for (size_t r = 0; r < mean.nx * mean.rows; ++r) host[r * mean.row] = mean.at(r);
     }
   }
   API_END

@@ -5,6 +5,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -73,6 +74,9 @@ struct DevScalars {
 
 // shortest row (nz1) of the half-wave y chunks
 static constexpr int YH_NZ1 = 8;
+
+// slots of the host reads' staging
+static constexpr int STAGE_SLOTS = 4;
 
 struct StatsZ; // arguments of the statistics' z kernels (otbl_stats_row.h)
 
@@ -206,6 +210,12 @@ struct Box {
   // column) and the tables of its eight systems
   int yL = 0;
   double *ytab = nullptr;
+  // reads of a mixed box's fields of read_min values or more through page-locked
+  // staging (otbl_hostio.cpp), and the events of its slots' copies
+  size_t read_min = size_t(1) << 27;
+  float *stage = nullptr;
+  hipEvent_t stage_ev[STAGE_SLOTS] = {};
+  std::shared_ptr<void> readers; // its hold on the process's widening threads
   // genflu / inflow
   double *um = nullptr, *u0 = nullptr, *v0 = nullptr, *gwork = nullptr;
   DevScalars *ds = nullptr;
@@ -317,6 +327,20 @@ template <typename T, bool REF> void kp_poisson_y(Box &b, T *P);
 // element conversions between FP64 and FP32 buffers on b.s
 void k_d2f(Box &b, const double *a, float *o, size_t n);
 void k_f2d(Box &b, const float *a, double *o, size_t n);
+// The FP64 mean flow of a field read to the host: the value of mode 0's real
+// part in row r = plane * rows + j, each row values long; v [nx][rows], or
+// [rows][nx] (tr); v null: none.
+struct HostMean {
+  const double *v = nullptr;
+  size_t row = 0, rows = 0, nx = 0;
+  bool tr = false;
+  double at(size_t r) const { return v[tr ? (r % rows) * nx + r / rows : r]; }
+};
+// n FP32 values to the host as doubles (otbl_hostio.cpp); false, and nothing
+// done, where that does not pay, for want of page-locked memory, or while
+// another read of the process has the threads
+bool field_to_host(Box &b, const float *dev, double *host, size_t n, const HostMean &mean);
+void free_stage(Box &b);
 void k_setup_attrs(Box &b);
 size_t k_dct_shm_bytes(int M);
 // register-resident z transforms (otbl_zfft.hip), valid when Box::zfast

@@ -323,7 +323,14 @@ std::string k_autotune(Box &b, int reps);
 // partitioned Poisson y solves of the modes kz >= 1 on pencils
 // (otbl_poisson.hip); REF: one FP64-residual refinement step
 int kp_chunk_rows(int ny);
-template <typename T, bool REF> void kp_poisson_y(Box &b, T *P);
+// the mean-flow mode (kr = 0, 1) that rides in the launch: its FP64 pencils,
+// scratch of the same layout, rows per y and line stride
+struct PoisMean {
+  double *P, *S;
+  int nz1, ld;
+};
+template <typename T, bool REF> void kp_poisson_y(Box &b, T *P, PoisMean m);
+void k_poisson_mean(Box &b, PoisMean m); // a launch of its own
 // element conversions between FP64 and FP32 buffers on b.s
 void k_d2f(Box &b, const double *a, float *o, size_t n);
 void k_f2d(Box &b, const float *a, double *o, size_t n);

@@ -15,6 +15,7 @@
 #include "otbl_kcommon.h"
 #include "otbl_fft.h"
 #include "otbl_predict.h"
+#include "otbl_ypencil.h"
 #include "otbl_ycol.h"
 
 #include <algorithm>
@@ -472,16 +473,30 @@ void k_vistyy(Box &b, const double *u, double *res, int R, int nplanes) {
 // layout per set (n = jee): f[0..n] a1 factored, f[n+1..2n+1] a2 (inverse
 // diagonal), f[2n+2..3n+2] a3, f[3n+3] = a1(2) and f[3n+4] = a3(jee-1)
 // before they are zeroed.  Dynamic LDS: 3*(ny+2) + 4*YNCH*L doubles.
-__global__ void impl_factor_kernel(double *fu, double *fv, DevCoef c, int ny, const DevScalars *ds,
-                                   double rkk_explicit, int use_explicit, double *tu, double *tv, int L, float *tuf,
-                                   float *tvf, float *thu, float *thv) {
+struct ImplArgs {
+  double *fu, *fv;
+  DevCoef c;
+  int ny;
+  const DevScalars *ds;
+  double rkk_explicit;
+  int use_explicit;
+  double *tu, *tv;
+  int L;
+  float *tuf, *tvf, *thu, *thv;
+};
+
+__device__ __forceinline__ void impl_factor_block(const ImplArgs &g) {
+  double *fu = g.fu, *fv = g.fv, *tu = g.tu, *tv = g.tv;
+  float *tuf = g.tuf, *tvf = g.tvf, *thu = g.thu, *thv = g.thv;
+  const DevCoef &c = g.c;
+  const int ny = g.ny, L = g.L;
   extern __shared__ double shf[];
   const int jee = blockIdx.x == 0 ? ny + 1 : ny;
   const double *icon = blockIdx.x == 0 ? c.vyui : c.vyvi;
   const double *econ = blockIdx.x == 0 ? c.cofvyu : c.cofvyv;
   double *f = blockIdx.x == 0 ? fu : fv;
   double *tab = blockIdx.x == 0 ? tu : tv;
-  const double v1 = use_explicit ? rkk_explicit : ds->rkk;
+  const double v1 = g.use_explicit ? g.rkk_explicit : g.ds->rkk;
   double *a1 = shf, *a2 = shf + (ny + 2), *a3 = shf + 2 * (ny + 2);
   for (int j = threadIdx.x + 2; j <= jee - 1; j += blockDim.x) {
     a1[j] = C3(icon, 1, j) + v1 * C3(econ, 3, j);
@@ -530,16 +545,21 @@ __global__ void impl_factor_kernel(double *fu, double *fv, DevCoef c, int ny, co
   }
 }
 
-static void launch_impl_factor(Box &b, double rkk, int use_explicit) {
-  double *tu = b.yL ? b.ytab + YT_IMPU * ytab_size(b.yL) : nullptr;
-  double *tv = b.yL ? b.ytab + YT_IMPV * ytab_size(b.yL) : nullptr;
-  float *tuf = b.ytab_f ? b.ytab_f + YT_IMPU * ytab_size(b.yL) : nullptr;
-  float *tvf = b.ytab_f ? b.ytab_f + YT_IMPV * ytab_size(b.yL) : nullptr;
-  float *thu = b.ytabh_f ? b.ytabh_f + YT_IMPU * ytabh_size(b.yL / 2) : nullptr;
-  float *thv = b.ytabh_f ? b.ytabh_f + YT_IMPV * ytabh_size(b.yL / 2) : nullptr;
-  const size_t shm = (3 * (size_t)(b.ny + 2) + 4 * (size_t)YNCH * b.yL) * sizeof(double);
-  LAUNCH(b, "impl_factor", 2, TPB, shm, impl_factor_kernel, b.implu, b.implv, b.dc, b.ny, b.ds, rkk,
-         use_explicit, tu, tv, b.yL, tuf, tvf, thu, thv);
+__global__ void impl_factor_kernel(ImplArgs g) { impl_factor_block(g); }
+
+static ImplArgs impl_args(const Box &b, double rkk, int use_explicit) {
+  ImplArgs g{b.implu, b.implv, b.dc, b.ny, b.ds, rkk, use_explicit, nullptr, nullptr, b.yL, nullptr, nullptr, nullptr,
+             nullptr};
+  if (b.yL) g.tu = b.ytab + YT_IMPU * ytab_size(b.yL), g.tv = b.ytab + YT_IMPV * ytab_size(b.yL);
+  if (b.ytab_f) g.tuf = b.ytab_f + YT_IMPU * ytab_size(b.yL), g.tvf = b.ytab_f + YT_IMPV * ytab_size(b.yL);
+  if (b.ytabh_f) g.thu = b.ytabh_f + YT_IMPU * ytabh_size(b.yL / 2), g.thv = b.ytabh_f + YT_IMPV * ytabh_size(b.yL / 2);
+  return g;
+}
+static size_t impl_shm(const Box &b) {
+  return (3 * (size_t)(b.ny + 2) + 4 * (size_t)YNCH * b.yL) * sizeof(double);
+}
+static void launch_impl_factor(Box &b, double rkk) {
+  LAUNCH(b, "impl_factor", 2, TPB, impl_shm(b), impl_factor_kernel, impl_args(b, rkk, 1));
 }
 
 // implzy (lip.f90:528-597): interior rows 2..jee-1 of u from res; rows 1 and
@@ -584,7 +604,7 @@ __global__ void implzy_kernel(double *u, const double *res, DevCoef c, const dou
 }
 
 void k_implzy_op(Box &b, double *u, const double *res, int R, double rkk, int nplanes) {
-  launch_impl_factor(b, rkk, 1);
+  launch_impl_factor(b, rkk);
   if (b.yL) {
     ky_implzy(b, u, res, R, nplanes);
     return;
@@ -1275,9 +1295,18 @@ __global__ void dt_kernel(DevScalars *ds, const unsigned long long *vmbits, cons
 //    factor, the zero modes from u0 / v0, the profile remapping, the copy of
 //    row ntop-3 above ntop-2 and the 1/gamma1 scaling, evaluated per element.
 // ibuf: kl[2][ny+1], ntop[2]; dbuf: fsca[2][ny+1], ysca[ny+1], wlwa[ny+1].
+//
+// The implicit factors for this dt (impl_factor_block, blocks 0 and 1) ride in
+// the launch of the statistics (block 2): both are serial chains of one
+// workgroup, and neither reads what the other writes.  Apart the factors took 21
+// us a substep at 387 x 113 x 98 and 27 at 640 x 144 x 160; here they add 2.
 template <typename T>
 __global__ void genflu_stats_kernel(const T *resu, double *um, int *ibuf, double *dbuf, DevCoef c, DevScalars *ds,
-                                    int ny, int nz1, int xout, double re) {
+                                    int ny, int nz1, int xout, double re, ImplArgs g) {
+  if (blockIdx.x < 2) {
+    impl_factor_block(g);
+    return;
+  }
   const int s = nz1;
   const T *ux = resu + (size_t)(xout - 1) * s * (ny + 1);
   __shared__ double sh_dtc;
@@ -1871,72 +1900,11 @@ div_pencils_kernel(const T *__restrict__ u, const T *__restrict__ v, const T *__
   }
 }
 
-// per-mode y tridiagonal on pencils (pois.f90:102-117, soltriy
-// pois.f90:211-239): one thread per (kr, kx-mode x), line (j-1, kr) at
-// P + ((j-1) nz1 + kr) ld, so rows at stride nz1 ld.
+// per-mode y tridiagonal on pencils, a thread per column (otbl_ypencil.h)
 __global__ void __launch_bounds__(TPB)
 poisson_y_pencil_kernel(double *__restrict__ P, double *__restrict__ S, DevCoef c, int nx, int ny, int nz1,
                         int kr_end, int ld) {
-  constexpr int RB = 8; // rows whose loads are issued together
-  const int N = nx - 1;
-  size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)kr_end * N) return; // columns kr < kr_end
-  const int x = (int)(t % N), kr = (int)(t / N), i = x + 2;
-  const size_t rs = (size_t)nz1 * ld;
-  double *col = P + (size_t)kr * ld + x;
-  double *d2 = S + (size_t)kr * ld + x;
-  const int ny1 = ny - 1;
-  if (kr == 1) { // the zero mode is real (pois.f90:102)
-    for (int j = 0; j < ny1; ++j) col[(size_t)j * rs] = 0.0;
-    return;
-  }
-  const double kz2 = c.kaz2[kr / 2], km = c.kmod[i - 1];
-  const bool pin = (i == 2 && kr == 0); // its last row: phi = 0 with a doubled diagonal
-  double a2prev = C3(c.ayp, 2, 1) - kz2 - km;
-  double a3prev = C3(c.ayp, 3, 1);
-  double y = (pin && ny1 == 1) ? 0.0 : col[0];
-  if (pin && ny1 == 1) col[0] = 0.0;
-  // forward elimination as soltriy, rows 2..ny-1
-  auto fwd = [&](int j, double b) {
-    if (pin && j == ny1) b = 0.0;
-    const double d = 1.0 / a2prev;
-    d2[(size_t)(j - 2) * rs] = d;
-    const double a1 = -C3(c.ayp, 1, j) * d;
-    double a2 = (pin && j == ny1) ? 2.0 * C3(c.ayp, 2, j) : C3(c.ayp, 2, j) - kz2 - km;
-    a2 = a2 + a1 * a3prev;
-    y = b + a1 * y;
-    col[(size_t)(j - 1) * rs] = y;
-    a2prev = a2;
-    a3prev = C3(c.ayp, 3, j);
-  };
-  int j = 2;
-  for (; j + RB - 1 <= ny1; j += RB) {
-    double bv[RB];
-#pragma unroll
-    for (int q = 0; q < RB; ++q) bv[q] = col[(size_t)(j + q - 1) * rs];
-#pragma unroll
-    for (int q = 0; q < RB; ++q) fwd(j + q, bv[q]);
-  }
-  for (; j <= ny1; ++j) fwd(j, col[(size_t)(j - 1) * rs]);
-  double x_ = y * (1.0 / a2prev);
-  col[(size_t)(ny1 - 1) * rs] = x_;
-  // back substitution, rows ny-2..1
-  auto bwd = [&](int j, double yv, double d) {
-    x_ = (yv - C3(c.ayp, 3, j) * x_) * d;
-    col[(size_t)(j - 1) * rs] = x_;
-  };
-  j = ny1 - 1;
-  for (; j - RB + 1 >= 1; j -= RB) {
-    double yv[RB], dv[RB];
-#pragma unroll
-    for (int q = 0; q < RB; ++q) {
-      yv[q] = col[(size_t)(j - q - 1) * rs];
-      dv[q] = d2[(size_t)(j - q - 1) * rs];
-    }
-#pragma unroll
-    for (int q = 0; q < RB; ++q) bwd(j - q, yv[q], dv[q]);
-  }
-  for (; j >= 1; --j) bwd(j, col[(size_t)(j - 1) * rs], d2[(size_t)(j - 1) * rs]);
+  poisson_y_march((size_t)blockIdx.x * blockDim.x + threadIdx.x, P, S, c, nx, ny, nz1, kr_end, ld);
 }
 
 // projection (pois.f90:144-162): p, w, v, u from phi = rest
@@ -2087,6 +2055,11 @@ static void project_launch(Box &b, double *u, double *v, double *w, double *p, c
   }
 }
 
+void k_poisson_mean(Box &b, PoisMean m) {
+  LAUNCH(b, "poisson_y0", nblk(2 * (size_t)(b.nx - 1)), TPB, 0, poisson_y_pencil_kernel, m.P, m.S, b.dc, b.nx, b.ny,
+         m.nz1, 2, m.ld);
+}
+
 // FP32 pressure solve of the mixed path: the kz = 0 lines run in FP64 on
 // their own pencils (divergence, both x transforms and the pinned y solve),
 // the other modes in FP32 with one FP64-residual refinement of the y solve.
@@ -2098,8 +2071,7 @@ static void pois_mixed(Box &b, double varstep, bool use_m) {
          fld<float>(b.f[OTBL_W]), P, b.pld, b.dcf, b.hc.idx, nx, ny, nz1, b.P0, b.dc, (const double *)b.um64);
   kz_dct_pencils<float>(b, P, -1, Lp, b.pld);
   kz_dct_pencils<double>(b, b.P0, -1, 2 * (ny - 1), N);
-  kp_poisson_y<float, true>(b, P);
-  LAUNCH(b, "poisson_y0", nblk(2 * (size_t)N), TPB, 0, poisson_y_pencil_kernel, b.P0, b.S0, b.dc, nx, ny, 2, 2, N);
+  kp_poisson_y<float, true>(b, P, {b.P0, b.S0, 2, N});
   kz_dct_pencils<float>(b, P, 1, Lp, b.pld);
   kz_dct_pencils<double>(b, b.P0, 1, 2 * (ny - 1), N);
   LAUNCH(b, "to_planes", tgrid(b), DIV_TPB, 0, pencils_to_planes_kernel<float>, P, F, Lp, N, b.pld, b.phs, b.P0, nz1);
@@ -2120,11 +2092,9 @@ void k_pois(Box &b, int m, double varstep, bool use_m) {
            b.pld, b.dc, b.hc.idx, nx, ny, nz1, (double *)nullptr, b.dc, (const double *)nullptr);
     dct_pencils(b, b.rest2, -1);
     if (b.pchunk) {
-      // modes kz >= 1 partitioned in registers; the pinned mean-flow mode
+      // modes kz >= 1 partitioned in registers, the pinned mean-flow mode
       // (kr = 0, 1) marching, one thread per column
-      kp_poisson_y<double, false>(b, b.rest2);
-      LAUNCH(b, "poisson_y0", nblk(2 * (size_t)N), TPB, 0, poisson_y_pencil_kernel, b.rest2, b.rest, b.dc, nx, ny,
-             nz1, 2, b.pld);
+      kp_poisson_y<double, false>(b, b.rest2, {b.rest2, b.rest, nz1, b.pld});
     } else {
       LAUNCH(b, "poisson_y", nblk((size_t)nz1 * N), TPB, 0, poisson_y_pencil_kernel, b.rest2, b.rest, b.dc, nx, ny,
              nz1, nz1, b.pld);
@@ -2263,12 +2233,13 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   std::swap(u, resu);
   std::swap(v, resv);
   std::swap(w, resw);
-  // recycling inflow (rhsp.F90:287)
+  // recycling inflow (rhsp.F90:287), and the implicit factors for this dt
   {
     int *ibuf = (int *)(b.gwork + (size_t)nz1 * (ny + 1));
     double *dbuf = b.gwork + (size_t)nz1 * (ny + 1) + 4 * (ny + 2);
-    LAUNCH(b, "genflu", 1, TPB, 8 * (size_t)(ny + 2) * sizeof(double), genflu_stats_kernel<T>, resu, b.um, ibuf,
-           dbuf, b.dc, b.ds, ny, nz1, b.xout, b.re);
+    const size_t gshm = std::max(8 * (size_t)(ny + 2) * sizeof(double), impl_shm(b));
+    LAUNCH(b, "genflu", 3, TPB, gshm, genflu_stats_kernel<T>, resu, b.um, ibuf, dbuf, b.dc, b.ds, ny, nz1, b.xout,
+           b.re, impl_args(b, 0.0, 0));
     LAUNCH(b, "genflu", dim3(nblk((size_t)nz1 * (ny + 1)), 3), TPB, 0, genflu_plane_kernel<T>, u, v, w, resu, resv,
            resw, b.u0, b.v0, ibuf, dbuf, b.dc, b.ds, ny, nz1, b.xout, um, nx);
     if (b.diag)
@@ -2308,8 +2279,7 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   }
   if (tail) {
     // plane loop 2's y terms, boun's rows and the final update per component
-    // in one pass each; the implicit factors for this dt first
-    launch_impl_factor(b, 0.0, 0);
+    // in one pass each
     ky_rk_tail<T>(b, 1, v, rhsv, resv, rp[1], ya, yb);
     if (um) k_boun_mean(b);
     ky_rk_tail<T>(b, 3, u, rhsu, resu, rp[0], (const T *)nullptr, (const T *)nullptr);
@@ -2326,8 +2296,7 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   auto kb = b.yL ? &boun_kernel<T, true> : &boun_kernel<T, false>;
   LAUNCH(b, "boun", nblk((size_t)nz1 * nx), TPB, 0, kb, u, v, w, rhsu, rhsv, rhsw, c, ny, nz1, nx, um, b.dc, resu,
          resw, b.ds, predictor<T>(b));
-  // implicit factors for this dt, then the final update per component
-  launch_impl_factor(b, 0.0, 0);
+  // the final update per component
   if (b.yL) {
     ky_rk_final<T>(b, 1, v, resv, rhsv, rp[1]);
     if constexpr (!F64) // the FP64 mean-flow u (kz = 0 real part)

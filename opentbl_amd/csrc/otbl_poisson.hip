@@ -26,11 +26,21 @@
 // formed in FP64 (rows of the neighbouring chunks from the interface
 // values) and the FP32 solution of A d = r, through the same factors and
 // spikes, is added: one step of iterative refinement.
-#include "otbl_kcommon.h"
+//
+// The pinned mean-flow mode (kr = 0, 1), a column per thread marching in FP64,
+// rides in the same launch where chunks are short (PMEAN): its 2 N columns are a
+// serial chain of 13 to 60 us that fills a few CUs, taken by the first workgroups
+// (four wavefronts of each) while the rest solve the other modes.  us per
+// substep, two launches -> one: 256 x 96 x 64 FP64 17 + 29 -> 39, 387 x 113 x 98
+// mixed 30 + 31 -> 43, 640 x 144 x 160 mixed 75 + 42 -> 76, 896 x 176 x 224 FP64
+// 178 + 50 -> 180.  Longer chunks spill with the march beside them: 1536 x 315 x
+// 1024 mixed 1457 + 101 -> 1704, so they keep two launches.
+#include "otbl_ypencil.h"
 
 namespace otbl {
 
 static constexpr int PK = 32;     // chunks per column = columns per workgroup
+static constexpr int PMEAN = 8;   // longest chunk that takes the mean-flow mode along
 static constexpr int PROWS = 512; // rows the LDS coefficient copy holds (ny - 1 <= PROWS)
 
 // 1 / x: the FP32 solves (followed by a refinement step whose FP64
@@ -45,7 +55,14 @@ template <typename T> __device__ __forceinline__ T prcp(T x) {
 
 template <int L, typename T, bool REF>
 __global__ void __launch_bounds__(1024, sizeof(T) == 4 ? 8 : 1)
-poisson_y_chunk(T *__restrict__ P, DevCoefT<T> c, DevCoef cd, int nx, int ny, int nz1, int ld) {
+poisson_y_chunk(T *__restrict__ P, DevCoefT<T> c, DevCoef cd, int nx, int ny, int nz1, int ld, PoisMean pm,
+                unsigned mb) {
+  if constexpr (L <= PMEAN)
+    if (blockIdx.x < mb) { // the mean-flow mode: mb workgroups of TPB columns
+      if (threadIdx.x < TPB)
+        poisson_y_march((size_t)blockIdx.x * TPB + threadIdx.x, pm.P, pm.S, cd, nx, ny, pm.nz1, 2, pm.ld);
+      return;
+    }
   // interface system per chunk and lane column: yF, yL, VF, VL, WF, WL; then
   // the interface unknowns F, L
   __shared__ T red[PK][6][PK];
@@ -76,7 +93,7 @@ poisson_y_chunk(T *__restrict__ P, DevCoefT<T> c, DevCoef cd, int nx, int ny, in
   const int col = lane & (PK - 1), k = wave * 2 + (lane >> 5);
   // XCD-contiguous block order: neighbouring workgroups share the cache
   // lines at the ends of their 16-mode runs
-  const size_t t = (size_t)N + (size_t)xcd_block() * (PK / 2) + (col >> 1); // kz >= 1 only
+  const size_t t = (size_t)N + (size_t)xcd_remap(blockIdx.x - mb, gridDim.x - mb) * (PK / 2) + (col >> 1); // kz >= 1 only
   const bool live = t < (size_t)nzh * N;
   const int kz = live ? (int)(t / N) : 1, x = live ? (int)(t % N) : 0;
   // 32-bit byte offsets from a wave-uniform base (the wave's first row, a
@@ -319,19 +336,21 @@ int kp_chunk_rows(int ny) {
   return 0;
 }
 
-template <typename T, bool REF> void kp_poisson_y(Box &b, T *P) {
+template <typename T, bool REF> void kp_poisson_y(Box &b, T *P, PoisMean m) {
   const int N = b.nx - 1, nzh = b.nz1 / 2;
   const size_t cols = (size_t)(nzh - 1) * N;
-  if (cols == 0) return;
   // a wave addresses 2 L rows plus one row of offsets in 32 bits
   if ((size_t)(2 * kp_chunk_rows(b.ny) + 1) * b.nz1 * b.pld * sizeof(T) >= (size_t(1) << 32))
     throw std::invalid_argument("Poisson pencil rows too long for 32-bit offsets");
-  const unsigned grid = (unsigned)((cols + PK / 2 - 1) / (PK / 2)); // 16 modes (Re, Im) per workgroup
+  const unsigned mb = kp_chunk_rows(b.ny) <= PMEAN ? nblk(2 * (size_t)N) : 0;
+  if (mb == 0) k_poisson_mean(b, m);
+  const unsigned grid = mb + (unsigned)((cols + PK / 2 - 1) / (PK / 2)); // 16 modes (Re, Im) per workgroup
+  if (grid == 0) return;
   switch (kp_chunk_rows(b.ny)) {
 #define PCASE(LL)                                                                                          \
   case LL: {                                                                                               \
     auto kf = &poisson_y_chunk<LL, T, REF>;                                                                \
-    LAUNCH(b, "poisson_y", grid, 1024, 0, kf, P, coefs<T>(b), b.dc, b.nx, b.ny, b.nz1, b.pld);             \
+    LAUNCH(b, "poisson_y", grid, 1024, 0, kf, P, coefs<T>(b), b.dc, b.nx, b.ny, b.nz1, b.pld, m, mb);      \
   } break;
     PCASE(2)
     PCASE(4)
@@ -346,7 +365,7 @@ template <typename T, bool REF> void kp_poisson_y(Box &b, T *P) {
   }
 }
 
-template void kp_poisson_y<double, false>(Box &, double *);
-template void kp_poisson_y<float, true>(Box &, float *);
+template void kp_poisson_y<double, false>(Box &, double *, PoisMean);
+template void kp_poisson_y<float, true>(Box &, float *, PoisMean);
 
 } // namespace otbl

@@ -367,6 +367,10 @@ void kxc_tables(Box &b);
 template <typename T> void kxc_interpxx(Box &b, const T *gen, T *geni, int which_u, int chi, int chi2, size_t P);
 template <typename T>
 void kxc_difvisxx(Box &b, const T *prod, const T *vel, T *out, int which_u, int chv, int ic, size_t P, int mode);
+// the three of a substep (u, v, w) in one launch; false, and nothing done, where
+// the lines are not chunked
+template <typename T> bool kxc_interpxx3(Box &b, const T *const *gen, T *const *geni);
+template <typename T> bool kxc_difvisxx3(Box &b, const T *const *prod, const T *const *vel, T *const *out);
 // register-resident transforms (otbl_zfft.hip): the z products and fourxz valid
 // when Box::zfast or Box::zteam.nz, the Poisson x transforms when
 // Box::dct_zfast

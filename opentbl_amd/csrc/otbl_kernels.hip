@@ -2186,9 +2186,13 @@ template <typename T> static void rhsp_t(Box &b, int m) {
     });
   }
   // x interpolation (rhsp.F90:105-107)
-  x_interp<T>(b, u, wki1, ru, 1);
-  x_interp<T>(b, v, wki2, ny, 0);
-  x_interp<T>(b, w, wki3, ru, 0);
+  const T *vel3[3] = {u, v, w}, *wki3c[3] = {wki1, wki2, wki3};
+  T *wk3[3] = {wki1, wki2, wki3}, *rhs3[3] = {rhsu, rhsv, rhsw};
+  if (!kxc_interpxx3<T>(b, vel3, wk3)) {
+    x_interp<T>(b, u, wki1, ru, 1);
+    x_interp<T>(b, v, wki2, ny, 0);
+    x_interp<T>(b, w, wki3, ru, 0);
+  }
   if (m == 1)
     LAUNCH(b, "energies", 3, 1024, 0, energies_kernel<T>, u, v, w, b.dc.hy, b.ds, nx, ny, nz1, b.nz2);
   // u interpolated to v rows in spectral space (interpyy is linear along y and
@@ -2212,9 +2216,11 @@ template <typename T> static void rhsp_t(Box &b, int m) {
     LAUNCH(b, "rhsu_loop1", nblk((size_t)nz1 * nx), TPB, 0, rhsu_loop1_kernel, wki2, wki3, rhsu, b.dc, ny, nz1,
            nx);
   // x derivatives (rhsp.F90:181-204)
-  x_difvis<T>(b, wki1, u, rhsu, ru, 1, 1);
-  x_difvis<T>(b, wki2, v, rhsv, ny, 0, 0);
-  x_difvis<T>(b, wki3, w, rhsw, ru, 0, 0);
+  if (!kxc_difvisxx3<T>(b, wki3c, vel3, rhs3)) {
+    x_difvis<T>(b, wki1, u, rhsu, ru, 1, 1);
+    x_difvis<T>(b, wki2, v, rhsv, ny, 0, 0);
+    x_difvis<T>(b, wki3, w, rhsw, ru, 0, 0);
+  }
   // time step and RK constants
   LAUNCH(b, "dt", 1, 64, 0, dt_kernel, b.ds, b.vmbits, b.dc.dymin, ny, m, b.dt_mode == OTBL_DT_EVERY_STEP ? 1 : 0,
          b.hc.dxmin, b.hc.dtret, b.hc.rex, b.hc.rkc[m], b.hc.rkd[m], b.hc.rkcv[m], b.hc.rkdv[m]);

@@ -36,6 +36,19 @@
 
 namespace otbl {
 
+// an operator's arrays: lines in, velocity (derivatives), lines out, table(s),
+// closure rows, mode, values per plane; and up to three of a launch
+template <typename T> struct XOp {
+  const T *in, *vel;
+  T *out;
+  const T *tab, *tabv;
+  int c1, c2, mode;
+  size_t P;
+};
+template <typename T> struct XOps {
+  XOp<T> op[3];
+};
+
 // Table of one system of n planes in nc chunks of L (NL = nc L planes), by
 // phase, so that a phase reads one stream of scalars:
 //   forward   [NL][4]: stencil E1, E2, E3, multiplier M
@@ -107,10 +120,9 @@ void kxc_tables(Box &b) {
 
 // interpxx (lip.f90:248-300): midpoint interpolation along x
 template <int L, typename T>
-__global__ void __launch_bounds__(XCT, sizeof(T) == 4 ? 8 : 1)
-interpxx_c(const T *__restrict__ gen, T *__restrict__ geni, const T *__restrict__ tab, const T *__restrict__ inbx,
-           int chi, int chi2, int nx, size_t P, XChunk x) {
-  __shared__ T xch[2 * XCT];
+__device__ __forceinline__ void interpxx_b(const T *__restrict__ gen, T *__restrict__ geni, const T *__restrict__ tab,
+                                           const T *__restrict__ inbx, int chi, int chi2, int nx, size_t P,
+                                           const XChunk &x, T *xch) {
   const XPlace w(x, P);
   const XTabP<T> t(tab, x, L, w.c);
   const int j0 = w.c * L;
@@ -154,15 +166,23 @@ interpxx_c(const T *__restrict__ gen, T *__restrict__ geni, const T *__restrict_
   }
 }
 
+template <int L, typename T>
+__global__ void __launch_bounds__(XCT, sizeof(T) == 4 ? 8 : 1)
+interpxx_c(XOps<T> a, const T *__restrict__ inbx, int nx, XChunk x) {
+  __shared__ T xch[2 * XCT];
+  const XOp<T> &o = a.op[blockIdx.y];
+  interpxx_b<L, T>(o.in, o.out, o.tab, inbx, o.c1, o.c2, nx, o.P, x, xch);
+}
+
 // difvisxx (lip.f90:52-142): convective d/dx of the product plus rex times the
 // compact d2/dx2 of the velocity; mode 1 adds to out except on plane nx, which
 // gets the outflow derivative U_inf du/dx (lip.f90:105,132).
 template <int L, typename T>
-__global__ void __launch_bounds__(XCT, sizeof(T) == 4 ? 8 : 4)
-difvisxx_c(const T *__restrict__ gp, const T *__restrict__ qv, T *__restrict__ out, const T *__restrict__ tabc,
-           const T *__restrict__ tabv, const T *__restrict__ dcbx, const T *__restrict__ cofvbx, int chv, int ic,
-           int nx, size_t P, double rex_d, double idx_d, int mode, XChunk x) {
-  __shared__ T xch[4 * XCT];
+__device__ __forceinline__ void difvisxx_b(const T *__restrict__ gp, const T *__restrict__ qv, T *__restrict__ out,
+                                           const T *__restrict__ tabc, const T *__restrict__ tabv,
+                                           const T *__restrict__ dcbx, const T *__restrict__ cofvbx, int chv, int ic,
+                                           int nx, size_t P, double rex_d, double idx_d, int mode, const XChunk &x,
+                                           T *xch) {
   const XPlace w(x, P);
   const XTabP<T> tc(tabc, x, L, w.c), tv(tabv, x, L, w.c);
   const int j0 = w.c * L;
@@ -241,6 +261,15 @@ difvisxx_c(const T *__restrict__ gp, const T *__restrict__ qv, T *__restrict__ o
   }
 }
 
+template <int L, typename T>
+__global__ void __launch_bounds__(XCT, sizeof(T) == 4 ? 8 : 4)
+difvisxx_c(XOps<T> a, const T *__restrict__ dcbx, const T *__restrict__ cofvbx, int nx, double rex, double idx,
+           XChunk x) {
+  __shared__ T xch[4 * XCT];
+  const XOp<T> &o = a.op[blockIdx.y];
+  difvisxx_b<L, T>(o.in, o.vel, o.out, o.tab, o.tabv, dcbx, cofvbx, o.c1, o.c2, nx, o.P, rex, idx, o.mode, x, xch);
+}
+
 #define XDISPATCH(x, ...)                                                    \
   switch ((x).L) {                                                             \
   case 4: { constexpr int L = 4; __VA_ARGS__; } break;                         \
@@ -258,25 +287,68 @@ template <typename T> static const T *xtab_of(const Box &b, int sys) {
   else return b.xtab_f + at;
 }
 
+template <typename T>
+static XOp<T> x_interp_op(Box &b, const T *gen, T *geni, int which_u, int chi, int chi2, size_t P) {
+  return {gen, nullptr, geni, xtab_of<T>(b, which_u ? XT_INXU : XT_INXV), nullptr, chi, chi2, 0, P};
+}
+template <typename T>
+static XOp<T> x_difvis_op(Box &b, const T *prod, const T *vel, T *out, int which_u, int chv, int ic, size_t P,
+                          int mode) {
+  return {prod, vel, out, xtab_of<T>(b, which_u ? XT_DCXU : XT_DCXV), xtab_of<T>(b, which_u ? XT_VIXU : XT_VIXV), chv,
+          ic, mode, P};
+}
+// n operators in one launch (blockIdx.y); a shorter plane's last workgroups
+// repeat its last line without storing
+template <typename T> static void x_interp_launch(Box &b, const XOps<T> &a, int n) {
+  const dim3 grid(nblk(a.op[0].P, 64) * (unsigned)b.xci.ns, n);
+  XDISPATCH(b.xci, auto kf = &interpxx_c<L, T>; LAUNCH(b, "interpxx", grid, XCT, 0, kf, a, coefs<T>(b).inbx, b.nx, b.xci));
+}
+template <typename T> static void x_difvis_launch(Box &b, const XOps<T> &a, int n) {
+  const dim3 grid(nblk(a.op[0].P, 64) * (unsigned)b.xcd.ns, n);
+  XDISPATCH(b.xcd, auto kf = &difvisxx_c<L, T>;
+            LAUNCH(b, "difvisxx", grid, XCT, 0, kf, a, coefs<T>(b).dcbx, coefs<T>(b).cofvbx, b.nx, b.hc.rex, b.hc.idx,
+                   b.xcd));
+}
+
 template <typename T> void kxc_interpxx(Box &b, const T *gen, T *geni, int which_u, int chi, int chi2, size_t P) {
-  const unsigned grid = nblk(P, 64) * (unsigned)b.xci.ns;
-  XDISPATCH(b.xci, auto kf = &interpxx_c<L, T>;
-            LAUNCH(b, "interpxx", grid, XCT, 0, kf, gen, geni, xtab_of<T>(b, which_u ? XT_INXU : XT_INXV),
-                   coefs<T>(b).inbx, chi, chi2, b.nx, P, b.xci));
+  x_interp_launch<T>(b, {{x_interp_op<T>(b, gen, geni, which_u, chi, chi2, P)}}, 1);
 }
 
 template <typename T>
 void kxc_difvisxx(Box &b, const T *prod, const T *vel, T *out, int which_u, int chv, int ic, size_t P, int mode) {
-  const unsigned grid = nblk(P, 64) * (unsigned)b.xcd.ns;
-  XDISPATCH(b.xcd, auto kf = &difvisxx_c<L, T>;
-            LAUNCH(b, "difvisxx", grid, XCT, 0, kf, prod, vel, out, xtab_of<T>(b, which_u ? XT_DCXU : XT_DCXV),
-                   xtab_of<T>(b, which_u ? XT_VIXU : XT_VIXV), coefs<T>(b).dcbx, coefs<T>(b).cofvbx, chv, ic, b.nx, P,
-                   b.hc.rex, b.hc.idx, mode, b.xcd));
+  x_difvis_launch<T>(b, {{x_difvis_op<T>(b, prod, vel, out, which_u, chv, ic, P, mode)}}, 1);
 }
 
-template void kxc_interpxx<double>(Box &, const double *, double *, int, int, int, size_t);
-template void kxc_interpxx<float>(Box &, const float *, float *, int, int, int, size_t);
-template void kxc_difvisxx<double>(Box &, const double *, const double *, double *, int, int, int, size_t, int);
-template void kxc_difvisxx<float>(Box &, const float *, const float *, float *, int, int, int, size_t, int);
+// The three interpolations, or derivatives, of a substep (u, v, w) in one launch:
+// apart, each leaves part of the chip idle in small boxes and drains it in larger
+// ones.  us per substep, three launches -> one, interpxx / difvisxx: 32 x 40 x 24
+// FP64 20 / 24 -> 7 / 8, 256 x 96 x 64 FP64 38 / 59 -> 18 / 27, 387 x 113 x 98
+// mixed 35 / 54 -> 26 / 40, 896 x 176 x 224 FP64 287 / 568 -> 266 / 541, 1536 x 315
+// x 1024 mixed interpxx 1992 -> 1968.
+template <typename T> bool kxc_interpxx3(Box &b, const T *const *gen, T *const *geni) {
+  if (!b.xchunk) return false;
+  x_interp_launch<T>(b,
+                     {{x_interp_op<T>(b, gen[0], geni[0], 1, 2, 3, b.pu), x_interp_op<T>(b, gen[1], geni[1], 0, 1, 4, b.pv),
+                       x_interp_op<T>(b, gen[2], geni[2], 0, 1, 4, b.pu)}},
+                     3);
+  return true;
+}
+template <typename T> bool kxc_difvisxx3(Box &b, const T *const *prod, const T *const *vel, T *const *out) {
+  if (!b.xchunk || !b.xcd.L) return false;
+  x_difvis_launch<T>(b,
+                     {{x_difvis_op<T>(b, prod[0], vel[0], out[0], 1, 1, 3, b.pu, 1),
+                       x_difvis_op<T>(b, prod[1], vel[1], out[1], 0, 2, 1, b.pv, 0),
+                       x_difvis_op<T>(b, prod[2], vel[2], out[2], 0, 2, 1, b.pu, 0)}},
+                     3);
+  return true;
+}
+
+#define XINST(T)                                                                                  \
+  template void kxc_interpxx<T>(Box &, const T *, T *, int, int, int, size_t);                    \
+  template void kxc_difvisxx<T>(Box &, const T *, const T *, T *, int, int, int, size_t, int);    \
+  template bool kxc_interpxx3<T>(Box &, const T *const *, T *const *);                            \
+  template bool kxc_difvisxx3<T>(Box &, const T *const *, const T *const *, T *const *);
+XINST(double)
+XINST(float)
 
 } // namespace otbl

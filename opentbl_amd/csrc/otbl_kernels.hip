@@ -2286,16 +2286,20 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   if (tail) {
     // plane loop 2's y terms, boun's rows and the final update per component
     // in one pass each
-    ky_rk_tail<T>(b, 1, v, rhsv, resv, rp[1], ya, yb);
-    if (um) k_boun_mean(b);
-    ky_rk_tail<T>(b, 3, u, rhsu, resu, rp[0], (const T *)nullptr, (const T *)nullptr);
-    if constexpr (!F64) {
+    if constexpr (F64) {
+      double *const uu[3] = {u, v, w}, *const rh[3] = {rhsu, rhsv, rhsw};
+      const double *const rs[3] = {resu, resv, resw};
+      ky_rk_tail3(b, uu, rh, rs, rp, ya, yb, yc);
+    } else {
+      ky_rk_tail<T>(b, 1, v, rhsv, resv, rp[1], ya, yb);
+      k_boun_mean(b);
+      ky_rk_tail<T>(b, 3, u, rhsu, resu, rp[0], nullptr, nullptr);
       // the FP64 mean-flow u (kz = 0 real part)
       ky_mean_rk_final<T>(b, um, b.rm64, rhsu, rp[0]);
       LAUNCH(b, "rk_mean", nblk((size_t)nx * (ny + 1)), TPB, 0, mean_to_field_kernel<T>, u, (const double *)um, nx,
              ny + 1, nz1);
+      ky_rk_tail<T>(b, 2, w, rhsw, resw, rp[2], yc, ya);
     }
-    ky_rk_tail<T>(b, 2, w, rhsw, resw, rp[2], yc, ya);
     return;
   }
   // boundary conditions (rhsp.F90:421-445)

@@ -213,9 +213,12 @@ void ky_rhs_loop2(Box &b, T *rhsu, T *rhsv, T *rhsw, const T *resu, const T *res
 template <typename T> void ky_rk_final(Box &b, int k, T *u, const T *res, const T *rhs, const T *rhsp);
 // plane loop 2's y terms, boun's rows and rk_final of one component in one
 // pass (k2 = 1 v, 2 w, 3 u); pa, pb: the loop's products (v: vw, vv; w: ww,
-// vw; u: none)
+// vw; u: none); ky_rk_tail3: the three of an FP64 box (arrays by component
+// u, v, w)
 template <typename T>
 void ky_rk_tail(Box &b, int k2, T *u, T *rhs, const T *res, const T *rhsp, const T *pa, const T *pb);
+void ky_rk_tail3(Box &b, double *const *u, double *const *rhs, const double *const *res, const double *const *rhsp,
+                 const double *vw, const double *vv, const double *ww);
 // boun's boundary rows of the FP64 mean-flow u of the mixed substep
 void k_boun_mean(Box &b);
 // FP32 tables of the half-wave chunking of the six fixed systems

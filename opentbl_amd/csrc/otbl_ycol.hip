@@ -802,31 +802,20 @@ rk_final_yh(float *u, const float *__restrict__ res, const float *__restrict__ r
 // the fused kernel spilled and measured slower than the three passes (9.0
 // against 7.7 ms per substep at 1536 x 315 x 1024), so those keep them; on
 // the full-wave chunks FP64 took 12.7 ms against 14.6.
+template <typename T> struct TailArgs { // one component's arrays and tables
+  T *u, *rhs;
+  const T *res, *rhsp, *pa, *pb, *tabv, *tabi, *tabd;
+  const double *f;
+};
+
 template <int L, typename T, int K2>
-__global__ void __launch_bounds__(YTPB)
-rk_tail_y(T *u, T *rhs, const T *__restrict__ res, const T *__restrict__ rhsp, const T *__restrict__ pa,
-          const T *__restrict__ pb, const T *__restrict__ tabv, const T *__restrict__ tabi,
-          const T *__restrict__ tabd, DevCoefT<T> c, const double *__restrict__ f,
-          const DevScalars *__restrict__ ds, const double *__restrict__ um, Predictor<T> P, int jee, int ny, int nz1,
-          int nx) {
+__device__ __forceinline__ void
+rk_tail_b(T *u, T *rhs, const T *__restrict__ res, const T *__restrict__ rhsp, const T *__restrict__ pa,
+          const T *__restrict__ pb, const T *__restrict__ tlv, const T *__restrict__ tli,
+          const T *__restrict__ tld, const DevCoefT<T> &c, const double *__restrict__ f,
+          const DevScalars *__restrict__ ds, const double *__restrict__ um, const Predictor<T> &P, int jee, int ny,
+          int nz1, int nx, T *xch, T *hal, T *bx) {
   constexpr bool SOLVE = K2 != 3;
-  __shared__ T xch[2 * YNCH * 64];
-  __shared__ T hal[2 * YNCH * 64];
-  __shared__ T bx[3 * 64];
-  constexpr bool STAGE = sizeof(T) == 4;
-  __shared__ T tlv_s[STAGE ? ytab_size(L) : 1], tli_s[STAGE ? ytab_size(L) : 1];
-  __shared__ T tld_s[STAGE && SOLVE ? ytab_size(L) : 1];
-  const T *tlv = tabv, *tli = tabi, *tld = tabd;
-  if constexpr (STAGE) {
-    ytab_stage<L>(tlv_s, tabv);
-    ytab_stage<L>(tli_s, tabi);
-    tlv = tlv_s;
-    tli = tli_s;
-    if constexpr (SOLVE) {
-      ytab_stage<L>(tld_s, tabd);
-      tld = tld_s;
-    }
-  }
   const YCol q = ycol((size_t)nz1 * nx, nz1, 0);
   const size_t s = nz1, off = q.ip * s * jee + q.kr;
   const size_t opu = q.ip * s * (ny + 1) + q.kr, opp = opu - q.kr + (q.kr ^ 1);
@@ -971,6 +960,53 @@ rk_tail_y(T *u, T *rhs, const T *__restrict__ res, const T *__restrict__ rhsp, c
     const int j = j0 + r;
     if (act && j >= 1 && j < jee - 1) u[off + (size_t)j * s2] = t[r];
   }
+}
+
+// one component; FP32 stages its tables in LDS
+template <int L, typename T, int K2>
+__global__ void __launch_bounds__(YTPB)
+rk_tail_y(T *u, T *rhs, const T *__restrict__ res, const T *__restrict__ rhsp, const T *__restrict__ pa,
+          const T *__restrict__ pb, const T *__restrict__ tabv, const T *__restrict__ tabi,
+          const T *__restrict__ tabd, DevCoefT<T> c, const double *__restrict__ f,
+          const DevScalars *__restrict__ ds, const double *__restrict__ um, Predictor<T> P, int jee, int ny, int nz1,
+          int nx) {
+  __shared__ T xch[2 * YNCH * 64], hal[2 * YNCH * 64], bx[3 * 64];
+  constexpr bool STAGE = sizeof(T) == 4, SOLVE = K2 != 3;
+  __shared__ T tlv_s[STAGE ? ytab_size(L) : 1], tli_s[STAGE ? ytab_size(L) : 1];
+  __shared__ T tld_s[STAGE && SOLVE ? ytab_size(L) : 1];
+  const T *tlv = tabv, *tli = tabi, *tld = tabd;
+  if constexpr (STAGE) {
+    ytab_stage<L>(tlv_s, tabv);
+    ytab_stage<L>(tli_s, tabi);
+    tlv = tlv_s;
+    tli = tli_s;
+    if constexpr (SOLVE) {
+      ytab_stage<L>(tld_s, tabd);
+      tld = tld_s;
+    }
+  }
+  rk_tail_b<L, T, K2>(u, rhs, res, rhsp, pa, pb, tlv, tli, tld, c, f, ds, um, P, jee, ny, nz1, nx, xch, hal, bx);
+}
+
+// The three components of an FP64 box in one launch (blockIdx.y: v, w, u), for
+// boxes whose workgroups (one per CU) all run at once: us per substep, three
+// launches -> one, 32 x 40 x 24 46 -> 21 (27 workgroups).  With the three bodies'
+// registers a workgroup itself is slower, so two rounds of them lose: 256 x 96 x
+// 64 (504 workgroups on 256 CUs) 74 -> 79.
+template <int L>
+__global__ void __launch_bounds__(YTPB)
+rk_tail3_y(TailArgs<double> v, TailArgs<double> w, TailArgs<double> u, DevCoef c, const DevScalars *__restrict__ ds,
+           Predictor<double> P, int ny, int nz1, int nx) {
+  __shared__ double xch[2 * YNCH * 64], hal[2 * YNCH * 64], bx[3 * 64];
+  if (blockIdx.y == 0)
+    rk_tail_b<L, double, 1>(v.u, v.rhs, v.res, v.rhsp, v.pa, v.pb, v.tabv, v.tabi, v.tabd, c, v.f, ds, nullptr, P, ny,
+                            ny, nz1, nx, xch, hal, bx);
+  else if (blockIdx.y == 1)
+    rk_tail_b<L, double, 2>(w.u, w.rhs, w.res, w.rhsp, w.pa, w.pb, w.tabv, w.tabi, w.tabd, c, w.f, ds, nullptr, P,
+                            ny + 1, ny, nz1, nx, xch, hal, bx);
+  else
+    rk_tail_b<L, double, 3>(u.u, u.rhs, u.res, u.rhsp, u.pa, u.pb, u.tabv, u.tabi, u.tabd, c, u.f, ds, nullptr, P,
+                            ny + 1, ny, nz1, nx, xch, hal, bx);
 }
 
 // boun's rows 1 and ny+1 of the FP64 mean-flow u of the mixed substep
@@ -1138,22 +1174,45 @@ template <typename T> void ky_rk_final(Box &b, int k, T *u, const T *res, const 
 // chunks; pa, pb the products of plane loop 2 (v: vw, vv; w: ww, vw; u:
 // unused)
 template <typename T>
+static TailArgs<T> tail_args(Box &b, int k2, T *u, T *rhs, const T *res, const T *rhsp, const T *pa, const T *pb) {
+  return {u, rhs, res, rhsp, k2 == 3 ? nullptr : pa, k2 == 3 ? nullptr : pb,
+          ytab<T>(b, k2 == 1 ? YT_VIYV : YT_VIYU), ytab<T>(b, k2 == 1 ? YT_IMPV : YT_IMPU),
+          ytab<T>(b, k2 == 1 ? YT_DCYV : YT_DCYU), k2 == 1 ? b.implv : b.implu};
+}
+
+template <typename T>
 void ky_rk_tail(Box &b, int k2, T *u, T *rhs, const T *res, const T *rhsp, const T *pa, const T *pb) {
   const int jee = k2 == 1 ? b.ny : b.ny + 1;
-  const bool uu = jee == b.ny + 1;
-  const int kv = uu ? YT_VIYU : YT_VIYV, ki = uu ? YT_IMPU : YT_IMPV, kd = k2 == 1 ? YT_DCYV : YT_DCYU;
-  const double *um = (k2 == 3 && b.precision == OTBL_MIXED) ? b.um64 : nullptr;
-  if (k2 == 3) pa = pb = nullptr;
+  const TailArgs<T> a = tail_args<T>(b, k2, u, rhs, res, rhsp, pa, pb);
+  const double *um = sizeof(T) == 4 && k2 == 3 ? b.um64 : nullptr;
   const unsigned g = ygrid((size_t)b.nz1 * b.nx);
   YDISPATCH(b.yL, auto kf = k2 == 1 ? &rk_tail_y<L, T, 1> : (k2 == 2 ? &rk_tail_y<L, T, 2> : &rk_tail_y<L, T, 3>);
-            LAUNCH(b, "rk_tail", g, YTPB, 0, kf, u, rhs, res, rhsp, pa, pb, ytab<T>(b, kv), ytab<T>(b, ki),
-                   ytab<T>(b, kd), coefs<T>(b), uu ? b.implu : b.implv, b.ds, um, predictor<T>(b), jee,
-                   b.ny, b.nz1, b.nx));
+            LAUNCH(b, "rk_tail", g, YTPB, 0, kf, a.u, a.rhs, a.res, a.rhsp, a.pa, a.pb, a.tabv, a.tabi, a.tabd,
+                   coefs<T>(b), a.f, b.ds, um, predictor<T>(b), jee, b.ny, b.nz1, b.nx));
 }
+
 template void ky_rk_tail<double>(Box &, int, double *, double *, const double *, const double *, const double *,
                                  const double *);
 template void ky_rk_tail<float>(Box &, int, float *, float *, const float *, const float *, const float *,
                                 const float *);
+
+void ky_rk_tail3(Box &b, double *const *u, double *const *rhs, const double *const *res, const double *const *rhsp,
+                 const double *vw, const double *vv, const double *ww) {
+  using T = double;
+  // one round of workgroups, and chunks that leave the fused kernel unspilled
+  if (b.yL > 8 || 3 * ygrid((size_t)b.nz1 * b.nx) > 256) {
+    ky_rk_tail<T>(b, 1, u[1], rhs[1], res[1], rhsp[1], vw, vv);
+    ky_rk_tail<T>(b, 3, u[0], rhs[0], res[0], rhsp[0], nullptr, nullptr);
+    ky_rk_tail<T>(b, 2, u[2], rhs[2], res[2], rhsp[2], ww, vw);
+    return;
+  }
+  const TailArgs<T> av = tail_args<T>(b, 1, u[1], rhs[1], res[1], rhsp[1], vw, vv);
+  const TailArgs<T> aw = tail_args<T>(b, 2, u[2], rhs[2], res[2], rhsp[2], ww, vw);
+  const TailArgs<T> au = tail_args<T>(b, 3, u[0], rhs[0], res[0], rhsp[0], nullptr, nullptr);
+  const dim3 g(ygrid((size_t)b.nz1 * b.nx), 3);
+  auto kf = b.yL == 4 ? &rk_tail3_y<4> : &rk_tail3_y<8>;
+  LAUNCH(b, "rk_tail", g, YTPB, 0, kf, av, aw, au, b.dc, b.ds, predictor<T>(b), b.ny, b.nz1, b.nx);
+}
 
 void k_boun_mean(Box &b) {
   LAUNCH(b, "boun", (b.nx + 255) / 256, 256, 0, boun_mean_kernel, b.um64, b.dc, b.ny, b.nx);

@@ -60,7 +60,7 @@ def kernel_model(cfg, s=8):
     m["rhsu_loop1"] = ((Rv + 2 * Ru) * f, 0.0, 1)
     # rhsu, rhsv, rhsw read and written; resu, resv, resw, vw, vv, ww read
     m["rhs_loop2"] = ((X - 2) * z * s * (2 * Ru + 2 * Rv + 2 * Ru + Ru + Rv + Ru + Ru + Rv + Rv), 0.0, 1)
-    # res, rhs, rhs_prev, u read; u written (rhs becomes rhs_prev by a role swap)
+    # res, p, rhs, rhs_prev read; u written (rhs becomes rhs_prev by a role swap)
     m["rk_final"] = ((5 * Ru + 5 * Rv + 5 * Ru) * f / 3, 0.0, 3)
     # the fused tail per component (FP64 / full-wave y): rhs and the field read
     # and written, res and rhs_prev read, and for v and w the two products of
@@ -86,8 +86,9 @@ def kernel_model(cfg, s=8):
 # kernel-event names -> HIP kernel function names in rocprofv3 output
 TRACE_NAMES = {"dct2_rows": "dct_rows_z", "dct3_rows": "dct_rows_z", "div": "div_pencils_kernel",
                "poisson_y": "poisson_y_chunk", "to_planes": "pencils_to_planes_kernel",
-               "products1": ("products1_zp", "products1_z"), "products2": "products2_z", "interpxx": "interpxx_w",
-               "difvisxx": "difvisxx_w", "interpyy": "interpyy_y", "rhsu_loop1": "rhsu_loop1_y",
+               "products1": ("products1_zp", "products1_z"), "products2": ("products2_t", "products2_z"),
+               "interpxx": ("interpxx_c", "interpxx_w"),
+               "difvisxx": ("difvisxx_w", "difvisxx_c"), "interpyy": "interpyy_y", "rhsu_loop1": "rhsu_loop1_y",
                "rhs_loop2": "rhs_loop2_y", "rk_final": ("rk_final_y", "rk_final_yh"), "rk_tail": "rk_tail_y",
                "project": ("project_kernel", "project_pair_kernel"),
                "save_predict": ("save_predict_kernel", "save_predict_pair_kernel")}
@@ -228,9 +229,12 @@ def run_box(cfg, st, precision, args):
 
 def report(name, rep, model):
     rows = []
+    substeps = rep.get("products1", (0, 0.0))[0]
     for kname, (n, ms) in sorted(rep.items(), key=lambda kv: -kv[1][1]):
         avg = ms / n
-        by, fl, _ = model.get(kname, (None, None, None))
+        by, fl, per = model.get(kname, (None, None, None))
+        if by and substeps and n < per * substeps:  # several components in one launch
+            by *= per * substeps / n
         gbs = by / (avg * 1e-3) / 1e9 if by else None
         tfs = fl / (avg * 1e-3) / 1e12 if fl else None
         rows.append((kname, n, ms, avg, gbs, tfs))

@@ -265,16 +265,18 @@ int otbl_d2d(void *dst, const void *src, size_t bytes);
 /* Kernel paths the context chose at setup, as text: "y:chunk<L>|march0
  * z:engine<nz>|stockham<nz> dct:engine<M>|stockham<M>|gemm<M> x:window|march
  * xseg:<threads per x line> pois:chunk<L>|march0 prun:<planes per thread>
- * tuned:0|1 streams:1|2" (streams:2: rhsp's plane loop 2 on a second stream
- * beside plane loop 1)
+ * tuned:0|1 streams:1|2 tail:0|1 zteam:<lanes per z row> xchunk:<planes>"
+ * (streams:2: rhsp's plane loop 2 on a second stream beside plane loop 1;
+ * tail:1: rhsp's tail fused per component; zteam, xchunk: 0 or the kernels with
+ * several z rows per wavefront, x lines in chunks)
  * (no counterpart in the reference; for tests and benchmark records). */
 int otbl_get_paths(otbl_ctx *ctx, char *buf, size_t len);
 
 /* Autotuner (no counterpart in the reference): times, on this box's sizes,
  * the candidate launch shapes of its kernels and keeps the fastest: the
  * segments per x line of the windowed x solves (1 up to the most the x
- * systems' decay allows), the planes per thread of the element-wise
- * predictor and projection (1, 2, 4, 8), and for the mixed substep the
+ * systems' decay allows) or their chunks, the planes per thread of the
+ * projection (1, 2, 4, 8), and for the mixed substep the
  * half-wave or full-wave chunks of rk_final.  Each candidate runs `reps`
  * times (after one untimed run) on the box's work fields, which hold nothing
  * between substeps, so the state is unchanged.  The plane run changes no

@@ -1,10 +1,12 @@
-// HIP kernels of the RK3 substep (FP64 path) for gfx950.
+// HIP kernels of the RK3 substep for gfx950: the general paths, the element-wise
+// and one-workgroup kernels, and the substep's order.  The chunked x and y lines,
+// the register z transforms and the Poisson chunks have files of their own.
 //
 // Data layout (the reference's planes): a complex field (0:nz2, R, 1:nx) as
 // doubles, real index kr = 0..nz1-1 fastest, then row j = 1..R, then plane i.
 // Element (kr, j, i) sits at (i-1)*P + (j-1)*nz1 + kr with P = R*nz1.
 //
-// Line solves map one thread to one line:
+// The line solves here map one thread to one line:
 //  * x lines (lip.f90 interpxx/difvisxx): a line is a fixed (kr, j); the
 //    thread marches over planes, so a wavefront reads 64 consecutive doubles
 //    of one plane per step (coalesced), no plane<->pencil transpose.
@@ -2229,7 +2231,7 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   // flow of the mixed substep is predicted here
   double *um = F64 ? nullptr : b.um64; // the FP64 mean-flow u of the mixed substep
   if (um)
-    LAUNCH(b, "save_predict", nblk((size_t)nx * (ny + 1)), TPB, 0, mean_predict_kernel, um, b.rm64,
+    LAUNCH(b, "mean_predict", nblk((size_t)nx * (ny + 1)), TPB, 0, mean_predict_kernel, um, b.rm64,
            (const double *)b.p0, (const float *)v, (float *)resv, b.dc.idyy, b.ds, b.hc.idxx, nx, ny, nz1);
   if constexpr (F64)
     if (!b.yL) save_predict_launch(b, resu, resv, resw, prun<T>(b));

@@ -8,15 +8,17 @@
 // of a substep:
 //   stats_x     x lines: u_x = midpoint interpolation of u (interpx_new)
 //               moved one plane up, and d/dx (diffx_inplace) of u_x, v, w;
+//               in chunks over the wavefronts of a workgroup (stats_xc), else
 //               one thread per line marching over the planes
 //   stats_y     y lines of every (kr, plane) column: the midpoint
 //               interpolations to the v rows (interpy_new) of u_x, w, dw/dx,
 //               du/dx and p, and d/dy (diffy_inplace) of (u_x)_y, w_y, v
-//   stats_z     one (j, i) row per workgroup: the sums over the spanwise
+//   stats_z     several (j, i) rows per wavefront (stats_t), one per engine team,
+//               or one per workgroup: the sums over the spanwise
 //               modes, the k = 0 means, and through three packed c2r
-//               transforms (LDS Stockham) the enstrophy and the triple
+//               transforms the enstrophy and the triple
 //               products in physical space; the row's 40 sums are added to
-//               the accumulators by one thread (no atomics: the sums are
+//               the accumulators by one lane (no atomics: the sums are
 //               reproducible).
 // Arithmetic is FP64; the mixed box's FP32 fields are widened on load and
 // its intermediate fields are held in FP32.

@@ -168,7 +168,18 @@ __device__ __forceinline__ void interpxx_b(const T *__restrict__ gen, T *__restr
 
 template <int L, typename T>
 __global__ void __launch_bounds__(XCT, sizeof(T) == 4 ? 8 : 1)
-interpxx_c(XOps<T> a, const T *__restrict__ inbx, int nx, XChunk x) {
+interpxx_c(const T *__restrict__ gen, T *__restrict__ geni, const T *__restrict__ tab, const T *__restrict__ inbx,
+           int chi, int chi2, int nx, size_t P, XChunk x) {
+  __shared__ T xch[2 * XCT];
+  interpxx_b<L, T>(gen, geni, tab, inbx, chi, chi2, nx, P, x, xch);
+}
+
+// the three components of a substep (blockIdx.y).  For one operator the kernel
+// above is faster (its arguments are known not to alias): 4% of the passes over
+// 98304 lines of 1024 planes.
+template <int L, typename T>
+__global__ void __launch_bounds__(XCT, sizeof(T) == 4 ? 8 : 1)
+interpxx3_c(XOps<T> a, const T *__restrict__ inbx, int nx, XChunk x) {
   __shared__ T xch[2 * XCT];
   const XOp<T> &o = a.op[blockIdx.y];
   interpxx_b<L, T>(o.in, o.out, o.tab, inbx, o.c1, o.c2, nx, o.P, x, xch);
@@ -263,7 +274,16 @@ __device__ __forceinline__ void difvisxx_b(const T *__restrict__ gp, const T *__
 
 template <int L, typename T>
 __global__ void __launch_bounds__(XCT, sizeof(T) == 4 ? 8 : 4)
-difvisxx_c(XOps<T> a, const T *__restrict__ dcbx, const T *__restrict__ cofvbx, int nx, double rex, double idx,
+difvisxx_c(const T *__restrict__ gp, const T *__restrict__ qv, T *__restrict__ out, const T *__restrict__ tabc,
+           const T *__restrict__ tabv, const T *__restrict__ dcbx, const T *__restrict__ cofvbx, int chv, int ic,
+           int nx, size_t P, double rex, double idx, int mode, XChunk x) {
+  __shared__ T xch[4 * XCT];
+  difvisxx_b<L, T>(gp, qv, out, tabc, tabv, dcbx, cofvbx, chv, ic, nx, P, rex, idx, mode, x, xch);
+}
+
+template <int L, typename T>
+__global__ void __launch_bounds__(XCT, sizeof(T) == 4 ? 8 : 4)
+difvisxx3_c(XOps<T> a, const T *__restrict__ dcbx, const T *__restrict__ cofvbx, int nx, double rex, double idx,
            XChunk x) {
   __shared__ T xch[4 * XCT];
   const XOp<T> &o = a.op[blockIdx.y];
@@ -297,26 +317,33 @@ static XOp<T> x_difvis_op(Box &b, const T *prod, const T *vel, T *out, int which
   return {prod, vel, out, xtab_of<T>(b, which_u ? XT_DCXU : XT_DCXV), xtab_of<T>(b, which_u ? XT_VIXU : XT_VIXV), chv,
           ic, mode, P};
 }
-// n operators in one launch (blockIdx.y); a shorter plane's last workgroups
-// repeat its last line without storing
-template <typename T> static void x_interp_launch(Box &b, const XOps<T> &a, int n) {
-  const dim3 grid(nblk(a.op[0].P, 64) * (unsigned)b.xci.ns, n);
-  XDISPATCH(b.xci, auto kf = &interpxx_c<L, T>; LAUNCH(b, "interpxx", grid, XCT, 0, kf, a, coefs<T>(b).inbx, b.nx, b.xci));
-}
-template <typename T> static void x_difvis_launch(Box &b, const XOps<T> &a, int n) {
-  const dim3 grid(nblk(a.op[0].P, 64) * (unsigned)b.xcd.ns, n);
-  XDISPATCH(b.xcd, auto kf = &difvisxx_c<L, T>;
-            LAUNCH(b, "difvisxx", grid, XCT, 0, kf, a, coefs<T>(b).dcbx, coefs<T>(b).cofvbx, b.nx, b.hc.rex, b.hc.idx,
-                   b.xcd));
-}
-
 template <typename T> void kxc_interpxx(Box &b, const T *gen, T *geni, int which_u, int chi, int chi2, size_t P) {
-  x_interp_launch<T>(b, {{x_interp_op<T>(b, gen, geni, which_u, chi, chi2, P)}}, 1);
+  const unsigned grid = nblk(P, 64) * (unsigned)b.xci.ns;
+  XDISPATCH(b.xci, auto kf = &interpxx_c<L, T>;
+            LAUNCH(b, "interpxx", grid, XCT, 0, kf, gen, geni, xtab_of<T>(b, which_u ? XT_INXU : XT_INXV),
+                   coefs<T>(b).inbx, chi, chi2, b.nx, P, b.xci));
 }
 
 template <typename T>
 void kxc_difvisxx(Box &b, const T *prod, const T *vel, T *out, int which_u, int chv, int ic, size_t P, int mode) {
-  x_difvis_launch<T>(b, {{x_difvis_op<T>(b, prod, vel, out, which_u, chv, ic, P, mode)}}, 1);
+  const unsigned grid = nblk(P, 64) * (unsigned)b.xcd.ns;
+  XDISPATCH(b.xcd, auto kf = &difvisxx_c<L, T>;
+            LAUNCH(b, "difvisxx", grid, XCT, 0, kf, prod, vel, out, xtab_of<T>(b, which_u ? XT_DCXU : XT_DCXV),
+                   xtab_of<T>(b, which_u ? XT_VIXU : XT_VIXV), coefs<T>(b).dcbx, coefs<T>(b).cofvbx, chv, ic, b.nx, P,
+                   b.hc.rex, b.hc.idx, mode, b.xcd));
+}
+
+// three operators in one launch; a shorter plane's last workgroups repeat its
+// last line without storing
+template <typename T> static void x_interp_launch(Box &b, const XOps<T> &a) {
+  const dim3 grid(nblk(a.op[0].P, 64) * (unsigned)b.xci.ns, 3);
+  XDISPATCH(b.xci, auto kf = &interpxx3_c<L, T>; LAUNCH(b, "interpxx", grid, XCT, 0, kf, a, coefs<T>(b).inbx, b.nx, b.xci));
+}
+template <typename T> static void x_difvis_launch(Box &b, const XOps<T> &a) {
+  const dim3 grid(nblk(a.op[0].P, 64) * (unsigned)b.xcd.ns, 3);
+  XDISPATCH(b.xcd, auto kf = &difvisxx3_c<L, T>;
+            LAUNCH(b, "difvisxx", grid, XCT, 0, kf, a, coefs<T>(b).dcbx, coefs<T>(b).cofvbx, b.nx, b.hc.rex, b.hc.idx,
+                   b.xcd));
 }
 
 // The three interpolations, or derivatives, of a substep (u, v, w) in one launch:
@@ -329,8 +356,7 @@ template <typename T> bool kxc_interpxx3(Box &b, const T *const *gen, T *const *
   if (!b.xchunk) return false;
   x_interp_launch<T>(b,
                      {{x_interp_op<T>(b, gen[0], geni[0], 1, 2, 3, b.pu), x_interp_op<T>(b, gen[1], geni[1], 0, 1, 4, b.pv),
-                       x_interp_op<T>(b, gen[2], geni[2], 0, 1, 4, b.pu)}},
-                     3);
+                       x_interp_op<T>(b, gen[2], geni[2], 0, 1, 4, b.pu)}});
   return true;
 }
 template <typename T> bool kxc_difvisxx3(Box &b, const T *const *prod, const T *const *vel, T *const *out) {
@@ -338,8 +364,7 @@ template <typename T> bool kxc_difvisxx3(Box &b, const T *const *prod, const T *
   x_difvis_launch<T>(b,
                      {{x_difvis_op<T>(b, prod[0], vel[0], out[0], 1, 1, 3, b.pu, 1),
                        x_difvis_op<T>(b, prod[1], vel[1], out[1], 0, 2, 1, b.pv, 0),
-                       x_difvis_op<T>(b, prod[2], vel[2], out[2], 0, 2, 1, b.pu, 0)}},
-                     3);
+                       x_difvis_op<T>(b, prod[2], vel[2], out[2], 0, 2, 1, b.pu, 0)}});
   return true;
 }
 

@@ -1,6 +1,7 @@
-// FFTs along z with several rows per wavefront, for the lengths up to 1024
-// that the engine of otbl_zfft.h (one row per wavefront or more) has no plan
-// for: every even 2^a 3^b 5^c 7^d.
+// FFTs along z with several rows per wavefront, for every even length
+// 2^a 3^b 5^c 7^d from 12 to 1024; the engine of otbl_zfft.h (one row per
+// wavefront or more) keeps FP32 plane loop 1 at 512 and 1024 and the lengths
+// above.
 //
 // A row of N points belongs to a team of G lanes; a wavefront carries
 // T = 64 / G teams (lanes past T G idle).  A transform is two or three

@@ -90,7 +90,7 @@ struct ZTeamFns {
   void (*p2f)(const float *, const float *, float *, float *, float *, const float2 *, int, int) = nullptr;
   void (*fx)(double *, double *, int, const double2 *, int) = nullptr;
   void (*std_)(StatsZ, const double2 *, int, int, int) = nullptr; // statistics
-  void (*stf)(StatsZ, const float2 *, int, int, int) = nullptr;
+  void (*stf)(StatsZ, const double2 *, int, int, int) = nullptr;
 };
 // row lengths of those kernels: even products of 2, 3, 5, 7 from 12 to 1024
 constexpr bool zteam_length(int n) {

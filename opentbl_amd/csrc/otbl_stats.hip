@@ -21,7 +21,8 @@
 //               the accumulators by one lane (no atomics: the sums are
 //               reproducible).
 // Arithmetic is FP64; the mixed box's FP32 fields are widened on load and
-// its intermediate fields are held in FP32.
+// its intermediate fields are held in FP32.  Only stats_zr on FP32 rows (512,
+// 1024, 2048, 4096 points) runs its three transforms in FP32.
 #include "otbl_kcommon.h"
 #include "otbl_fft.h"
 #include "otbl_zfft.h"
@@ -934,7 +935,10 @@ template <typename T> static void statsp_t(Box &b) {
   az.kaz = b.dc.kaz;
   az.acc = b.st;
   az.ens = b.ens;
-  if (b.zteam.nz) {
+  // the engine beyond the team lengths, and for the FP32 rows of 512 and 1024,
+  // where FP64 teams take 430 against 288 and 1005 against 508 us (256 x 96 rows;
+  // at 256 229 against 237)
+  if (b.zteam.nz && !(std::is_same<T, float>::value && b.zfast && b.nz > 256)) {
     kzt_stats<T>(b, az);
     return;
   }
@@ -946,14 +950,18 @@ template <typename T> static void statsp_t(Box &b) {
   case NN:                                                                                                         \
     LAUNCH(b, "stats_z", (unsigned)((nrows + ZTeam<NN>::TEAMS - 1) / ZTeam<NN>::TEAMS), ZTeam<NN>::TPB_, 0,       \
            (stats_zr<NN, T>), az, tw, nx, ny, nz1, nrows);                                                      \
-    break;
+    return;
+    if constexpr (std::is_same<T, float>::value)
+      switch (b.nz) {
+        SZR(512)
+        SZR(1024)
+      }
     switch (b.nz) {
       SZR(2048)
       SZR(4096)
 #undef SZR
     default: throw std::invalid_argument("stats: z length not on the register engine");
     }
-    return;
   }
   LAUNCH(b, "stats_z", dim3(ny, nx), TPB, k_stats_shm_bytes(b.nz), stats_z_kernel<T>, az, b.zplan, nx, ny, nz1,
          b.nz2);

@@ -639,7 +639,7 @@ template <> void kz_dct_pencils<float>(Box &b, float *P, int iopt, int Lp, int l
 template <typename R> void kzt_stats(Box &b, const StatsZ &a) {
   zcheck(b);
   const int nrows = b.ny * b.nx;
-  auto launch = [&](auto kf) { LAUNCH(b, "stats_z", tgrid(b, nrows), 64, 0, kf, a, ztw<R>(b), b.nx, b.ny, nrows); };
+  auto launch = [&](auto kf) { LAUNCH(b, "stats_z", tgrid(b, nrows), 64, 0, kf, a, ztw<double>(b), b.nx, b.ny, nrows); };
   if constexpr (sizeof(R) == 8) launch(b.zteam.std_);
   else launch(b.zteam.stf);
 }

@@ -199,13 +199,18 @@ template <int G> __device__ __forceinline__ double team_sum(double v, int t) {
   return v;
 }
 
-// Row sums of the statistics (stotf.F90:148-283) for one (j, i) row, as
-// stats_zr: three packed c2r transforms in the fields' precision, the physical
-// products and every sum in FP64.
+// Row sums of the statistics (stotf.F90:148-283) for one (j, i) row: three
+// packed c2r transforms, the physical products and every sum in FP64, whatever
+// the fields hold (R).  FP32 transforms would carry the round-off of the mean
+// flow, O(1), into the enstrophy and the triple products: 4 to 12 times the
+// error of the former and up to 1e3 times that of u^3 on a mixed box.  Bound by
+// FP64 arithmetic and the registers of its transforms.  us per sample of 256 x 96
+// rows, one row per workgroup (the LDS kernel) -> here: mixed rows of 64 points
+// 3254 -> 57, 96 3408 -> 86, 224 3658 -> 198; FP64 224 3722 -> 210.
 template <int N, typename R>
 __global__ void __launch_bounds__(64)
-stats_t(StatsZ a, const typename CT<R>::c *__restrict__ tw, int nx, int ny, int nrows) {
-  using C = typename CT<R>::c;
+stats_t(StatsZ a, const double2 *__restrict__ tw, int nx, int ny, int nrows) {
+  using C = double2;
   using Z = ZRow<N>;
   using F = ZRowPhys<N>;
   constexpr int nz1 = 2 * (N / 3), nz2 = N / 3 - 1;
@@ -222,22 +227,25 @@ stats_t(StatsZ a, const typename CT<R>::c *__restrict__ tw, int nx, int ny, int 
   for (int q = 0; q < 8; ++q) Bq[q] = (const R *)a.B[q] + ov;
   const R *V = (const R *)a.v + ov, *DV = (const R *)a.dvdx + ov;
   const size_t om = (size_t)j * nx + i; // (i, j) of the [ny][nx] mean-flow rows
-  // mode 0 of B1 (u_x at the v rows) with the FP64 mean flow of a mixed box
-  const R m1 = a.m1 ? (R)a.m1[om] : R(0);
-  auto b1at = [&](unsigned k) {
-    C b = tld<C>(Bq[0], o + k);
-    if (a.m1 && k == 0) b.x = m1;
+  auto at = [&](const R *p, unsigned k) {
+    const typename CT<R>::c b = tld<typename CT<R>::c>(p, o + k);
+    return make_double2((double)b.x, (double)b.y);
+  };
+  // B1 (u_x at the v rows), B4, B6 with the FP64 mean flow of a mixed box (m)
+  auto mean_at = [&](const R *p, const double *m, unsigned k) {
+    double2 b = at(p, k);
+    if (m && k == 0) b.x = m[om];
     return b;
   };
   double sum[NSUM];
 #pragma unroll
   for (int q = 0; q < NSUM; ++q) sum[q] = 0.0;
-  R s2[F::E], U[F::E];
+  double s2[F::E], U[F::E];
   C v[Z::E];
   // omega_x + i omega_y
   tload_modes<N, true, C>(v, t, [&](unsigned k, C &x, C &y) {
-    const R kz = (R)a.kaz[k];
-    const C b7 = tld<C>(Bq[6], o + k), vv = tld<C>(V, o + k), b1 = b1at(k), b3 = tld<C>(Bq[2], o + k);
+    const double kz = a.kaz[k];
+    const C b7 = at(Bq[6], k), vv = at(V, k), b1 = mean_at(Bq[0], a.m1, k), b3 = at(Bq[2], k);
     x = mkc<C>(b7.x + kz * vv.y, b7.y - kz * vv.x);
     y = mkc<C>(-kz * b1.y - b3.x, kz * b1.x - b3.y);
   });
@@ -246,9 +254,9 @@ stats_t(StatsZ a, const typename CT<R>::c *__restrict__ tw, int nx, int ny, int 
   for (int e = 0; e < F::E; ++e) s2[e] = v[e].x * v[e].x + v[e].y * v[e].y;
   // omega_z + i u
   tload_modes<N, true, C>(v, t, [&](unsigned k, C &x, C &y) {
-    const C dv = tld<C>(DV, o + k), b6 = tld<C>(Bq[5], o + k);
+    const C dv = at(DV, k), b6 = mean_at(Bq[5], a.m6, k);
     x = mkc<C>(dv.x - b6.x, dv.y - b6.y);
-    y = b1at(k);
+    y = mean_at(Bq[0], a.m1, k);
   });
   trun<N, +1, false>(v, t, tw, lds);
   float *ens = a.ens + (size_t)row * N;
@@ -258,14 +266,14 @@ stats_t(StatsZ a, const typename CT<R>::c *__restrict__ tw, int nx, int ny, int 
 #pragma unroll
     for (int q = 0; q < F::R; ++q) {
       const int e = m * F::R + q;
-      if (own) ens[t + Z::G * m + q * F::NB] = (float)sqrt((double)s2[e] + (double)v[e].x * (double)v[e].x);
+      if (own) ens[t + Z::G * m + q * F::NB] = (float)sqrt(s2[e] + v[e].x * v[e].x);
       U[e] = v[e].y;
     }
   }
   // v + i w (a lane without a butterfly holds zeros: nothing in the sums)
   tload_modes<N, true, C>(v, t, [&](unsigned k, C &x, C &y) {
-    x = tld<C>(V, o + k);
-    y = tld<C>(Bq[1], o + k);
+    x = at(V, k);
+    y = at(Bq[1], k);
   });
   trun<N, +1, false>(v, t, tw, lds);
 #pragma unroll
@@ -278,28 +286,19 @@ stats_t(StatsZ a, const typename CT<R>::c *__restrict__ tw, int nx, int ny, int 
     sum[25] += u * vv * vv;  // v2u
     sum[26] += vv * u * u;   // u2v
   }
-  auto wd = [](C x) { return make_double2((double)x.x, (double)x.y); };
 #pragma unroll 1
-  for (int k = t; k <= nz2; k += Z::G) {
-    double2 b1 = wd(tld<C>(Bq[0], o + k)), b4 = wd(tld<C>(Bq[3], o + k)), b6 = wd(tld<C>(Bq[5], o + k));
-    if (a.m1 && k == 0) {
-      b1.x = a.m1[om];
-      b4.x = a.m4[om];
-      b6.x = a.m6[om];
-    }
-    stats_mode(sum, k == 0 ? 1.0 : 2.0, a.kaz[k], b1, wd(tld<C>(Bq[1], o + k)), wd(tld<C>(Bq[2], o + k)), b4,
-               wd(tld<C>(Bq[4], o + k)), b6, wd(tld<C>(Bq[6], o + k)), wd(tld<C>(Bq[7], o + k)),
-               wd(tld<C>(V, o + k)), wd(tld<C>(DV, o + k)));
-  }
+  for (int k = t; k <= nz2; k += Z::G)
+    stats_mode(sum, k == 0 ? 1.0 : 2.0, a.kaz[k], mean_at(Bq[0], a.m1, k), at(Bq[1], k), at(Bq[2], k),
+               mean_at(Bq[3], a.m4, k), at(Bq[4], k), mean_at(Bq[5], a.m6, k), at(Bq[6], k), at(Bq[7], k), at(V, k),
+               at(DV, k));
 #pragma unroll
   for (int q = 0; q < NSUM; ++q) sum[q] = team_sum<Z::G>(sum[q], t);
   if (t != 0) return;
   const size_t S = (size_t)nx * (ny + 1);
   double *acc = a.acc + (size_t)i * (ny + 1) + j;
   stats_add_sums(acc, S, sum);
-  auto re0 = [&](const R *p) { return (double)tld<C>(p, o).x; };
-  stats_add_means(acc, S, a.m1 ? a.m1[om] : re0(Bq[0]), re0(Bq[1]), re0(Bq[2]), a.m1 ? a.m4[om] : re0(Bq[3]),
-                  re0(Bq[4]), a.m1 ? a.m6[om] : re0(Bq[5]), re0(Bq[6]), re0(Bq[7]), re0(V), re0(DV));
+  stats_add_means(acc, S, mean_at(Bq[0], a.m1, 0).x, at(Bq[1], 0).x, at(Bq[2], 0).x, mean_at(Bq[3], a.m4, 0).x,
+                  at(Bq[4], 0).x, mean_at(Bq[5], a.m6, 0).x, at(Bq[6], 0).x, at(Bq[7], 0).x, at(V, 0).x, at(DV, 0).x);
 }
 
 template <int N> static void team_fns(ZTeamFns &f) {
@@ -312,7 +311,7 @@ template <int N> static void team_fns(ZTeamFns &f) {
   f.p2f = &products2_t<N, float>;
   f.fx = &fourxz_t<N>;
   f.std_ = &stats_t<N, double>;
-  f.stf = &stats_t<N, float>;
+  if constexpr (N != 512 && N != 1024) f.stf = &stats_t<N, float>; // those: stats_zr
 }
 
 // the kernels of length n if it is one of LO, LO + 2, .. HI

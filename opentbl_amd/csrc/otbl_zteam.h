@@ -437,12 +437,13 @@ __device__ __forceinline__ void tload_spectral(typename CT<R>::c *v, int t, cons
 
 // After the last inverse pass (outputs j + q N / R in order): the spectra of
 // a and b of the transform of a + i b, modes 0..nz2, scaled by 1 / N (a null
-// B is not written), plus mean-flow terms A_0 += c0a XA_0, A_k += cka XA_k
-// (XA at A's offset, read before A is written: it may be A).
+// B is not written), plus mean-flow terms A_0 += c0a XA_0, A_k += cka XA_k and
+// B_k += cb XB_k (XA at A's offset, read before A is written: it may be A; XB, B
+// likewise).
 template <int N, typename R>
 __device__ __forceinline__ void tstore_spectral(const typename CT<R>::c *v, int t, typename CT<R>::c *lds, R *A,
                                                 unsigned oa, R *B, unsigned ob, const R *XA = nullptr, R c0a = R(0),
-                                                R cka = R(0)) {
+                                                R cka = R(0), const R *XB = nullptr, R cb = R(0)) {
   using C = typename CT<R>::c;
   constexpr int G = ZRow<N>::G, RD = ZRow<N>::rad(0), NB = N / RD, MB = (NB + G - 1) / G, nz2 = N / 3 - 1;
   constexpr int NI = (nz2 + G) / G; // trips over the nz2 + 1 modes
@@ -455,11 +456,12 @@ __device__ __forceinline__ void tstore_spectral(const typename CT<R>::c *v, int 
         if (!(lo > nz2 && hi < N - nz2)) lds[t + lo] = v[m * RD + q];
       }
     }
-  C xa[NI];
+  C xa[NI], xb[NI];
 #pragma unroll
   for (int it = 0; it < NI; ++it) {
     const int k = t + G * it < nz2 ? t + G * it : nz2;
     xa[it] = XA ? tld<C>(XA, oa + k) : mkc<C>(0.0, 0.0);
+    xb[it] = XB ? tld<C>(XB, ob + k) : mkc<C>(0.0, 0.0);
   }
   tsync();
   const R sc = R(1.0 / N);
@@ -475,7 +477,11 @@ __device__ __forceinline__ void tstore_spectral(const typename CT<R>::c *v, int 
       }
       tst(A, oa + k, mkc<C>(ar, ai));
       if (B) {
-        const R br = R(0.5) * (z.y + w.y) * sc, bi = (k == 0) ? R(0) : R(-0.5) * (z.x - w.x) * sc;
+        R br = R(0.5) * (z.y + w.y) * sc, bi = (k == 0) ? R(0) : R(-0.5) * (z.x - w.x) * sc;
+        if (XB) {
+          br += cb * xb[it].x;
+          bi += (k == 0) ? R(0) : cb * xb[it].y;
+        }
         tst(B, ob + k, mkc<C>(br, bi));
       }
     }

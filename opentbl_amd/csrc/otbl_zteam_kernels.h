@@ -35,13 +35,16 @@ template <int G, typename R> __device__ __forceinline__ R team_max(R v, int t) {
 
 // Plane loop 1 of rhsp (rhsp.F90:120-153) for one (j, i) row: r2c(u_x^2) ->
 // wki1, r2c(u w_x) -> wki3, r2c(v_x uy) -> wki2 (rows <= ny) and the row's
-// maxima of |u|, |w_x|, |v_x|.  The transforms, their pairing and, in FP32,
-// the mean flow kept out of them are those of products1_z.
+// maxima of |u|, |w_x|, |v_x|.  The transforms and their pairing are those of
+// products1_z.  In FP32 the mean flow of u_x, of uy and of u stays out of them:
+// u w_x = U w_x + u' w_x with the U term added in spectral space.  With U in the
+// transform that it shares with w_x, the error of w's right-hand side at 54 points
+// was twice as large.
 // Bound by the copy rate's latency side: a transform holds E complex values
 // and its twiddles, so few wavefronts fit.  FP64 is held to two per SIMD where
 // a lane has at most 16 values (a few dozen registers spilled; 459 -> 388 us on
 // a 896 x 176 x 224 box, 1.5 GB), the rest is left to the compiler: three per
-// SIMD in FP32 (forced to four it spills, 210 -> 288 us).  The LDS kernel took
+// SIMD in FP32 (222 us; forced to four it spills, +37%).  The LDS kernel took
 // 2610 us there, 1567 us in FP32.
 template <int N, typename R>
 __global__ void __launch_bounds__(64, sizeof(R) == 8 && ZRow<N>::E <= 16 ? 2 : 1)
@@ -86,10 +89,12 @@ products1_t(const R *__restrict__ u, R *wki1, R *wki2, R *wki3, const R *__restr
   }
   R s1[F::E];
   tload_spectral<N, true>(Q, t, u, ou, (const R *)wki3, ou);
+  const R U = SPLIT ? tld<C>(u, ou).x : R(0);
+  if (SPLIT && t == 0) Q[0].x = R(0);
   trun<N, +1, false>(Q, t, tw, lds);
 #pragma unroll
   for (int e = 0; e < F::E; ++e) {
-    um = fmax(um, fabs(Q[e].x));
+    um = fmax(um, fabs(SPLIT ? Q[e].x + U : Q[e].x));
     wm = fmax(wm, fabs(Q[e].y));
     s1[e] = Q[e].x * Q[e].y;
   }
@@ -100,7 +105,8 @@ products1_t(const R *__restrict__ u, R *wki1, R *wki2, R *wki3, const R *__restr
 #pragma unroll
   for (int e = 0; e < F::E; ++e) Q[e] = mkc<C>(Q[e].x * Q[e].x, s1[e]);
   trun<N, -1, true>(Q, t, tw, lds);
-  tstore_spectral<N, R>(Q, t, lds, wki1, ou, wki3, ou, SPLIT ? wki1 : nullptr, Ux, R(2) * Ux);
+  tstore_spectral<N, R>(Q, t, lds, wki1, ou, wki3, ou, SPLIT ? wki1 : nullptr, Ux, R(2) * Ux, SPLIT ? wki3 : nullptr,
+                        U);
   um = team_max<Z::G>(um, t);
   wm = team_max<Z::G>(wm, t);
   vm = team_max<Z::G>(vm, t);
@@ -112,9 +118,14 @@ products1_t(const R *__restrict__ u, R *wki1, R *wki2, R *wki3, const R *__restr
 }
 
 // Plane loop 2 of rhsp (rhsp.F90:367-415) for one (j, i) row, j <= ny, planes
-// 2..nx-1: r2c(v w_v) -> ya, r2c(v_u^2) -> yb, r2c(w^2) -> yc, as products2_z.
+// 2..nx-1: r2c(v w_v) -> ya, r2c(v_u^2) -> yb, r2c(w^2) -> yc, as products2_z.  In
+// FP32 an inverse transform's round-off in one product scales with the other, and
+// d/dz multiplies that of w^2 by kz, so the rows keep the pairs of the kernel that
+// ran them before: (v_u^2, w^2) and v w_v alone at the engine's lengths, else
+// (v w_v, v_u^2) and w^2 alone (ALONE) as on the LDS kernel (with the other pairs
+// the error of w's right-hand side was up to 4.9 times, at 980 points).
 // At the copy rate in FP64 (896 x 176 x 224: 1740 -> 258 us, 5.0 TB/s; FP32
-// 1005 -> 158 us, 4.1 TB/s).
+// 1005 -> 159 us, 4.1 TB/s).
 template <int N, typename R>
 __global__ void __launch_bounds__(64)
 products2_t(const R *__restrict__ resv, const R *__restrict__ resw, R *ya, R *yb, R *yc,
@@ -123,6 +134,7 @@ products2_t(const R *__restrict__ resv, const R *__restrict__ resw, R *ya, R *yb
   using Z = ZRow<N>;
   using F = ZRowPhys<N>;
   constexpr int nz1 = 2 * (N / 3);
+  constexpr bool ALONE = sizeof(R) == 4 && !(N == 256 || N == 512 || N == 1024);
   __shared__ C lds_all[Z::T * Z::lds()];
   TeamRow<N> w;
   if (!w.init(nrows)) return;
@@ -140,16 +152,26 @@ products2_t(const R *__restrict__ resv, const R *__restrict__ resw, R *ya, R *yb
   C Q[Z::E];
   tload_spectral<N, true>(Q, t, (const R *)yb, ou, resw, ou);
   trun<N, +1, false>(Q, t, tw, lds);
+  R s1[ALONE ? F::E : 1]; // v_u^2
 #pragma unroll
-  for (int e = 0; e < F::E; ++e) Q[e] = mkc<C>(Q[e].x * Q[e].x, Q[e].y * Q[e].y);
+  for (int e = 0; e < F::E; ++e) {
+    if constexpr (ALONE) {
+      s1[e] = Q[e].x * Q[e].x;
+      Q[e] = mkc<C>(Q[e].y * Q[e].y, R(0));
+    } else {
+      Q[e] = mkc<C>(Q[e].x * Q[e].x, Q[e].y * Q[e].y);
+    }
+  }
   trun<N, -1, true>(Q, t, tw, lds);
-  tstore_spectral<N, R>(Q, t, lds, yb, ou, yc, ou);
+  if constexpr (ALONE) tstore_spectral<N, R>(Q, t, lds, yc, ou, nullptr, 0);
+  else tstore_spectral<N, R>(Q, t, lds, yb, ou, yc, ou);
   tload_spectral<N, true>(Q, t, resv, ov, (const R *)ya, ou);
   trun<N, +1, false>(Q, t, tw, lds);
 #pragma unroll
-  for (int e = 0; e < F::E; ++e) Q[e] = mkc<C>(Q[e].x * Q[e].y, R(0));
+  for (int e = 0; e < F::E; ++e) Q[e] = mkc<C>(Q[e].x * Q[e].y, ALONE ? s1[ALONE ? e : 0] : R(0));
   trun<N, -1, true>(Q, t, tw, lds);
-  tstore_spectral<N, R>(Q, t, lds, ya, ou, nullptr, 0);
+  if constexpr (ALONE) tstore_spectral<N, R>(Q, t, lds, ya, ou, yb, ou);
+  else tstore_spectral<N, R>(Q, t, lds, ya, ou, nullptr, 0);
 }
 
 // fourxz (ffts.f90:27-67) on independent rows: iopt >= 0 c2r, < 0 r2c

@@ -327,7 +327,7 @@ stats_xc(const T *__restrict__ in, T *__restrict__ out, const double *__restrict
   for (int r = 0; r < L; ++r) {
     if (r % XGRP == 0) XFENCE();
     const int j = j0 + r;
-    const T o = (T)(v[r] + C * t.G(r) + D * t.S(r));
+    const T o = (T)(v[r] + fma(C, t.G(r), D * t.S(r)));
     if (KIND == 0) {
       if (w.ok && j < nx) (out + (size_t)j * P)[w.l] = o;
     } else {
@@ -374,7 +374,7 @@ stats_yc(StatsY a, const double *__restrict__ tiy, const double *__restrict__ ti
 #pragma unroll
     for (int r = 0; r < L; ++r) {
       if (r % XGRP == 0) XFENCE();
-      v[r] = v[r] + C * t.G(r) + D * t.S(r);
+      v[r] = v[r] + fma(C, t.G(r), D * t.S(r));
       if (ok && j0 + r < ny) out[(size_t)(j0 + r) * s] = (T)v[r];
     }
   };

@@ -161,7 +161,7 @@ __device__ __forceinline__ void interpxx_b(const T *__restrict__ gen, T *__restr
 #pragma unroll
   for (int r = 0; r < L; ++r) {
     if (r % XGRP == 0) XFENCE();
-    const T o = v[r] + C * t.G(r) + D * t.S(r);
+    const T o = v[r] + fma(C, t.G(r), D * t.S(r));
     if (w.ok && j0 + r < nx) (geni + (size_t)(j0 + r) * P)[w.l] = o;
   }
 }
@@ -265,7 +265,7 @@ __device__ __forceinline__ void difvisxx_b(const T *__restrict__ gp, const T *__
 #pragma unroll
     for (int k = 0; k < XGRP; ++k) {
       const int r = r0 + k, j = j0 + r;
-      const T xc = a[r] + C * tc.G(r) + D * tc.S(r), xv = b[r] + Cv * tv.G(r) + Dv * tv.S(r);
+      const T xc = a[r] + fma(C, tc.G(r), D * tc.S(r)), xv = b[r] + fma(Cv, tv.G(r), Dv * tv.S(r));
       const T o = j == nx - 1 ? flow : prev[k] + (xc + rex * xv);
       if (w.ok && j < nx) (out + (size_t)j * P)[w.l] = o;
     }

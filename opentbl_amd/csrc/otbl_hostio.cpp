@@ -11,11 +11,13 @@
 // x 160 1.6 -> 6.7 (1.0 with idle CPUs), 387 x 113 x 98 0.54 -> 6.3 (0.43).  From
 // 2^27 values on the link's saving, 10 ms, is above that.
 #include <emmintrin.h>
+#include <sched.h>
 
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstdint>
+#include <cstdio>
 #include <memory>
 #include <mutex>
 #include <system_error>
@@ -30,6 +32,31 @@ namespace otbl {
 static constexpr size_t STAGE = size_t(2) << 20;
 // widening threads: about 6 GB/s each, and the host's memory is full at 10
 static constexpr int THREADS = 10;
+// fewest CPUs of the calling thread for which the threads are worth waking: ten of
+// them bound to 1, 2, 4, 6 CPUs widen the largest field above (2.7 GB of doubles)
+// in 180, 92, 61, 52 ms at best, the GPU's widening takes 48
+static constexpr int MIN_CPUS = 6;
+
+// CPUs that the calling thread may run on: its affinity mask, and the quota of
+// its control group where there is one
+static int usable_cpus() {
+  static const int quota = [] {
+    int n = 1 << 20;
+    if (std::FILE *f = std::fopen("/sys/fs/cgroup/cpu.max", "r")) {
+      long q = 0, p = 0; // "max 100000": no quota
+      if (std::fscanf(f, "%ld %ld", &q, &p) == 2 && q > 0 && p > 0) n = (int)std::max(1L, q / p);
+      std::fclose(f);
+    }
+    return n;
+  }();
+  const int most = 1 << 14; // CPUs in the mask
+  cpu_set_t *set = CPU_ALLOC(most);
+  if (!set) return 0;
+  const size_t bytes = CPU_ALLOC_SIZE(most);
+  const int n = sched_getaffinity(0, bytes, set) == 0 ? CPU_COUNT_S(bytes, set) : 0;
+  CPU_FREE(set);
+  return std::min(n, quota);
+}
 
 void free_stage(Box &b) {
   if (b.stage) (void)hipHostFree(b.stage);
@@ -172,13 +199,13 @@ std::weak_ptr<Pool> g_pool;
 std::shared_ptr<Pool> the_pool() {
   std::lock_guard<std::mutex> l(g_pool_mu);
   std::shared_ptr<Pool> p = g_pool.lock();
-  if (!p) g_pool = p = std::make_shared<Pool>((int)std::min(THREADS, (int)std::thread::hardware_concurrency() - 1));
+  if (!p) g_pool = p = std::make_shared<Pool>(std::min(THREADS, usable_cpus() - 1));
   return p;
 }
 } // namespace
 
 bool field_to_host(Box &b, const float *dev, double *host, size_t n, const HostMean &mean) {
-  if (n < b.read_min || !make_stage(b)) return false;
+  if (n < b.read_min || usable_cpus() < MIN_CPUS || !make_stage(b)) return false;
   if (!b.readers) b.readers = the_pool();
   Pool &pool = *static_cast<Pool *>(b.readers.get());
   std::unique_lock<std::mutex> mine(pool.busy, std::try_to_lock);

@@ -316,6 +316,21 @@ static void x_difvis(Box &b, const T *prod, const T *vel, T *out, int R, int whi
   }
 }
 
+// the x interpolations and derivatives of a substep's components u, v, w
+// (rhsp.F90:105-107,181-204)
+template <typename T> static void x_interp3(Box &b, const T *const *vel, T *const *wki) {
+  if (kxc_interpxx3<T>(b, vel, wki)) return;
+  x_interp<T>(b, vel[0], wki[0], b.ny + 1, 1);
+  x_interp<T>(b, vel[1], wki[1], b.ny, 0);
+  x_interp<T>(b, vel[2], wki[2], b.ny + 1, 0);
+}
+template <typename T> static void x_difvis3(Box &b, const T *const *wki, const T *const *vel, T *const *rhs) {
+  if (kxc_difvisxx3<T>(b, wki, vel, rhs)) return;
+  x_difvis<T>(b, wki[0], vel[0], rhs[0], b.ny + 1, 1, 1);
+  x_difvis<T>(b, wki[1], vel[1], rhs[1], b.ny, 0, 0);
+  x_difvis<T>(b, wki[2], vel[2], rhs[2], b.ny + 1, 0, 0);
+}
+
 // ---------------------------------------------------------------------------
 // y-line operators.  Column c = (kr, plane); rows at stride nz1.
 // ---------------------------------------------------------------------------
@@ -2187,14 +2202,10 @@ template <typename T> static void rhsp_t(Box &b, int m) {
       }
     });
   }
-  // x interpolation (rhsp.F90:105-107)
+  // x interpolation
   const T *vel3[3] = {u, v, w}, *wki3c[3] = {wki1, wki2, wki3};
   T *wk3[3] = {wki1, wki2, wki3}, *rhs3[3] = {rhsu, rhsv, rhsw};
-  if (!kxc_interpxx3<T>(b, vel3, wk3)) {
-    x_interp<T>(b, u, wki1, ru, 1);
-    x_interp<T>(b, v, wki2, ny, 0);
-    x_interp<T>(b, w, wki3, ru, 0);
-  }
+  x_interp3<T>(b, vel3, wk3);
   if (m == 1)
     LAUNCH(b, "energies", 3, 1024, 0, energies_kernel<T>, u, v, w, b.dc.hy, b.ds, nx, ny, nz1, b.nz2);
   // u interpolated to v rows in spectral space (interpyy is linear along y and
@@ -2217,12 +2228,8 @@ template <typename T> static void rhsp_t(Box &b, int m) {
   else if constexpr (F64)
     LAUNCH(b, "rhsu_loop1", nblk((size_t)nz1 * nx), TPB, 0, rhsu_loop1_kernel, wki2, wki3, rhsu, b.dc, ny, nz1,
            nx);
-  // x derivatives (rhsp.F90:181-204)
-  if (!kxc_difvisxx3<T>(b, wki3c, vel3, rhs3)) {
-    x_difvis<T>(b, wki1, u, rhsu, ru, 1, 1);
-    x_difvis<T>(b, wki2, v, rhsv, ny, 0, 0);
-    x_difvis<T>(b, wki3, w, rhsw, ru, 0, 0);
-  }
+  // x derivatives
+  x_difvis3<T>(b, wki3c, vel3, rhs3);
   // time step and RK constants
   LAUNCH(b, "dt", 1, 64, 0, dt_kernel, b.ds, b.vmbits, b.dc.dymin, ny, m, b.dt_mode == OTBL_DT_EVERY_STEP ? 1 : 0,
          b.hc.dxmin, b.hc.dtret, b.hc.rex, b.hc.rkc[m], b.hc.rkd[m], b.hc.rkcv[m], b.hc.rkdv[m]);
@@ -2441,32 +2448,37 @@ template <typename F> static double time_launches(Box &b, int reps, F &&launch) 
   return (double)ms / reps;
 }
 
+// the x lines of a substep as it launches them
 template <typename T> static void x_lines_once(Box &b) {
-  x_interp<T>(b, fld<T>(b.f[OTBL_U]), fld<T>(b.wki1), b.ny + 1, 1);
-  x_difvis<T>(b, fld<T>(b.wki1), fld<T>(b.f[OTBL_U]), fld<T>(b.rhsu), b.ny + 1, 1, 0);
+  const T *vel[3] = {fld<T>(b.f[OTBL_U]), fld<T>(b.f[OTBL_V]), fld<T>(b.f[OTBL_W])};
+  T *wki[3] = {fld<T>(b.wki1), fld<T>(b.wki2), fld<T>(b.wki3)};
+  T *rhs[3] = {fld<T>(b.rhsu), fld<T>(b.rhsv), fld<T>(b.rhsw)};
+  x_interp3<T>(b, vel, wki);
+  const T *prod[3] = {wki[0], wki[1], wki[2]};
+  x_difvis3<T>(b, prod, vel, rhs);
 }
 
 template <typename T> static std::string autotune_t(Box &b, int reps) {
   char buf[256];
   std::string rep;
-  // x lines: segments per line of the windowed kernels, or the chunked ones
+  // x lines: chunked (interpolations in chunks and derivatives in segments where
+  // only the former are planned so), or windowed in segments
   {
     double best = 1e30;
     int pick = b.xseg;
-    bool chunk = b.xci.L > 0;
-    if (chunk) {
-      b.xchunk = true;
-      best = time_launches(b, reps, [&] { x_lines_once<T>(b); });
-      std::snprintf(buf, sizeof buf, "xchunk=%.4fms ", best);
-      rep += buf;
-    }
-    b.xchunk = false;
-    for (int n = 1; n <= b.xseg_max; ++n) {
-      b.xseg = n;
-      const double ms = time_launches(b, reps, [&] { x_lines_once<T>(b); });
-      std::snprintf(buf, sizeof buf, "xseg%d=%.4fms ", n, ms);
-      rep += buf;
-      if (ms < best) best = ms, pick = n, chunk = false;
+    bool chunk = b.xchunk;
+    for (bool c : {true, false}) {
+      if (c && !b.xci.L) continue;
+      b.xchunk = c;
+      const bool seg = !c || !b.xcd.L; // whether any line is cut into segments
+      for (int n = 1; n <= (seg ? b.xseg_max : 1); ++n) {
+        if (seg) b.xseg = n;
+        const double ms = time_launches(b, reps, [&] { x_lines_once<T>(b); });
+        if (c && !seg) std::snprintf(buf, sizeof buf, "xchunk=%.4fms ", ms);
+        else std::snprintf(buf, sizeof buf, "%sxseg%d=%.4fms ", c ? "xchunk+" : "", n, ms);
+        rep += buf;
+        if (ms < best) best = ms, pick = b.xseg, chunk = c;
+      }
     }
     b.xchunk = chunk;
     b.xseg = pick;

@@ -189,7 +189,9 @@ void k_interpxx(Box &b, const double *gen, double *geni, int R, int which_u) {
   const double *econ = which_u ? b.dc.cofiux : b.dc.cofivx;
   int chi = which_u ? 2 : 1;
   int chi2 = which_u ? chi + 1 : chi + 3;
-  if (b.xchunk) {
+  // in place: one workgroup has to hold the whole line (a span's halo chunks are
+  // another's to overwrite)
+  if (b.xchunk && (gen != geni || b.xci.ns == 1)) {
     kxc_interpxx(b, gen, geni, which_u, chi, chi2, P);
     return;
   }

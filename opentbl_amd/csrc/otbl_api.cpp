@@ -600,6 +600,7 @@ int otbl_create(const otbl_params *prm, const double *y, otbl_ctx **out) {
   b->nv = b->pv * b->nx;
   need(b->nu < (size_t(1) << 32), "a field must have fewer than 2^32 elements");
   OTBL_HIP(hipGetDevice(&b->dev));
+  OTBL_HIP(hipDeviceGetAttribute(&b->cus, hipDeviceAttributeMultiprocessorCount, b->dev));
   (void)scratch_of(b->dev); // the no-allocation entry point's scratch on this device
   OTBL_HIP(hipStreamCreateWithFlags(&b->s, hipStreamNonBlocking));
   build_coef(b->hc, b->nx, b->ny, b->nz, b->re, b->ax, b->az, b->cfl, y);

@@ -116,6 +116,7 @@ enum { XT_INXU = 0, XT_INXV, XT_DCXU, XT_DCXV, XT_VIXU, XT_VIXV };
 struct Box {
   int nx, ny, nz, nz1, nz2, mz, xout, precision, dt_mode;
   int dev = 0; // the HIP device the box lives on (current at otbl_create)
+  int cus = 0; // its compute units
   // bytes per field element: 8 (OTBL_FP64) or 4 (OTBL_MIXED, FP32 fields);
   // fields and work fields are allocated at that size
   int esz = 8;

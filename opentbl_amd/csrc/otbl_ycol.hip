@@ -1199,8 +1199,9 @@ template void ky_rk_tail<float>(Box &, int, float *, float *, const float *, con
 void ky_rk_tail3(Box &b, double *const *u, double *const *rhs, const double *const *res, const double *const *rhsp,
                  const double *vw, const double *vv, const double *ww) {
   using T = double;
-  // one round of workgroups, and chunks that leave the fused kernel unspilled
-  if (b.yL > 8 || 3 * ygrid((size_t)b.nz1 * b.nx) > 256) {
+  // one round of workgroups (one per CU), and chunks that leave the fused kernel
+  // unspilled
+  if (b.yL > 8 || 3 * ygrid((size_t)b.nz1 * b.nx) > (unsigned)b.cus) {
     ky_rk_tail<T>(b, 1, u[1], rhs[1], res[1], rhsp[1], vw, vv);
     ky_rk_tail<T>(b, 3, u[0], rhs[0], res[0], rhsp[0], nullptr, nullptr);
     ky_rk_tail<T>(b, 2, u[2], rhs[2], res[2], rhsp[2], ww, vw);

@@ -84,13 +84,15 @@ def kernel_model(cfg, s=8):
 
 
 # kernel-event names -> HIP kernel function names in rocprofv3 output
+# (save_predict_pair_kernel: the FP32 pass that the final update replaced, in the
+# last section of the mixed summary)
 TRACE_NAMES = {"dct2_rows": "dct_rows_z", "dct3_rows": "dct_rows_z", "div": "div_pencils_kernel",
                "poisson_y": "poisson_y_chunk", "to_planes": "pencils_to_planes_kernel",
-               "products1": ("products1_zp", "products1_z"), "products2": ("products2_t", "products2_z"),
-               "interpxx": ("interpxx_c", "interpxx_w"),
-               "difvisxx": ("difvisxx_w", "difvisxx_c"), "interpyy": "interpyy_y", "rhsu_loop1": "rhsu_loop1_y",
-               "rhs_loop2": "rhs_loop2_y", "rk_final": ("rk_final_y", "rk_final_yh"), "rk_tail": "rk_tail_y",
-               "project": ("project_kernel", "project_pair_kernel"),
+               "products1": ("products1_zp", "products1_t", "products1_z"), "products2": ("products2_t", "products2_z"),
+               "interpxx": ("interpxx3_c", "interpxx_c", "interpxx_w"),
+               "difvisxx": ("difvisxx3_c", "difvisxx_c", "difvisxx_w"), "interpyy": "interpyy_y",
+               "rhsu_loop1": "rhsu_loop1_y", "rhs_loop2": "rhs_loop2_y", "rk_final": ("rk_final_y", "rk_final_yh"),
+               "rk_tail": ("rk_tail_y", "rk_tail3_y"), "project": ("project_kernel", "project_pair_kernel"),
                "save_predict": ("save_predict_kernel", "save_predict_pair_kernel")}
 
 
@@ -249,7 +251,8 @@ def roofline(rows, model, workload, precision, hbm_only=False):
     the model covers (hbm_only: among those without a flop count, the
     streaming kernels)."""
     name, n, ms, avg, gbs, tfs = next(r for r in rows if r[0] in model and not (hbm_only and model[r[0]][1]))
-    by, fl, _ = model[name]
+    fl = model[name][1]
+    by = gbs * 1e9 * avg * 1e-3  # the launch's own: report() counts every component that it holds
     peak_tf = FP32_PEAK_TFLOPS if precision == "mixed" else FP64_PEAK_TFLOPS
     intensity = fl / by if fl else 0.0
     if intensity > peak_tf * 1e12 / (HBM_PEAK_GBS * 1e9):

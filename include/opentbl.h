@@ -268,7 +268,11 @@ int otbl_d2d(void *dst, const void *src, size_t bytes);
  * tuned:0|1 streams:1|2 tail:0|1 zteam:<lanes per z row> xchunk:<planes>"
  * (streams:2: rhsp's plane loop 2 on a second stream beside plane loop 1;
  * tail:1: rhsp's tail fused per component; zteam, xchunk: 0 or the kernels with
- * several z rows per wavefront, x lines in chunks)
+ * several z rows per wavefront, x lines in chunks).  z and x name the kernels
+ * beside those: with zteam not 0 the z rows run on its kernels, except that an
+ * FP32 engine box of 512 or 1024 points keeps the engine for plane loop 1's
+ * products and the statistics; with xchunk not 0 x is what lines that are not
+ * chunked run on.
  * (no counterpart in the reference; for tests and benchmark records). */
 int otbl_get_paths(otbl_ctx *ctx, char *buf, size_t len);
 

@@ -94,17 +94,25 @@ template <int S, typename C> __device__ __forceinline__ void bfly3(C *v) {
   v[2] = csub(m, r);
 }
 
+// cos and sin of 2 pi k / R, R = 5 or 7, k < R
+template <int R> __device__ constexpr double odd_cos(int k) {
+  constexpr double c5[5] = {1.0, 0.30901699437494742410, -0.80901699437494742410, -0.80901699437494742410,
+                            0.30901699437494742410};
+  constexpr double c7[7] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624,
+                            -0.90096886790241912624, -0.22252093395631440429, 0.62348980185873353053};
+  return R == 5 ? c5[k % 5] : c7[k];
+}
+template <int R> __device__ constexpr double odd_sin(int k) {
+  constexpr double s5[5] = {0.0, 0.95105651629515357212, 0.58778525229247312917, -0.58778525229247312917,
+                            -0.95105651629515357212};
+  constexpr double s7[7] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048,
+                            -0.43388373911755812048, -0.97492791218182360702, -0.78183148246802980871};
+  return R == 5 ? s5[k % 5] : s7[k];
+}
+
 template <int R, int S, typename C> __device__ __forceinline__ void bfly_odd(C *v) {
   // direct DFT with constant roots, R = 5 or 7
   using T = decltype(v[0].x);
-  constexpr double c5[5] = {1.0, 0.30901699437494742410, -0.80901699437494742410, -0.80901699437494742410,
-                            0.30901699437494742410};
-  constexpr double s5[5] = {0.0, 0.95105651629515357212, 0.58778525229247312917, -0.58778525229247312917,
-                            -0.95105651629515357212};
-  constexpr double c7[7] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624,
-                            -0.90096886790241912624, -0.22252093395631440429, 0.62348980185873353053};
-  constexpr double s7[7] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048,
-                            -0.43388373911755812048, -0.97492791218182360702, -0.78183148246802980871};
   C o[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) {
@@ -112,8 +120,7 @@ template <int R, int S, typename C> __device__ __forceinline__ void bfly_odd(C *
 #pragma unroll
     for (int r = 1; r < R; ++r) {
       const int t = (r * q) % R;
-      const T cr = (T)(R == 5 ? c5[t] : c7[t]);
-      const T sr = (T)(S * (R == 5 ? s5[t] : s7[t]));
+      const T cr = (T)odd_cos<R>(t), sr = (T)(S * odd_sin<R>(t));
       ax += v[r].x * cr - v[r].y * sr;
       ay += v[r].x * sr + v[r].y * cr;
     }

@@ -2138,13 +2138,12 @@ void k_pois(Box &b, int m, double varstep, bool use_m) {
 // ---------------------------------------------------------------------------
 // rhsp (rhsp.F90:22-489)
 // ---------------------------------------------------------------------------
-// Swap the roles of the velocity fields and their saved copies (after
-// save_predict_kernel); a captured substep applies the same swap on replay.
-// Role swap of a substep: the velocities with their saved copies (the
-// predictor wrote the new velocities into the save buffers) and the rhs work
-// fields with the previous-substep rhs fields (the rhs just formed is the
-// next substep's rhs_prev, rhsp.F90:475, and the old rhs_prev buffer is
-// rewritten whole by the next substep).
+// Role swap of a substep: the velocities become the saved ones and the save
+// buffers take the new ones (genflu's plane 1, then the final update; on marched
+// columns save_predict_kernel has filled them), and the rhs work fields swap with
+// the previous-substep rhs fields (the rhs just formed is the next substep's
+// rhs_prev, rhsp.F90:475, and the old rhs_prev buffer is rewritten whole by the
+// next substep).  A captured substep applies the same swap on replay.
 void k_swap_saved(Box &b) {
   std::swap(b.f[OTBL_U], b.resu);
   std::swap(b.f[OTBL_V], b.resv);

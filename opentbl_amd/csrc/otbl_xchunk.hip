@@ -29,8 +29,8 @@
 // The derivatives of larger boxes stay on the marching kernel, whose two arrays
 // in flight fill the memory system there: FP64 from 30000 lines on (128
 // registers leave one workgroup per CU, whose load and store phases do not
-// overlap: 1024 x 192 x 768, calls of several boxes in flight, 524 against 694
-// us), FP32 where it needs at most three segments per line (1536 x 315 x 1024:
+// overlap: 1024 x 192 x 768, calls of three boxes in flight, 524 against 712
+// us; a launch alone is faster in chunks, 643 against 705), FP32 where it needs at most three segments per line (1536 x 315 x 1024:
 // 1033 against 1061 us).
 #include "otbl_chunk.h"
 

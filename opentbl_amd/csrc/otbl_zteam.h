@@ -129,14 +129,6 @@ template <int N> struct ZRow {
 // odd prime R from the sums and differences of the pairs v_r, v_{R-r}
 template <int R, int S, typename C> __device__ __forceinline__ void tbfly_odd(C *v) {
   using T = decltype(v[0].x);
-  constexpr double c5[5] = {1.0, 0.30901699437494742410, -0.80901699437494742410, -0.80901699437494742410,
-                            0.30901699437494742410};
-  constexpr double s5[5] = {0.0, 0.95105651629515357212, 0.58778525229247312917, -0.58778525229247312917,
-                            -0.95105651629515357212};
-  constexpr double c7[7] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624,
-                            -0.90096886790241912624, -0.22252093395631440429, 0.62348980185873353053};
-  constexpr double s7[7] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048,
-                            -0.43388373911755812048, -0.97492791218182360702, -0.78183148246802980871};
   constexpr int H = R / 2;
   C t[H], d[H];
   C s0 = v[0];
@@ -153,7 +145,7 @@ template <int R, int S, typename C> __device__ __forceinline__ void tbfly_odd(C 
 #pragma unroll
     for (int r = 1; r <= H; ++r) {
       const int k = (r * q) % R;
-      const T cr = (T)(R == 5 ? c5[k] : c7[k]), sr = (T)(S * (R == 5 ? s5[k] : s7[k]));
+      const T cr = (T)odd_cos<R>(k), sr = (T)(S * odd_sin<R>(k));
       a.x += cr * t[r - 1].x;
       a.y += cr * t[r - 1].y;
       // i sr d

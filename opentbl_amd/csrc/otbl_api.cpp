@@ -1516,6 +1516,29 @@ void ens_before_boxes(otbl_ensemble &e) {
   for (Box *b : e.boxes) OTBL_HIP(hipStreamWaitEvent(b->s, e.done, 0));
 }
 
+// Whether the runtime of this process is older than the one the library was built
+// with: a program may have loaded its own before (a Python package that brings one
+// along).  With 7.0 in place of 7.2 the first step of an ensemble with a two-stream
+// box, whose fork lies inside the ensemble's, ended in a segmentation fault on the
+// host, while captures with one level of forks run.
+bool older_runtime() {
+  static const bool older = [] {
+    int v = 0;
+    return hipRuntimeGetVersion(&v) == hipSuccess && v / 100000 < HIP_VERSION / 100000;
+  }();
+  return older;
+}
+
+// A box on one stream while this lives (the same results bit for bit)
+struct OneStream {
+  Box &b;
+  hipStream_t s2;
+  explicit OneStream(Box &box, bool on) : b(box), s2(box.s2) {
+    if (on) b.s2 = nullptr;
+  }
+  ~OneStream() { b.s2 = s2; }
+};
+
 // Substep m of every box (with the end-of-step time update after m = 3).
 void ens_substep(otbl_ensemble &e, int m) {
   bool eager = false;
@@ -1553,6 +1576,7 @@ void ens_substep(otbl_ensemble &e, int m) {
       OTBL_HIP(hipEventRecord(e.fork, e.s));
       for (; done < e.boxes.size(); ++done) {
         Box &b = *e.boxes[done];
+        const OneStream one(b, older_runtime());
         OTBL_HIP(hipStreamWaitEvent(b.s, e.fork, 0));
         enqueue_substep(b, m, (smask >> done) & 1ull);
         if (m == 3) k_end_step(b);

@@ -1,6 +1,7 @@
 """bench.py's kernel records against the sources (no GPU): every HIP function of a
-timed kernel is known to the look-up of profiled traffic, and the bytes quoted
-beside a launch's time are those of all the components that it holds."""
+timed kernel is known to the look-up of profiled traffic, the bytes quoted beside a
+launch's time are those of all the components that it holds, and the committed
+profiles list kernels that the sources have."""
 import glob
 import os
 import re
@@ -42,3 +43,12 @@ def test_bytes_of_a_shared_launch(kname):
     assert r["kernel"] == kname
     assert r["algorithmic_bytes"] == pytest.approx(3 * m[kname][0])
     assert r["achieved"] == pytest.approx(r["algorithmic_bytes"] / (r["avg_ms"] * 1e-3) / 1e9)
+
+
+@pytest.mark.parametrize("path", sorted(glob.glob(os.path.join(ROOT, "profiles", "*.md"))), ids=os.path.basename)
+def test_profiles_list_present_kernels(path):
+    fns = hip_functions()
+    text = open(path).read().split("## Replaced since")[0]
+    names = {m.group(1) for m in re.finditer(r"^\| (\w+)(?:<[^|]*>)? \|", text, re.M)} - {"kernel"}
+    names = {n for n in names if not n.startswith("__amd_rocclr")}
+    assert len(names) > 3 and names <= fns, names - fns

@@ -359,9 +359,11 @@ __device__ __forceinline__ void trun(C *v, int t, const C *__restrict__ tw, C *l
 }
 
 // radix and butterflies per lane of the physical side (the forward
-// transform's last pass): slot m R + q of lane t is point t + G m + q N / R
-template <int N> struct ZRowPhys {
-  static constexpr int R = ZRow<N>::rad(ZRow<N>::NP - 1), NB = N / R, MB = (NB + ZRow<N>::G - 1) / ZRow<N>::G;
+// transform's last pass): slot m R + q of lane t is point t + G m + q N / R.
+// REV, here and below: the forward transform takes the radices reversed (and the
+// inverse as they are)
+template <int N, bool REV = false> struct ZRowPhys {
+  static constexpr int R = ZRow<N>::rad(REV ? 0 : ZRow<N>::NP - 1), NB = N / R, MB = (NB + ZRow<N>::G - 1) / ZRow<N>::G;
   static constexpr int E = MB * R;
 };
 
@@ -384,10 +386,10 @@ template <typename C, typename R> __device__ __forceinline__ void tst(R *base, u
 // gives both signals' mode k (PAIR false: y is absent).  Slots that lie in the
 // zero band nz2 < k < N - nz2 for every lane load nothing, slots wholly on one
 // side of it need no select.
-template <int N, bool PAIR, typename C, class Get>
+template <int N, bool PAIR, typename C, bool REV = false, class Get>
 __device__ __forceinline__ void tload_modes(C *v, int t, Get get) {
   using R = decltype(v[0].x);
-  constexpr int G = ZRow<N>::G, RD = ZRow<N>::rad(0), NB = N / RD, MB = (NB + G - 1) / G, nz2 = N / 3 - 1;
+  constexpr int G = ZRow<N>::G, RD = ZRow<N>::rad(REV ? ZRow<N>::NP - 1 : 0), NB = N / RD, MB = (NB + G - 1) / G, nz2 = N / 3 - 1;
 #pragma unroll
   for (int m = 0; m < MB; ++m)
 #pragma unroll
@@ -417,11 +419,11 @@ __device__ __forceinline__ void tload_modes(C *v, int t, Get get) {
 }
 
 // the same from the signals' spectral rows
-template <int N, bool PAIR, typename R>
+template <int N, bool PAIR, bool REV = false, typename R>
 __device__ __forceinline__ void tload_spectral(typename CT<R>::c *v, int t, const R *X, unsigned ox, const R *Y,
                                                unsigned oy) {
   using C = typename CT<R>::c;
-  tload_modes<N, PAIR, C>(v, t, [&](unsigned k, C &x, C &y) {
+  tload_modes<N, PAIR, C, REV>(v, t, [&](unsigned k, C &x, C &y) {
     x = tld<C>(X, ox + k);
     if (PAIR) y = tld<C>(Y, oy + k);
   });
@@ -432,12 +434,12 @@ __device__ __forceinline__ void tload_spectral(typename CT<R>::c *v, int t, cons
 // B is not written), plus mean-flow terms A_0 += c0a XA_0, A_k += cka XA_k and
 // B_k += cb XB_k (XA at A's offset, read before A is written: it may be A; XB, B
 // likewise).
-template <int N, typename R>
+template <int N, typename R, bool REV = false>
 __device__ __forceinline__ void tstore_spectral(const typename CT<R>::c *v, int t, typename CT<R>::c *lds, R *A,
                                                 unsigned oa, R *B, unsigned ob, const R *XA = nullptr, R c0a = R(0),
                                                 R cka = R(0), const R *XB = nullptr, R cb = R(0)) {
   using C = typename CT<R>::c;
-  constexpr int G = ZRow<N>::G, RD = ZRow<N>::rad(0), NB = N / RD, MB = (NB + G - 1) / G, nz2 = N / 3 - 1;
+  constexpr int G = ZRow<N>::G, RD = ZRow<N>::rad(REV ? ZRow<N>::NP - 1 : 0), NB = N / RD, MB = (NB + G - 1) / G, nz2 = N / 3 - 1;
   constexpr int NI = (nz2 + G) / G; // trips over the nz2 + 1 modes
 #pragma unroll
   for (int m = 0; m < MB; ++m)

@@ -123,7 +123,11 @@ products1_t(const R *__restrict__ u, R *wki1, R *wki2, R *wki3, const R *__restr
 // d/dz multiplies that of w^2 by kz, so the rows keep the pairs of the kernel that
 // ran them before: (v_u^2, w^2) and v w_v alone at the engine's lengths, else
 // (v w_v, v_u^2) and w^2 alone (ALONE) as on the LDS kernel (with the other pairs
-// the error of w's right-hand side was up to 4.9 times, at 980 points).
+// the error of w's right-hand side was up to 4.9 times, at 980 points).  They keep
+// the engine's order of radices, too, the larger at the spectral end (REV): 4 x 16 x
+// 16 left 1.26 times the engine's round-off in the highest modes of v's right-hand
+// side at 1024 points, 16 x 16 x 4 leaves 1.03 times (plane loop 1 gains nothing from
+// it and loses 27% of its time).
 // At the copy rate in FP64 (896 x 176 x 224: 1740 -> 258 us, 5.0 TB/s; FP32
 // 1005 -> 159 us, 4.1 TB/s).
 template <int N, typename R>
@@ -132,9 +136,10 @@ products2_t(const R *__restrict__ resv, const R *__restrict__ resw, R *ya, R *yb
             const typename CT<R>::c *__restrict__ tw, int ny, int nrows) {
   using C = typename CT<R>::c;
   using Z = ZRow<N>;
-  using F = ZRowPhys<N>;
   constexpr int nz1 = 2 * (N / 3);
-  constexpr bool ALONE = sizeof(R) == 4 && !(N == 256 || N == 512 || N == 1024);
+  constexpr bool ENGINE = N == 256 || N == 512 || N == 1024, ALONE = sizeof(R) == 4 && !ENGINE;
+  constexpr bool REV = ENGINE && Z::rad(0) < Z::rad(Z::NP - 1);
+  using F = ZRowPhys<N, REV>;
   __shared__ C lds_all[Z::T * Z::lds()];
   TeamRow<N> w;
   if (!w.init(nrows)) return;
@@ -150,8 +155,8 @@ products2_t(const R *__restrict__ resv, const R *__restrict__ resw, R *ya, R *yb
   yb += bu;
   yc += bu;
   C Q[Z::E];
-  tload_spectral<N, true>(Q, t, (const R *)yb, ou, resw, ou);
-  trun<N, +1, false>(Q, t, tw, lds);
+  tload_spectral<N, true, REV>(Q, t, (const R *)yb, ou, resw, ou);
+  trun<N, +1, REV>(Q, t, tw, lds);
   R s1[ALONE ? F::E : 1]; // v_u^2
 #pragma unroll
   for (int e = 0; e < F::E; ++e) {
@@ -162,16 +167,16 @@ products2_t(const R *__restrict__ resv, const R *__restrict__ resw, R *ya, R *yb
       Q[e] = mkc<C>(Q[e].x * Q[e].x, Q[e].y * Q[e].y);
     }
   }
-  trun<N, -1, true>(Q, t, tw, lds);
-  if constexpr (ALONE) tstore_spectral<N, R>(Q, t, lds, yc, ou, nullptr, 0);
-  else tstore_spectral<N, R>(Q, t, lds, yb, ou, yc, ou);
-  tload_spectral<N, true>(Q, t, resv, ov, (const R *)ya, ou);
-  trun<N, +1, false>(Q, t, tw, lds);
+  trun<N, -1, !REV>(Q, t, tw, lds);
+  if constexpr (ALONE) tstore_spectral<N, R, REV>(Q, t, lds, yc, ou, nullptr, 0);
+  else tstore_spectral<N, R, REV>(Q, t, lds, yb, ou, yc, ou);
+  tload_spectral<N, true, REV>(Q, t, resv, ov, (const R *)ya, ou);
+  trun<N, +1, REV>(Q, t, tw, lds);
 #pragma unroll
   for (int e = 0; e < F::E; ++e) Q[e] = mkc<C>(Q[e].x * Q[e].y, ALONE ? s1[ALONE ? e : 0] : R(0));
-  trun<N, -1, true>(Q, t, tw, lds);
-  if constexpr (ALONE) tstore_spectral<N, R>(Q, t, lds, ya, ou, yb, ou);
-  else tstore_spectral<N, R>(Q, t, lds, ya, ou, nullptr, 0);
+  trun<N, -1, !REV>(Q, t, tw, lds);
+  if constexpr (ALONE) tstore_spectral<N, R, REV>(Q, t, lds, ya, ou, yb, ou);
+  else tstore_spectral<N, R, REV>(Q, t, lds, ya, ou, nullptr, 0);
 }
 
 // fourxz (ffts.f90:27-67) on independent rows: iopt >= 0 c2r, < 0 r2c

@@ -800,8 +800,9 @@ rk_final_yh(float *u, const float *__restrict__ res, const float *__restrict__ r
 // rows 2..4 also to LDS for row 1, and the RK update reads it back from cache.
 // On the half-wave FP32 chunks, whose rk_final alone fills its 64 registers,
 // the fused kernel spilled and measured slower than the three passes (9.0
-// against 7.7 ms per substep at 1536 x 315 x 1024), so those keep them; on
-// the full-wave chunks FP64 took 12.7 ms against 14.6.
+// against 7.7 ms per substep at 1536 x 315 x 1024, before either formed the
+// predictor), so those keep them; on the full-wave chunks FP64 takes 14.0 ms
+// against 15.8 (30 GB a launch of v, with res read three times).
 template <typename T> struct TailArgs { // one component's arrays and tables
   T *u, *rhs;
   const T *res, *rhsp, *pa, *pb, *tabv, *tabi, *tabd;
